@@ -10,6 +10,7 @@
 #include "dropout.hpp"
 #include "esep_body.h"
 #include "head.hpp"
+#include "lora.hpp"
 #include "nf4.hpp"
 #include "rmsnorm.hpp"
 #include "rope.hpp"
@@ -716,6 +717,100 @@ int esep_lora_dropout_bwd(const void* x, const void* g, const int64_t* key, void
                                                 static_cast<hipStream_t>(stream), &sup);
   if (!sup) return fail(ESEP_EINVAL, "lora_dropout_bwd: unsupported dtype");
   return e == hipSuccess ? 0 : hip_fail(e, "lora_dropout_bwd launch");
+}
+
+namespace {
+// The sizes every fused LoRA product takes (dim2 may be 0: absent); 0, or the failure's code.
+int lora_sizes(const char* what, int64_t T, int64_t dim1, int64_t dim2, int r, int dt) {
+  if (dt != ESEP_F16 && dt != ESEP_BF16)
+    return fail(ESEP_EINVAL, "%s: bad dtype code %d (fp16 or bf16)", what, dt);
+  if (r < 8 || r > esep::kLoraMaxRank || r % 8 != 0)
+    return fail(ESEP_ESHAPE, "%s: rank %d is not a multiple of 8 up to %d", what, r,
+                esep::kLoraMaxRank);
+  if (T < 0 || T > (int64_t)esep::kLoraMaxRows || dim1 < 0 || dim2 < 0 || dim1 % 8 != 0 ||
+      dim2 % 8 != 0 || dim1 > (1 << 24) || dim2 > (1 << 24))
+    return fail(ESEP_ESHAPE, "%s: bad sizes T=%lld, %lld, %lld", what, (long long)T,
+                (long long)dim1, (long long)dim2);
+  return 0;
+}
+bool aligned8(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7u) == 0; }
+}  // namespace
+
+int esep_lora_down(const void* x, int64_t ld_x, const void* w, int w_kr, const int64_t* key,
+                   float p, float scale, void* out, int64_t T, int64_t K, int r, int dt,
+                   void* stream) {
+  g_err[0] = 0;
+  if (const int rc = lora_sizes("lora_down", T, K, 0, r, dt)) return rc;
+  if (K < 8 || ld_x < K || ld_x % 8 != 0)
+    return fail(ESEP_ESHAPE, "lora_down: bad K=%lld / row stride %lld", (long long)K,
+                (long long)ld_x);
+  if (key != nullptr && (w_kr != 0 || !(p > 0.f && p < 1.f)))
+    return fail(ESEP_EINVAL, "lora_down: dropout takes W as [r, K] and p in (0, 1)");
+  if (T == 0) return 0;
+  if (x == nullptr || w == nullptr || out == nullptr)
+    return fail(ESEP_EINVAL, "lora_down: x, w and out are required");
+  if (!aligned16(x) || !aligned16(w) || !aligned16(out) || !aligned8(key))
+    return fail(ESEP_EALIGN, "lora_down: pointers need 16-byte (key 8-byte) alignment");
+  const esep::LoraDownArgs a{x, ld_x, w, key, p, key != nullptr ? 1.f / (1.f - p) : 1.f, scale,
+                             out, T, K, r};
+  bool sup = false;
+  const hipError_t e = esep::launch_lora_down(a, w_kr, dt, static_cast<hipStream_t>(stream), &sup);
+  return e == hipSuccess ? 0 : hip_fail(e, "lora_down launch");
+}
+
+int esep_lora_up(const void* xa, const void* b, const void* base, int64_t ld_base, void* out,
+                 int64_t ld_out, float scale, int64_t T, int64_t N, int r, int dt, void* stream) {
+  g_err[0] = 0;
+  if (const int rc = lora_sizes("lora_up", T, N, 0, r, dt)) return rc;
+  if (N < 8 || ld_out < N || ld_out % 8 != 0 ||
+      (base != nullptr && (ld_base < N || ld_base % 8 != 0)))
+    return fail(ESEP_ESHAPE, "lora_up: bad N=%lld / row strides", (long long)N);
+  if (T == 0) return 0;
+  if (xa == nullptr || b == nullptr || out == nullptr)
+    return fail(ESEP_EINVAL, "lora_up: xa, b and out are required");
+  if (!aligned16(xa) || !aligned16(b) || !aligned16(base) || !aligned16(out))
+    return fail(ESEP_EALIGN, "lora_up: pointers need 16-byte alignment");
+  const esep::LoraUpArgs a{xa, b, base, ld_base, out, ld_out, scale, T, N, r};
+  bool sup = false;
+  const hipError_t e = esep::launch_lora_up(a, dt, static_cast<hipStream_t>(stream), &sup);
+  return e == hipSuccess ? 0 : hip_fail(e, "lora_up launch");
+}
+
+int64_t esep_lora_grads_workspace(int64_t T, int64_t K, int64_t N, int r) {
+  if (T <= 0 || K < 0 || N < 0 || K + N == 0 || r < 1 || r > esep::kLoraMaxRank) return 0;
+  const int64_t rows = esep::lora_chunk_rows(T, K, N, r);
+  return (T + rows - 1) / rows * r * (K + N);
+}
+
+int esep_lora_grads(const void* x, const void* a, const void* dxa, const int64_t* key, float p,
+                    void* dx, int accumulate, float* da, const void* dterm, int64_t ld_dterm,
+                    const void* xa, float scale, float* db, float* workspace, int64_t T, int64_t K,
+                    int64_t N, int r, int dt, void* stream) {
+  g_err[0] = 0;
+  if (x == nullptr) K = 0;
+  if (dterm == nullptr) N = 0;
+  if (const int rc = lora_sizes("lora_grads", T, K, N, r, dt)) return rc;
+  if (K + N == 0 || (x != nullptr && K < 8) || (dterm != nullptr && N < 8))
+    return fail(ESEP_EINVAL, "lora_grads: x [T, K] or dterm [T, N] is required");
+  if (x != nullptr && (dxa == nullptr || da == nullptr || (dx != nullptr && a == nullptr)))
+    return fail(ESEP_EINVAL, "lora_grads: x needs dxa and da, dx needs a");
+  if (dterm != nullptr && (xa == nullptr || db == nullptr || ld_dterm < N || ld_dterm % 8 != 0))
+    return fail(ESEP_EINVAL, "lora_grads: dterm needs xa, db and a row stride of at least N");
+  if (key != nullptr && !(p > 0.f && p < 1.f))
+    return fail(ESEP_EINVAL, "lora_grads: p must be in (0, 1)");
+  if (T <= 0) return fail(ESEP_ESHAPE, "lora_grads: T=%lld", (long long)T);
+  if (workspace == nullptr) return fail(ESEP_EINVAL, "lora_grads: no workspace");
+  for (const void* q : {x, a, dxa, static_cast<const void*>(dx), static_cast<const void*>(da), dterm,
+                        xa, static_cast<const void*>(db), static_cast<const void*>(workspace)})
+    if (!aligned16(q)) return fail(ESEP_EALIGN, "lora_grads: pointers need 16-byte alignment");
+  if (!aligned8(key)) return fail(ESEP_EALIGN, "lora_grads: key needs 8-byte alignment");
+  const int64_t rows = esep::lora_chunk_rows(T, K, N, r);
+  const esep::LoraGradArgs g{x, a, dxa, key, p, key != nullptr ? 1.f / (1.f - p) : 1.f, scale, dx,
+                             accumulate ? 1 : 0, dterm, ld_dterm, xa, da, db, workspace, T, K, N,
+                             r, rows, (int)((T + rows - 1) / rows)};
+  bool sup = false;
+  const hipError_t e = esep::launch_lora_grads(g, dt, static_cast<hipStream_t>(stream), &sup);
+  return e == hipSuccess ? 0 : hip_fail(e, "lora_grads launch");
 }
 
 int esep_nf4_dequant(const void* packed, const uint8_t* absmax, const float* absmax2,

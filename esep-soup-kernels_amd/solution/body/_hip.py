@@ -56,6 +56,12 @@ SIGNATURES = {
                                      _f32, _i32, _vp]),
     "esep_nf4_dequant_multi": (_i32, [_vp, _i32, _i32, _vp]),
     "esep_lora_dropout_bwd": (_i32, [_vp, _vp, _vp, _vp, _vp, _i64, _f32, _i32, _i32, _vp]),
+    "esep_lora_down": (_i32, [_vp, _i64, _vp, _i32, _vp, _f32, _f32, _vp, _i64, _i64, _i32, _i32,
+                              _vp]),
+    "esep_lora_up": (_i32, [_vp, _vp, _vp, _i64, _vp, _i64, _f32, _i64, _i64, _i32, _i32, _vp]),
+    "esep_lora_grads_workspace": (_i64, [_i64, _i64, _i64, _i32]),
+    "esep_lora_grads": (_i32, [_vp, _vp, _vp, _vp, _f32, _vp, _i32, _vp, _vp, _i64, _vp, _f32, _vp,
+                               _vp, _i64, _i64, _i64, _i32, _i32, _vp]),
     "esep_swiglu_bwd": (_i32, [_vp, _vp, _vp, _vp, _vp, _i64, _i32, _vp]),
     "esep_attn_bwd": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp,
                              _vp, _i64, _vp, _i64, _vp, _i64, _i32, _i64, _i32, _i32, _i32, _vp,
@@ -467,6 +473,75 @@ def lora_dropout_bwd(x, g, key, xd, dx, p, accumulate=False, name="_lora_dropout
                                      int(bool(accumulate)), dtype_code(x.dtype), _stream(dev))
     _check(rc, "esep_lora_dropout_bwd")
     _record(name)
+
+
+def lora_down(x, w, out, scale=1.0, w_kr=False, key=None, p=0.0):
+    """out [T, r] = scale * drop(x) W^T (esep_lora_down): x [T, K] with unit column stride; W
+    [r, K], or [K, r] with w_kr; dropout when key is given (recorded as the reference's dropout
+    kernel then)."""
+    dev = _dev(x, w, out, key)
+    T, K = x.shape
+    r = out.shape[1]
+    if w.dtype != x.dtype or out.dtype != x.dtype or tuple(w.shape) != ((K, r) if w_kr else (r, K)):
+        raise EsepError("lora_down: w and out must match x [T, K] and the rank")
+    if not w.is_contiguous() or not out.is_contiguous() or out.shape[0] != T:
+        raise EsepError("lora_down: w and out must be contiguous")
+    if key is not None and not x.is_contiguous():
+        raise EsepError("lora_down: dropout needs a contiguous x")
+    rc = lib().esep_lora_down(_p(x), _rows_ld(x, K), _p(w), int(w_kr),
+                              None if key is None else _p(_key(key, dev)), float(p), float(scale),
+                              _p(out), T, K, r, dtype_code(x.dtype), _stream(dev))
+    _check(rc, "esep_lora_down")
+    _record("_lora_down" if key is None else "_lora_dropout_fwd")
+
+
+def lora_up(xa, b, out, scale, base=None, name="_lora_up"):
+    """out [T, N] = [base +] scale * xa B^T (esep_lora_up); out may be base."""
+    dev = _dev(xa, b, out, base)
+    T, r = xa.shape
+    N = b.shape[0]
+    if any(t is not None and t.dtype != xa.dtype for t in (b, out, base)):
+        raise EsepError("lora_up: one dtype")
+    if (not xa.is_contiguous() or not b.is_contiguous() or b.shape[1] != r or out.shape[0] != T
+            or (base is not None and base.shape != out.shape)):
+        raise EsepError("lora_up: xa [T, r], b [N, r], out (and base) [T, N]")
+    rc = lib().esep_lora_up(_p(xa), _p(b), _p(base), 0 if base is None else _rows_ld(base, N),
+                            _p(out), _rows_ld(out, N), float(scale), T, N, r,
+                            dtype_code(xa.dtype), _stream(dev))
+    _check(rc, "esep_lora_up")
+    _record(name)
+
+
+def lora_grads(x=None, a=None, dxa=None, key=None, p=0.0, dx=None, accumulate=False, da=None,
+               dterm=None, xa=None, scale=1.0, db=None):
+    """dx = [dx +] (dxa A) * keep / (1 - p), dA = dxa^T drop(x) and dB = scale * dterm^T xa in one
+    launch and a reduction (esep_lora_grads); either half alone without x or without dterm. x
+    and dx contiguous; dA, dB fp32."""
+    dev = _dev(x, a, dxa, key, dx, da, dterm, xa, db)
+    lead, lo = (x, dxa) if x is not None else (dterm, xa)
+    T, r = lo.shape
+    K = 0 if x is None else x.shape[1]
+    N = 0 if dterm is None else dterm.shape[1]
+    for t, shape in ((x, (T, K)), (a, (r, K)), (dxa, (T, r)), (dx, (T, K)), (dterm, (T, N)),
+                     (xa, (T, r))):
+        if t is not None and (tuple(t.shape) != shape or t.dtype != lead.dtype
+                              or (t is not dterm and not t.is_contiguous())):
+            raise EsepError("lora_grads: operands do not match [T, K], [T, N] and the rank")
+    for t, shape in ((da, (r, K)), (db, (N, r))):
+        if t is not None and (tuple(t.shape) != shape or t.dtype != torch.float32
+                              or not t.is_contiguous()):
+            raise EsepError("lora_grads: da [r, K] and db [N, r] must be contiguous fp32 tensors")
+    ws = torch.empty(int(lib().esep_lora_grads_workspace(T, K, N, r)), device=dev,
+                     dtype=torch.float32)
+    rc = lib().esep_lora_grads(
+        _p(x), _p(a), _p(dxa), None if key is None else _p(_key(key, dev)), float(p), _p(dx),
+        int(bool(accumulate)), _p(da), _p(dterm), 0 if dterm is None else _rows_ld(dterm, N),
+        _p(xa), float(scale), _p(db), _p(ws), T, K, N, r, dtype_code(lead.dtype), _stream(dev))
+    _check(rc, "esep_lora_grads")
+    if x is None or key is None:
+        _record("_lora_grads")
+    else:
+        _record("_lora_dropout_bwd" if dx is not None else "_lora_dropout_fwd")
 
 
 def nf4_dequant(packed, absmax, absmax2, code2, offset, nf4, out, name="_nf4_dequant"):

@@ -1,5 +1,6 @@
-"""LoRA terms of q_proj / v_proj with dropout on the LoRA input, on this repository's HIP
-dropout kernels (esep_lora_dropout_fwd / esep_lora_dropout_bwd) around vendor-BLAS products.
+"""LoRA terms of q_proj / v_proj with dropout on the LoRA input, on this repository's fused HIP
+products (esep_lora_down / esep_lora_up / esep_lora_grads: the mask regenerated inside them), or
+its dropout kernels around vendor-BLAS products for the ranks and sizes those do not take.
 
 Public API as in the reference's solution/body/lora.py (reference lora.py:140-359):
 new_dropout_key, cast_lora_weights, lora_dropout, lora_down_fwd, lora_down_bwd, lora_delta,
@@ -20,8 +21,7 @@ torch's own dropout stream; the law is the same.
 Gradients (xa = drop(x) A^T, dterm the incoming gradient):
     dxa = scaling * dterm @ B        dB = scaling * dterm^T @ xa   (fp32)
     dA  = dxa^T @ drop(x)  (fp32)    dx = (dxa @ A) * keep / (1 - p)
-The products run on the vendor BLAS; the HIP kernels regenerate the mask and do the
-element-wise passes. Compute dtype: fp16 (the reference's), or bf16 when x is bf16.
+Compute dtype: fp16 (the reference's), or bf16 when x is bf16.
 
 LoRAFunction adds the term to the base projection's output (in place when that output is a
 fresh dense tensor of the compute dtype: v_proj); LoRADeltaFunction returns the term alone
@@ -57,6 +57,21 @@ def lora_dropout(x, key, p):
     return out
 
 
+def _fused(rank, *mats):
+    """The fused products take this rank and these 16-bit [rows, width] operands: a rank that is a
+    multiple of 8 up to 64 (the kernels' tiles; a wider term is an ordinary GEMM, which the
+    vendor BLAS runs well), and widths, row strides and addresses of whole 16-byte chunks."""
+    if rank % 8 or not 8 <= rank <= 64:
+        return False
+    for t in mats:
+        if (not t.is_cuda or t.dim() != 2 or t.dtype not in (torch.float16, torch.bfloat16)
+                or not 0 < t.shape[0] <= 1 << 22 or t.shape[1] % 8 or not t.shape[1]
+                or t.stride(1) != 1 or t.stride(0) % 8 or t.stride(0) < t.shape[1]
+                or t.data_ptr() % 16):
+            return False
+    return True
+
+
 _OUT_DTYPE_OK = True
 
 
@@ -73,14 +88,48 @@ def _mm_fp32(a, b):
 
 
 def lora_down_fwd(x, a16, key, p):
-    """xa = drop(x) @ A^T for a dense x [T, in] (no dropout pass when p == 0)."""
+    """xa = drop(x) @ A^T for a dense x [T, in] (no dropout when p == 0)."""
+    if _fused(a16.shape[0], x, a16) and x.is_contiguous() and a16.is_contiguous():
+        xa = torch.empty((x.shape[0], a16.shape[0]), device=x.device, dtype=x.dtype)
+        _hip.lora_down(x, a16, xa, key=key if p > 0.0 else None, p=p)
+        return xa
     return torch.mm(lora_dropout(x, key, p) if p > 0.0 else x, a16.t())
+
+
+def _dense(t, like):
+    return (t.dtype == like.dtype and t.shape == like.shape and t.is_contiguous()
+            and t.data_ptr() % 16 == 0)
+
+
+def _grads_fused(x, a16, dxa):
+    return (_fused(a16.shape[0], x, a16, dxa) and x.is_contiguous() and a16.is_contiguous()
+            and dxa.is_contiguous())
+
+
+def _up_bwd_fused(dout, xa, b16):
+    """The fused dxa and dB take dout (any row stride), xa and B."""
+    return (_fused(b16.shape[1], dout, xa, b16) and xa.is_contiguous() and b16.is_contiguous()
+            and dout.dtype == xa.dtype == b16.dtype)
+
+
+def _dxa(dout, b16, scaling):
+    dxa = torch.empty((dout.shape[0], b16.shape[1]), device=dout.device, dtype=dout.dtype)
+    _hip.lora_down(dout, b16, dxa, scale=scaling, w_kr=True)
+    return dxa
 
 
 def lora_down_bwd(x, a16, dxa, key, p, need_dx=True, dx_accum=None):
     """Backward of lora_down_fwd: (dx or None, dA fp32 [r, in]). With dx_accum (a dense
     [T, in] buffer, e.g. the base projection's dx) the LoRA part of dx is added into it in
     place and it is returned as dx."""
+    if _grads_fused(x, a16, dxa) and (not need_dx or dx_accum is None or _dense(dx_accum, x)):
+        dx = None
+        if need_dx:
+            dx = torch.empty_like(x) if dx_accum is None else dx_accum
+        da = torch.empty(a16.shape, device=x.device, dtype=torch.float32)
+        _hip.lora_grads(x=x, a=a16, dxa=dxa, key=key if p > 0.0 else None, p=p, dx=dx,
+                        accumulate=dx_accum is not None, da=da)
+        return dx, da
     if not need_dx:
         dropped = lora_dropout(x, key, p) if p > 0.0 else x
         return None, _mm_fp32(dxa.t(), dropped)
@@ -98,12 +147,21 @@ def lora_down_bwd(x, a16, dxa, key, p, need_dx=True, dx_accum=None):
 
 def lora_delta(xa, b16, scaling):
     """The term scaling * xa @ B^T on its own."""
+    if _fused(b16.shape[1], xa, b16) and xa.is_contiguous() and b16.is_contiguous() \
+            and b16.shape[0] % 8 == 0:
+        term = torch.empty((xa.shape[0], b16.shape[0]), device=xa.device, dtype=xa.dtype)
+        _hip.lora_up(xa, b16, term, scaling)
+        return term
     term = torch.mm(xa, b16.t())
     return term.mul_(scaling)
 
 
 def lora_up_bwd(dout, xa, b16, scaling):
     """(dxa [T, r], dB fp32 [out, r]) for the term's gradient dout."""
+    if _up_bwd_fused(dout, xa, b16):
+        db = torch.empty(b16.shape, device=dout.device, dtype=torch.float32)
+        _hip.lora_grads(dterm=dout, xa=xa, scale=scaling, db=db)
+        return _dxa(dout, b16, scaling), db
     return torch.mm(dout, b16).mul_(scaling), _mm_fp32(dout.t(), xa).mul_(scaling)
 
 
@@ -142,9 +200,19 @@ class _LoRATerm:
     @staticmethod
     def grads(ctx, dterm, x_index, a_index):
         x2, xa, a16, b16, key = ctx.saved_tensors
-        dxa, db = lora_up_bwd(_rows_mm(dterm, ctx.dtype), xa, b16, ctx.scaling)
-        dx, da = lora_down_bwd(x2, a16, dxa, key, ctx.p, need_dx=ctx.needs_input_grad[x_index])
         need = ctx.needs_input_grad
+        dt2 = _rows_mm(dterm, ctx.dtype)
+        if _up_bwd_fused(dt2, xa, b16) and _grads_fused(x2, a16, xa):
+            # dx, dA and dB in one launch after dxa
+            dxa = _dxa(dt2, b16, ctx.scaling)
+            dx = torch.empty_like(x2) if need[x_index] else None
+            da = torch.empty(a16.shape, device=x2.device, dtype=torch.float32)
+            db = torch.empty(b16.shape, device=x2.device, dtype=torch.float32)
+            _hip.lora_grads(x=x2, a=a16, dxa=dxa, key=key, p=ctx.p, dx=dx, da=da, dterm=dt2,
+                            xa=xa, scale=ctx.scaling, db=db)
+        else:
+            dxa, db = lora_up_bwd(dt2, xa, b16, ctx.scaling)
+            dx, da = lora_down_bwd(x2, a16, dxa, key, ctx.p, need_dx=need[x_index])
         return (dx.view(ctx.x_shape).to(ctx.x_dtype) if dx is not None else None,
                 da.to(ctx.a_dtype) if need[a_index] else None,
                 db.to(ctx.b_dtype) if need[a_index + 1] else None)
@@ -160,10 +228,18 @@ class LoRAFunction(torch.autograd.Function):
         xa, b16 = _LoRATerm.begin(ctx, x, weight_a, weight_b, p, scaling)
         ctx.base_dtype = base.dtype
         if base.dtype == ctx.dtype and base.is_contiguous() and not base._is_view():
-            base.view(-1, base.shape[-1]).addmm_(xa, b16.t(), alpha=scaling)
+            flat = base.view(-1, base.shape[-1])
+            if _fused(b16.shape[1], flat, xa, b16) and xa.is_contiguous() and b16.is_contiguous():
+                _hip.lora_up(xa, b16, flat, scaling, base=flat)
+            else:
+                flat.addmm_(xa, b16.t(), alpha=scaling)
             ctx.mark_dirty(base)
             return base
         flat = base.reshape(-1, base.shape[-1]).to(ctx.dtype)
+        if _fused(b16.shape[1], flat, xa, b16) and xa.is_contiguous() and b16.is_contiguous():
+            out = torch.empty(flat.shape, device=flat.device, dtype=flat.dtype)
+            _hip.lora_up(xa, b16, out, scaling, base=flat)
+            return out.view(base.shape)
         return torch.addmm(flat, xa, b16.t(), alpha=scaling).view(base.shape)
 
     @staticmethod

@@ -296,6 +296,35 @@ int esep_lora_dropout_bwd(const void* x, const void* g, const int64_t* key, void
                           int64_t n, float p, int accumulate, int dt, void* stream);
 
 /*
+ * The LoRA term's products with the dropout mask regenerated inside them (the reference runs its
+ * dropout kernels around library products, solution/body/lora.py:140-245). fp16 / bf16 operands
+ * of dt, fp32 sums, one rounding at each 16-bit store; the mask is esep_lora_dropout_fwd's with
+ * element row * K + column (key NULL: no dropout). r a multiple of 8 up to 64, K and N multiples
+ * of 8; rows unit-stride with the given row strides (multiples of 8, at least the row), the
+ * others dense; every pointer 16-byte aligned (key 8). Replaces lora.py:160-161 (esep_lora_down on x) and
+ * :180-182 (esep_lora_grads).
+ *   esep_lora_down   out[T, r] = scale * drop(x)[T, K] . W^T   W [r, K], or [K, r] with w_kr (then
+ *                    without key: dterm . B)
+ *   esep_lora_up     out[T, N] = [base +] scale * xa[T, r] . b[N, r]^T   out may be base
+ *   esep_lora_grads  with x:     da[r, K] (fp32) = dxa^T . drop(x) and, with dx,
+ *                                dx[T, K] = [dx +] (dxa . a) * keep / (1 - p)   (accumulate)
+ *                    with dterm: db[N, r] (fp32) = scale * dterm^T . xa
+ *                    either or both (x or dterm NULL); workspace: fp32, 16-byte aligned,
+ *                    esep_lora_grads_workspace(T, K or 0, N or 0, r) elements
+ * All sums have a fixed order (no atomics).
+ */
+int esep_lora_down(const void* x, int64_t ld_x, const void* w, int w_kr, const int64_t* key,
+                   float p, float scale, void* out, int64_t T, int64_t K, int r, int dt,
+                   void* stream);
+int esep_lora_up(const void* xa, const void* b, const void* base, int64_t ld_base, void* out,
+                 int64_t ld_out, float scale, int64_t T, int64_t N, int r, int dt, void* stream);
+int64_t esep_lora_grads_workspace(int64_t T, int64_t K, int64_t N, int r);
+int esep_lora_grads(const void* x, const void* a, const void* dxa, const int64_t* key, float p,
+                    void* dx, int accumulate, float* da, const void* dterm, int64_t ld_dterm,
+                    const void* xa, float scale, float* db, float* workspace, int64_t T, int64_t K,
+                    int64_t N, int r, int dt, void* stream);
+
+/*
  * NF4 double-quant weight dequantization (QLoRA / bitsandbytes Linear4bit format). Replaces the
  * reference's Triton launch at solution/nf4/dequant.py:85-89 (dequantize_nf4; kernel math
  * dequant.py:35-57):
