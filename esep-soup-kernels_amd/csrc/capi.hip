@@ -9,6 +9,7 @@
 #include "attention.hpp"
 #include "dropout.hpp"
 #include "esep_body.h"
+#include "gemm.hpp"
 #include "head.hpp"
 #include "lora.hpp"
 #include "nf4.hpp"
@@ -811,6 +812,51 @@ int esep_lora_grads(const void* x, const void* a, const void* dxa, const int64_t
   bool sup = false;
   const hipError_t e = esep::launch_lora_grads(g, dt, static_cast<hipStream_t>(stream), &sup);
   return e == hipSuccess ? 0 : hip_fail(e, "lora_grads launch");
+}
+
+namespace {
+bool gemm_sizes_ok(int64_t M, int64_t N, int64_t K) {
+  return M >= 1 && N >= 8 && K >= 64 && N % 8 == 0 && K % 64 == 0 && M <= (1 << 24) &&
+         N <= (1 << 24) && K <= (1 << 24);
+}
+}  // namespace
+
+int esep_gemm_pays(int64_t M, int64_t N, int64_t K, int b_kn) {
+  return gemm_sizes_ok(M, N, K) && esep::gemm_pays(M, N, K, b_kn != 0) ? 1 : 0;
+}
+
+int64_t esep_gemm_workspace(int64_t M, int64_t N, int64_t K) {
+  if (!gemm_sizes_ok(M, N, K)) return 0;
+  const esep::GemmPlan p = esep::gemm_plan(M, N, K);
+  return p.splits > 1 ? p.splits * M * N : 0;
+}
+
+int esep_gemm(const void* a, int64_t lda, const void* b, int64_t ldb, int b_kn, const void* bias,
+              void* c, int64_t ldc, int c_dt, float* workspace, int64_t M, int64_t N, int64_t K,
+              int dt, void* stream) {
+  g_err[0] = 0;
+  if ((dt != ESEP_F16 && dt != ESEP_BF16) || (c_dt != dt && c_dt != ESEP_F32))
+    return fail(ESEP_EINVAL, "gemm: bad dtype codes %d -> %d", dt, c_dt);
+  if (!gemm_sizes_ok(M, N, K))
+    return fail(ESEP_ESHAPE, "gemm: bad sizes %lld x %lld x %lld", (long long)M, (long long)N,
+                (long long)K);
+  if (lda < K || ldb < (b_kn ? N : K) || ldc < N || lda % 8 != 0 || ldb % 8 != 0 || ldc % 8 != 0 ||
+      lda >= (1 << 23) || ldb >= (1 << 23))  // 2 * 255 * ld fits the 32-bit row offsets
+    return fail(ESEP_ESHAPE, "gemm: bad row strides %lld, %lld, %lld", (long long)lda,
+                (long long)ldb, (long long)ldc);
+  if (a == nullptr || b == nullptr || c == nullptr)
+    return fail(ESEP_EINVAL, "gemm: a, b and c are required");
+  if (bias != nullptr && c_dt == ESEP_F32)
+    return fail(ESEP_EINVAL, "gemm: a bias needs a 16-bit output");
+  const esep::GemmPlan p = esep::gemm_plan(M, N, K);
+  if (p.splits > 1 && workspace == nullptr) return fail(ESEP_EINVAL, "gemm: no workspace");
+  if (!aligned16(a) || !aligned16(b) || !aligned16(c) || !aligned16(bias) || !aligned16(workspace))
+    return fail(ESEP_EALIGN, "gemm: pointers need 16-byte alignment");
+  const esep::GemmArgs g{a, lda, b, ldb, bias, c, ldc, workspace, M, N, K, 0, 0, p.splits, 0};
+  bool sup = false;
+  const hipError_t e = esep::launch_gemm(g, p.shape, b_kn ? 1 : 0, dt, c_dt,
+                                         static_cast<hipStream_t>(stream), &sup);
+  return e == hipSuccess ? 0 : hip_fail(e, "gemm launch");
 }
 
 int esep_nf4_dequant(const void* packed, const uint8_t* absmax, const float* absmax2,

@@ -62,6 +62,10 @@ SIGNATURES = {
     "esep_lora_grads_workspace": (_i64, [_i64, _i64, _i64, _i32]),
     "esep_lora_grads": (_i32, [_vp, _vp, _vp, _vp, _f32, _vp, _i32, _vp, _vp, _i64, _vp, _f32, _vp,
                                _vp, _i64, _i64, _i64, _i32, _i32, _vp]),
+    "esep_gemm_pays": (_i32, [_i64, _i64, _i64, _i32]),
+    "esep_gemm_workspace": (_i64, [_i64, _i64, _i64]),
+    "esep_gemm": (_i32, [_vp, _i64, _vp, _i64, _i32, _vp, _vp, _i64, _i32, _vp, _i64, _i64, _i64,
+                         _i32, _vp]),
     "esep_swiglu_bwd": (_i32, [_vp, _vp, _vp, _vp, _vp, _i64, _i32, _vp]),
     "esep_attn_bwd": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp,
                              _vp, _i64, _vp, _i64, _vp, _i64, _i32, _i64, _i32, _i32, _i32, _vp,
@@ -542,6 +546,73 @@ def lora_grads(x=None, a=None, dxa=None, key=None, p=0.0, dx=None, accumulate=Fa
         _record("_lora_grads")
     else:
         _record("_lora_dropout_bwd" if dx is not None else "_lora_dropout_fwd")
+
+
+def gemm_takes(a, b, b_kn, pays=True):
+    """esep_gemm takes the 2-D a [M, K] and b ([N, K], or [K, N] with b_kn) as they are, and (with
+    `pays`) is expected to be faster there than the vendor BLAS."""
+    if a.dim() != 2 or b.dim() != 2 or a.dtype != b.dtype or not a.is_cuda or a.device != b.device:
+        return False
+    if a.dtype not in (torch.float16, torch.bfloat16):
+        return False
+    M, K = a.shape
+    N = b.shape[1] if b_kn else b.shape[0]
+    if (b.shape[0] if b_kn else b.shape[1]) != K or M < 1 or N < 8 or K < 64 or N % 8 or K % 64:
+        return False
+    for t in (a, b):
+        ld = t.stride(0)
+        if t.stride(1) != 1 or ld % 8 or not t.shape[1] <= ld < 1 << 23 or t.data_ptr() % 16:
+            return False
+    return not pays or bool(lib().esep_gemm_pays(M, N, K, int(b_kn)))
+
+
+def gemm(a, b, out, b_kn=False, bias=None, name="_gemm"):
+    """out [M, N] = a [M, K] b (+ bias) (esep_gemm): b [N, K], or [K, N] with b_kn; out in a's dtype
+    or fp32."""
+    dev = _dev(a, b, out, bias)
+    M, K = a.shape
+    N = out.shape[1]
+    if not gemm_takes(a, b, b_kn, pays=False) or tuple(out.shape) != (
+            M, b.shape[1] if b_kn else b.shape[0]):
+        raise EsepError(f"gemm: operands {tuple(a.shape)} and {tuple(b.shape)} of {a.dtype}")
+    if bias is not None and (bias.dtype != a.dtype or bias.numel() != N or not bias.is_contiguous()):
+        raise EsepError("gemm: bias must be a contiguous [N] tensor of the operands' dtype")
+    need = int(lib().esep_gemm_workspace(M, N, K))
+    ws = torch.empty(need, device=dev, dtype=torch.float32) if need else None
+    rc = lib().esep_gemm(_p(a), a.stride(0), _p(b), b.stride(0), int(b_kn), _p(bias), _p(out),
+                         _rows_ld(out, N), dtype_code(out.dtype), _p(ws), M, N, K,
+                         dtype_code(a.dtype), _stream(dev))
+    _check(rc, "esep_gemm")
+    _record(name)
+
+
+def _no_cast(a):
+    return (not torch.is_autocast_enabled("cuda")
+            or torch.get_autocast_dtype("cuda") == a.dtype)
+
+
+def linear(x, w, bias=None):
+    """F.linear(x, w, bias) without autograd: esep_gemm where it takes the operands and pays, else
+    the vendor BLAS."""
+    x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
+    if (_no_cast(x) and gemm_takes(x2, w, False)
+            and (bias is None or (bias.dtype == x.dtype and bias.dim() == 1 and bias.is_contiguous()
+                                  and bias.data_ptr() % 16 == 0))):
+        out = torch.empty((x2.shape[0], w.shape[0]), device=x.device, dtype=x.dtype)
+        gemm(x2, w, out, bias=bias)
+        return out.view(*x.shape[:-1], w.shape[0])
+    return torch.nn.functional.linear(x, w, bias)
+
+
+def matmul(x, w):
+    """x @ w for a 2-D w [K, N] without autograd: esep_gemm where it takes the operands and pays, else
+    the vendor BLAS."""
+    x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
+    if _no_cast(x) and gemm_takes(x2, w, True):
+        out = torch.empty((x2.shape[0], w.shape[1]), device=x.device, dtype=x.dtype)
+        gemm(x2, w, out, b_kn=True)
+        return out.view(*x.shape[:-1], w.shape[1])
+    return torch.matmul(x, w)
 
 
 def nf4_dequant(packed, absmax, absmax2, code2, offset, nf4, out, name="_nf4_dequant"):

@@ -625,10 +625,10 @@ class _RecomputeMLP(torch.autograd.Function):
             dt = torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else None
             weights = tuple(lin.weight if dt is None else lin.weight.to(dt)
                             for lin in (gate, up, down))
-            h = F.linear(x2, weights[0]).contiguous()
-            u = F.linear(x2, weights[1]).contiguous()
+            h = _hip.linear(x2, weights[0]).contiguous()
+            u = _hip.linear(x2, weights[1]).contiguous()
             _hip.swiglu_fwd(h, u, h)
-            out = F.linear(h, weights[2])
+            out = _hip.linear(h, weights[2])
         del h, u
         saved = (x2,) if r is None else (r, w_norm)
         ctx.n_x = len(saved)
@@ -657,13 +657,13 @@ class _RecomputeMLP(torch.autograd.Function):
         if ctx.nf4:
             nf4 = _nf4()
             w = nf4.dequantize_nf4(down.weight, down.weight.quant_state)
-            dh = torch.matmul(dout2.to(w.dtype), w)
+            dh = _hip.matmul(dout2.to(w.dtype), w)
             del w
             w_gu = nf4.dequant_multi([gate, up])
             n_gate = gate.weight.quant_state.shape[0]
             w_gate, w_up = w_gu[:n_gate], w_gu[n_gate:]
-            g = F.linear(x2, w_gate).contiguous()
-            u = F.linear(x2, w_up).contiguous()
+            g = _hip.linear(x2, w_gate).contiguous()
+            u = _hip.linear(x2, w_up).contiguous()
             del x2
             _hip.swiglu_bwd(dh.contiguous(), g, u, g, u)  # dg into g, du into u
             del dh
@@ -671,15 +671,15 @@ class _RecomputeMLP(torch.autograd.Function):
             dx.addmm_(u, w_up)
             return dx.view(ctx.shape), None, None, None, None, None, None, None
         w_gate, w_up, w_down = weights
-        dh = torch.matmul(dout2, w_down)
-        g = F.linear(x2, w_gate).contiguous()
-        u = F.linear(x2, w_up).contiguous()
+        dh = _hip.matmul(dout2, w_down)
+        g = _hip.linear(x2, w_gate).contiguous()
+        u = _hip.linear(x2, w_up).contiguous()
         del x2
         _hip.swiglu_bwd(dh.to(g.dtype).contiguous(), g, u, g, u)  # dg into g, du into u
         del dh
-        dx_gate = torch.matmul(g, w_gate).to(ctx.x_dtype)
+        dx_gate = _hip.matmul(g, w_gate).to(ctx.x_dtype)
         del g
-        dx_up = torch.matmul(u, w_up).to(ctx.x_dtype)
+        dx_up = _hip.matmul(u, w_up).to(ctx.x_dtype)
         return dx_gate.view(ctx.shape), dx_up.view(ctx.shape), None, None, None, None, None, None
 
 

@@ -13,10 +13,10 @@ stats: detached [N] tensors "lse", "target_logit" (0 where ignored), "ce" (0 whe
 "entropy" (fp32) and "argmax" (int64), for every row.
 
 Never materializes all N x V logits. Rows go through in chunks of `chunk_rows`: the chunk's
-logits z = x_c W^T (hipBLASLt, the weight's dtype, fp32 accumulation) land in one reused
+logits z = x_c W^T (esep_gemm or hipBLASLt, the weight's dtype, fp32 accumulation) land in one reused
 [chunk, V] buffer; the row kernel reads them once for the statistics and, when a gradient is
 wanted, rewrites the rows that carry a loss with g = (softmax - onehot) * G_SCALE; then
-dX_c = g W (hipBLASLt, fp32 out) for those rows, scaled by ce_weight / G_SCALE. The rows that
+dX_c = g W (esep_gemm or hipBLASLt, fp32 out) for those rows, scaled by ce_weight / G_SCALE. The rows that
 carry a loss are moved to the front first (a stable partition), so the g pass and the dX
 product work on a prefix of each chunk. dX is finished in the forward; the backward only
 scales it by the incoming gradient.
@@ -96,7 +96,10 @@ class _Chunks:
     def _chunk(self, r0, nr):
         rows = slice(r0, r0 + nr)
         z = self.z[:nr]
-        torch.mm(self.x16[rows], self.w16.t(), out=z)
+        if _hip.gemm_takes(self.x16[rows], self.w16, False):
+            _hip.gemm(self.x16[rows], self.w16, z)
+        else:
+            torch.mm(self.x16[rows], self.w16.t(), out=z)
         _hip.head_row_softmax(z, self.target[rows], self.cew[rows], self.lse[rows],
                               self.tlogit[rows], self.ent[rows], self.amax[rows],
                               self.want_dx, G_SCALE)
@@ -107,7 +110,10 @@ class _Chunks:
     def _dx(self, r0, nr, live):
         scale = (self.cew[r0:r0 + live] * (1.0 / G_SCALE)).unsqueeze(1)
         out = self.dx[r0:r0 + live]
-        if live < self.rows <= 2 * live:
+        if _hip.gemm_takes(self.z[:live], self.w16, True):
+            _hip.gemm(self.z[:live], self.w16, out, b_kn=True)
+            out.mul_(scale)
+        elif live < self.rows <= 2 * live:
             # hipBLASLt runs this product much faster at the chunk's full row count than at a
             # ragged one (MI355X, K = 151936, N = 1536: M = 2925 2.06 ms, M = 4096 1.67 ms), so
             # it covers the whole buffer and keeps the first `live` rows (the others hold

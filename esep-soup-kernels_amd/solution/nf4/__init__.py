@@ -99,7 +99,7 @@ class NF4Linear(torch.autograd.Function):
         w_dtype = x.dtype if x.dtype != torch.float32 else torch.float16
         w = dequantize_nf4(packed, quant_state, dtype=w_dtype)
         x2 = x if x.dtype == w_dtype else x.to(w_dtype)
-        y = torch.nn.functional.linear(x2, w, None if bias is None else bias.to(w_dtype))
+        y = _hip.linear(x2, w, None if bias is None else bias.to(w_dtype))
         ctx.packed, ctx.qs, ctx.x_dtype, ctx.w_dtype = packed, quant_state, x.dtype, w_dtype
         ctx.bias_dtype = None if bias is None else bias.dtype
         return y
@@ -111,7 +111,7 @@ class NF4Linear(torch.autograd.Function):
             dbias = dy.reshape(-1, dy.shape[-1]).sum(0, dtype=ctx.bias_dtype)
         if ctx.needs_input_grad[0]:
             w = dequantize_nf4(ctx.packed, ctx.qs, dtype=ctx.w_dtype)
-            dx = torch.matmul(dy.to(ctx.w_dtype), w).to(ctx.x_dtype)
+            dx = _hip.matmul(dy.to(ctx.w_dtype), w).to(ctx.x_dtype)
         return dx, None, dbias, None
 
 
@@ -131,7 +131,7 @@ class NF4MultiLinear(torch.autograd.Function):
         weights, states, _ = group
         w = dequantize_nf4_multi(weights, states)
         ctx.group = group
-        return torch.nn.functional.linear(x, w, bias_cat)
+        return _hip.linear(x, w, bias_cat)
 
     @staticmethod
     def backward(ctx, dy):
@@ -141,7 +141,7 @@ class NF4MultiLinear(torch.autograd.Function):
             dbias = dy.reshape(-1, dy.shape[-1]).sum(0, dtype=bias_dtype)
         if ctx.needs_input_grad[0]:
             w = dequantize_nf4_multi(weights, states)
-            dx = torch.matmul(dy if dy.dtype == w.dtype else dy.to(w.dtype), w)
+            dx = _hip.matmul(dy if dy.dtype == w.dtype else dy.to(w.dtype), w)
         return dx, dbias, None
 
 

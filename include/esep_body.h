@@ -325,6 +325,23 @@ int esep_lora_grads(const void* x, const void* a, const void* dxa, const int64_t
                     int64_t N, int r, int dt, void* stream);
 
 /*
+ * C[M, N] = A[M, K] . B (+ bias), fp16 / bf16 operands of dt, fp32 accumulation, C in dt or fp32
+ * (c_dt), for the products of the frozen projections that the vendor BLAS serves badly (the
+ * reference leaves every one to cuBLAS: solution/nf4/autograd.py:24-92). B is [N, K] (b_kn = 0) or
+ * [K, N] (b_kn = 1). K a multiple of 64, N of 8; unit column strides, row strides multiples of 8 and
+ * at least the row; 16-byte aligned pointers; a row stride times 256 rows below 4 GiB. bias [N] of
+ * dt or NULL (with C in dt only). workspace: fp32, 16-byte aligned, esep_gemm_workspace elements.
+ * Deterministic (no atomics).
+ *   esep_gemm_pays        1 where this product is expected to beat the vendor BLAS, else 0
+ *   esep_gemm_workspace   fp32 elements (0 for most sizes)
+ */
+int esep_gemm_pays(int64_t M, int64_t N, int64_t K, int b_kn);
+int64_t esep_gemm_workspace(int64_t M, int64_t N, int64_t K);
+int esep_gemm(const void* a, int64_t lda, const void* b, int64_t ldb, int b_kn, const void* bias,
+              void* c, int64_t ldc, int c_dt, float* workspace, int64_t M, int64_t N, int64_t K,
+              int dt, void* stream);
+
+/*
  * NF4 double-quant weight dequantization (QLoRA / bitsandbytes Linear4bit format). Replaces the
  * reference's Triton launch at solution/nf4/dequant.py:85-89 (dequantize_nf4; kernel math
  * dequant.py:35-57):
