@@ -10,9 +10,9 @@
 //
 // Forward mapping (flash-attention style, one pass, online softmax). A block of 4 wavefronts
 // owns 128 queries of one sequence and one query head; wavefront w owns queries 32w..32w+31 of
-// the block, heaviest query tiles first. At D = 128 the keys come in tiles of 32 moved by LDS
-// DMA through a two-buffer ring (the next tile in flight during the current one); at D = 64 in
-// tiles of 64 staged through registers and consumed in halves of 32. Scores are computed transposed, S^T = K Q^T, with
+// the block, heaviest query tiles first. The keys come in tiles of 32 (D = 128) or 64 (D = 64) moved
+// by LDS DMA through a two-buffer ring (the next tile in flight during the current one) and are
+// consumed 32 at a time. Scores are computed transposed, S^T = K Q^T, with
 // v_mfma_f32_32x32x16 (K from LDS as the A operand, the wave's Q held in registers as the B
 // operand), so each lane owns one query and 16 of a half's 32 scores; the other 16 sit in lane
 // l ^ 32, and a row max or sum is a register reduction plus one cross-half exchange. The probabilities go straight from the
@@ -63,9 +63,7 @@ struct AttnBwdArgs {
 };
 
 constexpr int kAttnBM = 128;  // queries per forward / dQ block (4 wavefronts x 32)
-constexpr int kAttnBN = 64;   // keys per tile
 constexpr int kAttnThreads = 256;
-constexpr int kAttnBQ = 64;   // queries per dK / dV tile
 
 hipError_t launch_attn_fwd(const AttnArgs& a, int dt, int D, int max_seqlen, hipStream_t s,
                            bool* supported);
@@ -94,13 +92,6 @@ struct Mfma<_Float16> {
   }
 };
 
-// Row pitch (elements) of the row-major LDS tiles: D + kRowPad. At D = 128 the pitch is 152 bf16
-// = 76 dwords, rows at bank offsets 12 r mod 64: the 8 rows a transposing operand read (ld_tr)
-// touches and the 16 rows of a 16-byte row read both spread over the banks. Measured on the
-// backward at config 5: +8 (68 dwords) 11.6 ms, +16 11.4, +24 10.8, +32 (16 r: 4-way row
-// conflicts) 13.2, +40 10.7, +48 11.0.
-constexpr int kRowPad = 24;
-
 // 2^x on the hardware's v_exp_f32 alone (no denormal-range scaling: results below 2^-126 flush
 // to 0, far below what a probability contributes next to the sums they enter).
 __device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
@@ -125,22 +116,13 @@ __device__ __forceinline__ V ld16(const void* p) {
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x8 __attribute__((ext_vector_type(8)));
 
-// A operand (8 elements) of v_mfma_f32_32x32x16 read transposed out of a row-major LDS matrix M
-// (pitch P elements): A[i][kk] = M[r0 + pi(kk)][c0 + i], i < 32, kk < 16, where pi is the
-// permuted contraction order of the score accumulators (kk 0-3, 4-7, 8-11, 12-15 -> rows 0-3,
+// Transposing operand reads (SwzTr): A operand (8 elements) of v_mfma_f32_32x32x16 read transposed
+// out of a row-major LDS matrix M: A[i][kk] = M[r0 + pi(kk)][c0 + i], i < 32, kk < 16, where pi is
+// the permuted contraction order of the score accumulators (kk 0-3, 4-7, 8-11, 12-15 -> rows 0-3,
 // 8-11, 4-7, 12-15: the rows a lane holds in its B operand). Two ds_read_b64_tr_b16: within a
 // 16-lane group the hardware hands lane j, slot k, element j % 4 of the 8-byte segment
 // addressed by lane 4 k + j / 4 (checked on the device), so lane 16 g + 4 k + m addresses row
 // r0 + 4 (g / 2) + k (+ 8 for the second read), columns c0 + 16 (g % 2) + 4 m .. + 3.
-template <typename V, int P, typename T>
-__device__ __forceinline__ V ld_tr(const T* M, int r0, int c0, int lane) {
-  const int g = lane >> 4, k = (lane >> 2) & 3, m = lane & 3;
-  T* p = const_cast<T*>(M) + (r0 + 4 * (g >> 1) + k) * P + c0 + 16 * (g & 1) + 4 * m;
-  typedef __attribute__((address_space(3))) s16x4* lds_ptr;
-  const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(p));
-  const s16x4 up = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(p + 8 * P));
-  return __builtin_bit_cast(V, __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7));
-}
 
 // One LDS DMA instruction: lane l reads the dword at g (its own address) and the wavefront
 // writes the 64 dwords to LDS bytes lds .. lds + 255 (lane l at lds + 4 l). Issued from asm so
@@ -160,16 +142,17 @@ __device__ __forceinline__ void lds_dma_dword(const void* g, const void* lds) {
 constexpr int kWaitVm0 = 0x0F70;
 
 // ---------------------------------------------------------------------------------------
-// Swizzled, unpadded LDS tiles of 256-byte token rows (D = 128, 16-bit elements), filled 1 KiB
-// per DMA instruction.
+// Swizzled, unpadded LDS tiles of RB-byte token rows (256: D = 128, 128: D = 64, 16-bit elements),
+// filled 1 KiB per DMA instruction.
 //
-// Chunk c (16 bytes) of tile row r sits at chunk position c ^ swz(r), swz(r) = 4 (r & 3) +
-// ((r >> 2) & 3): the 16 rows a row-operand read touches (one chunk each, SwzRow) and the
-// 4 rows x 4 chunks a transposing read touches in one pass (SwzTr) land on 16 different
-// positions, so neither read has bank conflicts without a pitch pad (checked on the CPU).
-// global_load_lds_dwordx4 writes lane l's 16 bytes at M0 + 16 l (checked on the device), so one
-// instruction fills 4 whole rows: lane l loads the global chunk that belongs at its position,
-// ((l & 15) ^ swz(row)) of row l >> 4 of its 4-row group.
+// Chunk c (16 bytes) of tile row r sits at chunk position c ^ swz<RB>(r): at 256 bytes swz(r) =
+// 4 (r & 3) + ((r >> 2) & 3), at 128 bytes (two rows per 256 bytes of banks) swz(r) =
+// 2 ((r >> 1) & 3) + ((r >> 3) & 1). The 16 rows a row-operand read touches (one chunk each) and
+// the 4 rows x 4 chunks (4 rows x 2 chunks at 128 bytes) a transposing read touches in one pass
+// (SwzTr) then land on different positions, so neither read has bank conflicts without a pitch
+// pad (checked on the CPU). global_load_lds_dwordx4 writes lane l's 16 bytes at M0 + 16 l (checked
+// on the device), so one instruction fills 1024 / RB whole rows: each lane loads the global chunk
+// that belongs at its position.
 // ---------------------------------------------------------------------------------------
 __device__ __forceinline__ void lds_dma_x4_s(const void* base, uint32_t voff, const void* lds) {
   const uint32_t m = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds);
@@ -180,16 +163,22 @@ __device__ __forceinline__ void lds_dma_x4(const void* g, const void* lds) {
   asm volatile("global_load_lds_dwordx4 %0, off" ::"v"(g), "{m0}"(m) : "memory");
 }
 
-__device__ __forceinline__ int swz(int r) { return 4 * (r & 3) + ((r >> 2) & 3); }
+template <int RB>
+__host__ __device__ constexpr __forceinline__ int swz(int r) {
+  static_assert(RB == 256 || RB == 128, "row bytes");
+  return RB == 256 ? 4 * (r & 3) + ((r >> 2) & 3) : 2 * ((r >> 1) & 3) + ((r >> 3) & 1);
+}
 
 // One wavefront's share of filling a ROWS-row swizzled tile from token rows r0 .. r0 + ROWS - 1
 // of a tensor (base: row 0's first element of the head; rs: bytes between token rows): with
-// NW wavefronts (a multiple of 4), wavefront w fills the 4-row groups w, w + NW, ... Rows at or
-// past rend repeat row rend - 1. A whole tile is addressed from an SGPR base; a partial one
-// clamps each lane's row.
-template <int ROWS, int NW>
+// NW wavefronts (a multiple of 4), wavefront w fills the row groups (one instruction each) w,
+// w + NW, ... Rows at or past rend repeat row rend - 1. A whole tile is addressed from an SGPR
+// base; a partial one clamps each lane's row.
+template <int ROWS, int NW, int RB = 256>
 struct SwzFill {
-  static_assert(NW % 4 == 0 && ROWS % (4 * NW) == 0, "groups per wavefront");
+  static constexpr int GR = 1024 / RB;  // rows per group: 4 or 8
+  static constexpr int CH = RB / 16;    // chunks per row
+  static_assert(NW % 4 == 0 && ROWS % (GR * NW) == 0, "groups per wavefront");
   int w, lrow, lchunk;
   int64_t rs;
   const char* cur;  // seq_begin / seq_whole: the next whole tile's first row group
@@ -197,47 +186,47 @@ struct SwzFill {
   uint32_t voff;
   __device__ __forceinline__ SwzFill(int lane, int w_, int64_t rs_)
       : w(w_), rs(rs_), cur(nullptr), tstep(0) {
-    lrow = lane >> 4;
-    lchunk = (lane & 15) ^ (4 * lrow + (w & 3));  // swz(4 q + lrow) with q & 3 = w & 3
+    lrow = lane / CH;
+    lchunk = (lane % CH) ^ swz<RB>(GR * (w & 3) + lrow);  // groups w + NW i: the same pattern
     voff = (uint32_t)(lrow * rs) + 16u * (uint32_t)lchunk;
   }
   __device__ __forceinline__ void whole(char* dst, const char* base, int r0) const {
 #pragma unroll
-    for (int i = 0; i < ROWS / (4 * NW); ++i) {
+    for (int i = 0; i < ROWS / (GR * NW); ++i) {
       const int q = w + NW * i;
-      lds_dma_x4_s(base + (int64_t)(r0 + 4 * q) * rs, voff, dst + 1024 * q);
+      lds_dma_x4_s(base + (int64_t)(r0 + GR * q) * rs, voff, dst + 1024 * q);
     }
   }
   __device__ __forceinline__ void partial(char* dst, const char* base, int r0, int rend) const {
 #pragma unroll
-    for (int i = 0; i < ROWS / (4 * NW); ++i) {
+    for (int i = 0; i < ROWS / (GR * NW); ++i) {
       const int q = w + NW * i;
-      const int r = r0 + 4 * q + lrow < rend ? r0 + 4 * q + lrow : rend - 1;
+      const int r = r0 + GR * q + lrow < rend ? r0 + GR * q + lrow : rend - 1;
       lds_dma_x4(base + (int64_t)r * rs + 16 * lchunk, dst + 1024 * q);
     }
   }
 
-  // Consecutive whole tiles: `cur` (an SGPR pair) addresses this wavefront's first 4-row group
+  // Consecutive whole tiles: `cur` (an SGPR pair) addresses this wavefront's first row group
   // of the next tile and moves ROWS rows per tile; the wavefront's other groups of a tile are
   // per-lane offsets from it. A tile then costs one 64-bit add instead of a 64-bit multiply and
   // add per DMA instruction (forward: config 5 1.46 -> 1.445 ms, the packed decoder's shape
   // 39.3 -> 38.0 us; the backward unchanged).
   __device__ __forceinline__ void seq_begin(const char* base, int r0) {
-    cur = base + (int64_t)(r0 + 4 * w) * rs;
+    cur = base + (int64_t)(r0 + GR * w) * rs;
     tstep = (int64_t)ROWS * rs;
   }
   __device__ __forceinline__ void seq_whole(char* dst) {
 #pragma unroll
-    for (int i = 0; i < ROWS / (4 * NW); ++i)
-      lds_dma_x4_s(cur, voff + (uint32_t)(4 * NW * i) * (uint32_t)rs, dst + 1024 * (w + NW * i));
+    for (int i = 0; i < ROWS / (GR * NW); ++i)
+      lds_dma_x4_s(cur, voff + (uint32_t)(GR * NW * i) * (uint32_t)rs, dst + 1024 * (w + NW * i));
     cur += tstep;
   }
 };
 
 // Two tiles of the same rows (e.g. K and V) with one whole-or-partial decision.
-template <int ROWS, int NW>
-__device__ __forceinline__ void swz_fill2(const SwzFill<ROWS, NW>& fa, char* da, const char* ba,
-                                          const SwzFill<ROWS, NW>& fb, char* db, const char* bb,
+template <int ROWS, int NW, int RB>
+__device__ __forceinline__ void swz_fill2(const SwzFill<ROWS, NW, RB>& fa, char* da, const char* ba,
+                                          const SwzFill<ROWS, NW, RB>& fb, char* db, const char* bb,
                                           int r0, int rend) {
   if (r0 + ROWS <= rend) {
     fa.whole(da, ba, r0);
@@ -250,31 +239,32 @@ __device__ __forceinline__ void swz_fill2(const SwzFill<ROWS, NW>& fa, char* da,
 
 // Row operand (A or B of v_mfma_f32_32x32x16 with the rows in lanes): lane (lq, hi) reads
 // chunk 2c + hi of tile row lq (+ 32 h for rows 32 h + lq) at byte
-// (swz_row_base(lane) ^ 32 c) + 8192 h.
+// (swz_row_base(lane) ^ 32 c) + 32 RB h.
+template <int RB = 256>
 __device__ __forceinline__ uint32_t swz_row_base(int lane) {
-  const int lq = lane & 31, hi = lane >> 5, f = swz(lq);
-  return 256u * lq + 16u * ((hi ^ f) & 1) + 32u * (f >> 1);
+  const int lq = lane & 31, hi = lane >> 5, f = swz<RB>(lq);
+  return (uint32_t)RB * lq + 16u * ((hi ^ f) & 1) + 32u * (f >> 1);
 }
 
 // Transposing operand read (ld_tr's lane mapping) out of a swizzled tile: rows rb + 4 (g >> 1)
 // + k (+ 8), columns 32 md + 16 (g & 1) + 4 m, for rb a multiple of 16. Byte offset
-// ((o_u | 64 k) ^ 64 md) + 256 rb for the lower (u = 0) and upper (u = 1) read, with
-// o_u = 256 (4 (g >> 1) + k + 8 u) + 16 L_u + 8 (m & 1) and
-// L_u = (2 (g & 1) + (m >> 1)) ^ (((g >> 1) + 2 u) & 3).
+// (o_u ^ 64 md) + RB rb for the lower (u = 0) and upper (u = 1) read, o_u being the offset of row
+// r = 4 (g >> 1) + k + 8 u, chunk (2 (g & 1) + (m >> 1)) ^ swz(r), half m & 1.
+template <int RB = 256>
 struct SwzTr {
   uint32_t o[2];
   __device__ __forceinline__ explicit SwzTr(int lane) {
     const int g = lane >> 4, k = (lane >> 2) & 3, m = lane & 3;
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      const int L = (2 * (g & 1) + (m >> 1)) ^ (((g >> 1) + 2 * u) & 3);
-      o[u] = (256u * (4 * (g >> 1) + k + 8 * u) + 16u * L + 8u * (m & 1)) | (64u * k);
+      const int r = 4 * (g >> 1) + k + 8 * u;
+      o[u] = (uint32_t)RB * r + 16u * ((2 * (g & 1) + (m >> 1)) ^ swz<RB>(r)) + 8u * (m & 1);
     }
   }
   template <typename V>
   __device__ __forceinline__ V read(const char* tile, int rb, int md) const {
     typedef __attribute__((address_space(3))) s16x4* lds_ptr;
-    const uint32_t x = 64u * md, y = 256u * rb;
+    const uint32_t x = 64u * md, y = (uint32_t)RB * rb;
     const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(tile + ((o[0] ^ x) + y)));
     const s16x4 up = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(tile + ((o[1] ^ x) + y)));
     return __builtin_bit_cast(V, __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7));
@@ -375,11 +365,9 @@ inline int attn_order(int64_t blocks, int per_cu, int n_seq) {
 }
 
 // A [ROWS x D] tile (token rows r0 .. r0 + ROWS - 1 below rend; the rest reads as 0) moved
-// through registers into LDS. load() issues every global read of the thread before any is
-// used (one memory round trip per tile, not one per chunk); the tile can be loaded before the
-// barrier that frees its LDS buffer and stored after it.
-//   rows():  thread tid holds chunks idx = tid + NT j: row idx % ROWS, 8-column chunk
-//            idx / ROWS; store_rows() writes them row-major with pitch P.
+// through registers into a swizzled LDS tile. load() issues every global read of the thread
+// before any is used (one memory round trip per tile, not one per chunk); thread tid holds chunks
+// idx = tid + NT j: row idx % ROWS, 8-column chunk idx / ROWS.
 template <typename T, int D, int ROWS, int NT = kAttnThreads>
 struct TileRows {
   static constexpr int N = ROWS * (D / 8) / NT;
@@ -396,30 +384,16 @@ struct TileRows {
     }
   }
 
-  template <int P>
-  __device__ __forceinline__ void store(T* dst, int tid) const {
+  __device__ __forceinline__ void store_swz(char* dst, int tid) const {
+    constexpr int RB = D * (int)sizeof(T);
 #pragma unroll
     for (int j = 0; j < N; ++j) {
       const int idx = tid + NT * j;
-      *reinterpret_cast<uint4*>(&dst[(idx % ROWS) * P + 8 * (idx / ROWS)]) = r[j];
+      const int row = idx % ROWS, chunk = idx / ROWS;
+      *reinterpret_cast<uint4*>(dst + RB * row + 16 * (chunk ^ swz<RB>(row))) = r[j];
     }
   }
-
-  // the same rows into a swizzled, unpadded tile (256-byte rows: D = 128 of 16-bit elements;
-  // chunk c of row r at position c ^ swz(r))
-  __device__ __forceinline__ void store_swz(char* dst, int tid) const;
 };
-
-template <typename T, int D, int ROWS, int NT>
-__device__ __forceinline__ void TileRows<T, D, ROWS, NT>::store_swz(char* dst, int tid) const {
-  static_assert(D * sizeof(T) == 256, "swizzled tiles have 256-byte rows");
-#pragma unroll
-  for (int j = 0; j < N; ++j) {
-    const int idx = tid + NT * j;
-    const int row = idx % ROWS, chunk = idx / ROWS;
-    *reinterpret_cast<uint4*>(dst + 256 * row + 16 * (chunk ^ swz(row))) = r[j];
-  }
-}
 
 // Store a wavefront's [32 tokens x D] result held transposed in MFMA accumulators (acc[md]
 // element 4 j + e is column 32 md + 8 j + 4 hi + e of token `row`), times `mul`.
