@@ -64,9 +64,11 @@ def _fused(rank, *mats):
     if rank % 8 or not 8 <= rank <= 64:
         return False
     for t in mats:
-        if (not t.is_cuda or t.dim() != 2 or t.dtype not in (torch.float16, torch.bfloat16)
-                or not 0 < t.shape[0] <= 1 << 22 or t.shape[1] % 8 or not t.shape[1]
-                or t.stride(1) != 1 or t.stride(0) % 8 or t.stride(0) < t.shape[1]
+        if not t.is_cuda or t.dim() != 2 or t.dtype not in (torch.float16, torch.bfloat16):
+            return False
+        rows, width = t.shape
+        ld, col = t.stride()
+        if (not 0 < rows <= 1 << 22 or width % 8 or not width or col != 1 or ld % 8 or ld < width
                 or t.data_ptr() % 16):
             return False
     return True
@@ -182,7 +184,8 @@ def _rows_mm(t, dtype):
 
 class _LoRATerm:
     """The parts both Functions share: set up the forward (compute dtype, casts, key, xa) and
-    turn the term's gradient into (dx, dA, dB) in the dtypes autograd expects."""
+    turn the term's gradient into (dx, dA, dB) in the dtypes autograd expects. ctx.fused: the
+    fused products take x, the rank and the output width (everything between them is dense)."""
 
     @staticmethod
     def begin(ctx, x, weight_a, weight_b, p, scaling):
@@ -190,7 +193,13 @@ class _LoRATerm:
         x2 = _rows(x, dtype)
         a16, b16 = cast_lora_weights(weight_a, weight_b, dtype)
         key = new_dropout_key(x2.device) if p > 0.0 else None
-        xa = lora_down_fwd(x2, a16, key, p)
+        ctx.fused = (_fused(a16.shape[0], x2, a16, b16) and a16.is_contiguous()
+                     and b16.is_contiguous() and b16.shape[0] % 8 == 0)
+        if ctx.fused:
+            xa = torch.empty((x2.shape[0], a16.shape[0]), device=x2.device, dtype=dtype)
+            _hip.lora_down(x2, a16, xa, key=key, p=p)
+        else:
+            xa = lora_down_fwd(x2, a16, key, p)
         ctx.save_for_backward(x2, xa, a16, b16, key)
         ctx.p, ctx.scaling, ctx.dtype = p, scaling, dtype
         ctx.x_shape, ctx.x_dtype = x.shape, x.dtype
@@ -202,7 +211,7 @@ class _LoRATerm:
         x2, xa, a16, b16, key = ctx.saved_tensors
         need = ctx.needs_input_grad
         dt2 = _rows_mm(dterm, ctx.dtype)
-        if _up_bwd_fused(dt2, xa, b16) and _grads_fused(x2, a16, xa):
+        if ctx.fused and _fused(b16.shape[1], dt2):
             # dx, dA and dB in one launch after dxa
             dxa = _dxa(dt2, b16, ctx.scaling)
             dx = torch.empty_like(x2) if need[x_index] else None
@@ -213,8 +222,9 @@ class _LoRATerm:
         else:
             dxa, db = lora_up_bwd(dt2, xa, b16, ctx.scaling)
             dx, da = lora_down_bwd(x2, a16, dxa, key, ctx.p, need_dx=need[x_index])
-        return (dx.view(ctx.x_shape).to(ctx.x_dtype) if dx is not None else None,
-                da.to(ctx.a_dtype) if need[a_index] else None,
+        if dx is not None and (dx.shape != ctx.x_shape or dx.dtype != ctx.x_dtype):
+            dx = dx.view(ctx.x_shape).to(ctx.x_dtype)
+        return (dx, da.to(ctx.a_dtype) if need[a_index] else None,
                 db.to(ctx.b_dtype) if need[a_index + 1] else None)
 
 
@@ -229,14 +239,14 @@ class LoRAFunction(torch.autograd.Function):
         ctx.base_dtype = base.dtype
         if base.dtype == ctx.dtype and base.is_contiguous() and not base._is_view():
             flat = base.view(-1, base.shape[-1])
-            if _fused(b16.shape[1], flat, xa, b16) and xa.is_contiguous() and b16.is_contiguous():
+            if ctx.fused and _fused(b16.shape[1], flat):
                 _hip.lora_up(xa, b16, flat, scaling, base=flat)
             else:
                 flat.addmm_(xa, b16.t(), alpha=scaling)
             ctx.mark_dirty(base)
             return base
         flat = base.reshape(-1, base.shape[-1]).to(ctx.dtype)
-        if _fused(b16.shape[1], flat, xa, b16) and xa.is_contiguous() and b16.is_contiguous():
+        if ctx.fused and _fused(b16.shape[1], flat):
             out = torch.empty(flat.shape, device=flat.device, dtype=flat.dtype)
             _hip.lora_up(xa, b16, out, scaling, base=flat)
             return out.view(base.shape)
@@ -256,7 +266,11 @@ class LoRADeltaFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight_a, weight_b, p, scaling):
         xa, b16 = _LoRATerm.begin(ctx, x, weight_a, weight_b, p, scaling)
-        term = lora_delta(xa, b16, scaling)
+        if ctx.fused:
+            term = torch.empty((xa.shape[0], b16.shape[0]), device=xa.device, dtype=xa.dtype)
+            _hip.lora_up(xa, b16, term, scaling)
+        else:
+            term = lora_delta(xa, b16, scaling)
         return term.view(*x.shape[:-1], term.shape[-1])
 
     @staticmethod

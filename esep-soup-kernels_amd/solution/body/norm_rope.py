@@ -36,7 +36,6 @@ rmsnorm(x, weight, eps, out_dtype=None, recompute_rstd=False) -> y
 
 import math
 import threading
-import weakref
 
 import torch
 
@@ -88,7 +87,9 @@ def special_channels(weight):
 def _weight_f32(weight, grad):
     """The norm weight as the kernels read it: contiguous fp32 [H]. Differentiable when the
     weight gets a gradient (the cast's backward returns dw in the weight's dtype)."""
-    w = weight if grad else weight.detach()
+    w = weight if grad or not weight.requires_grad else weight.detach()
+    if w.dtype is torch.float32 and w.is_contiguous():
+        return w
     return w.to(torch.float32).contiguous()
 
 
@@ -98,8 +99,7 @@ def _wants_weight_grad(weight):
 
 def _rows_of(t, dtype=None):
     """t [..., n] as a dense [rows, n] tensor (optionally cast): the kernels' row layout."""
-    n = t.shape[-1]
-    flat = t.reshape(-1, n)
+    flat = t if t.dim() == 2 else t.reshape(-1, t.shape[-1])
     if dtype is not None and flat.dtype != dtype:
         flat = flat.to(dtype)
     return flat.contiguous()
@@ -192,6 +192,9 @@ class _PassToken:
     def __init__(self, task):
         self.task = task
 
+    def __del__(self):
+        _drop_task(self.task)
+
 
 def _drop_task(task):
     with _defer_lock:
@@ -217,7 +220,6 @@ def _defer(leaf, partials):
             entries = _deferred[task] = []
     if first:
         token = _PassToken(task)
-        weakref.finalize(token, _drop_task, task)
         try:
             queue_callback(lambda: _finish_deferred(token))
         except Exception:
@@ -331,7 +333,7 @@ class AddRMSNorm(torch.autograd.Function):
             (x, rstd, w), slots, xs = ctx.saved_tensors, None, None
         n = x.shape[-1]
         rows = x.shape[0]
-        dys = [d.reshape(-1, n).contiguous() for d in dys if d is not None]
+        dys = [_rows_of(d) for d in dys if d is not None]
         has_dr = dr_out is not None
         want_r = ctx.needs_input_grad[0]
         write_dd = ctx.has_delta and ctx.needs_input_grad[1]
@@ -343,7 +345,7 @@ class AddRMSNorm(torch.autograd.Function):
         dr = torch.empty((rows, n), device=dev, dtype=torch.float32) if want_r else None
         ddelta = torch.empty((rows, n), device=dev, dtype=ctx.delta_dtype) if write_dd else None
         dw, partials = _weight_grad_target(ctx, w, rows, 2)
-        dr2 = dr_out.reshape(-1, n).to(torch.float32).contiguous() if has_dr else None
+        dr2 = _rows_of(dr_out, torch.float32) if has_dr else None
         if rows > 0 and (dr is not None or ddelta is not None or want_w):
             _hip.rmsnorm_bwd(dys, x, w, ctx.eps, from_y=ctx.from_y, rstd=rstd, dr_out=dr2,
                              slot=slots if ctx.n_special else None, xs=xs,
@@ -436,7 +438,7 @@ class RMSNorm(torch.autograd.Function):
         dx = torch.empty((rows, n), device=x2.device, dtype=x2.dtype) if want_x else None
         dw, partials = _weight_grad_target(ctx, w, rows, 1)
         if rows > 0 and (want_x or want_w):
-            dy2 = dy.reshape(-1, n).contiguous()
+            dy2 = _rows_of(dy)
             out = dict(dr=dx) if x2.dtype == torch.float32 else dict(dx=dx)
             _hip.rmsnorm_bwd([dy2], x2, w, ctx.eps, rstd=rstd, dw=dw, partials=partials, **out)
             if partials is not None:

@@ -43,11 +43,18 @@ def supported(quant_state) -> bool:
         return False
 
 
+def _f32(t):
+    """A table of the quant state as the kernel reads it: dense fp32 (as it is stored)."""
+    if t.dtype is torch.float32 and t.is_contiguous():
+        return t
+    return t.to(torch.float32).contiguous()
+
+
 def _offset(qs):
     off = qs.offset
     if not isinstance(off, torch.Tensor):
         off = torch.tensor([float(off)], dtype=torch.float32, device=qs.absmax.device)
-    return off.reshape(1).to(torch.float32)
+    return off if off.dtype is torch.float32 and off.numel() == 1 else off.reshape(1).to(torch.float32)
 
 
 def dequantize_nf4(packed, quant_state, out=None, dtype=torch.float16):
@@ -57,10 +64,8 @@ def dequantize_nf4(packed, quant_state, out=None, dtype=torch.float16):
     if out is None:
         out = torch.empty(shape, dtype=dtype, device=packed.device)
     qs2 = quant_state.state2
-    _hip.nf4_dequant(packed.reshape(-1) if packed.is_contiguous() else packed.contiguous().reshape(-1),
-                     quant_state.absmax, qs2.absmax.to(torch.float32).contiguous(),
-                     qs2.code.to(torch.float32).contiguous(), _offset(quant_state),
-                     quant_state.code.to(torch.float32).contiguous(), out.reshape(-1))
+    _hip.nf4_dequant(packed.contiguous(), quant_state.absmax, _f32(qs2.absmax), _f32(qs2.code),
+                     _offset(quant_state), _f32(quant_state.code), out)
     return out
 
 
@@ -78,10 +83,8 @@ def dequantize_nf4_multi(weights, quant_states, out=None, dtype=torch.float16):
     items, r = [], 0
     for w, qs in zip(weights, quant_states):
         qs2 = qs.state2
-        items.append((w.reshape(-1) if w.is_contiguous() else w.contiguous().reshape(-1),
-                      qs.absmax.contiguous(), qs2.absmax.to(torch.float32).contiguous(),
-                      qs2.code.to(torch.float32).contiguous(), _offset(qs),
-                      qs.code.to(torch.float32).contiguous(), out[r:r + qs.shape[0]].reshape(-1)))
+        items.append((w.contiguous(), qs.absmax.contiguous(), _f32(qs2.absmax), _f32(qs2.code),
+                      _offset(qs), _f32(qs.code), out[r:r + qs.shape[0]]))
         r += qs.shape[0]
     for i in range(0, len(items), _hip.NF4_MULTI_MAX):
         _hip.nf4_dequant_multi(items[i:i + _hip.NF4_MULTI_MAX])
