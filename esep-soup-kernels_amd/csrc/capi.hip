@@ -916,9 +916,10 @@ int esep_nf4_dequant_multi(const esep_nf4_weight* weights, int n_weights, int ou
   return e == hipSuccess ? 0 : hip_fail(e, "nf4_dequant_multi launch");
 }
 
-int esep_head_row_softmax(void* z, int64_t ld, const int64_t* target, const float* cew,
-                          float* lse, float* tlogit, float* ent, int32_t* amax, int64_t rows,
-                          int64_t V, int write_g, float g_scale, int dt, void* stream) {
+namespace {
+int head_rows(void* z, int64_t ld, const int64_t* target, const float* cew, const int32_t* perm,
+              float* lse, float* tlogit, float* ce, float* ent, int32_t* amax, int64_t* amax64,
+              int64_t rows, int64_t V, int write_g, float g_scale, int dt, void* stream) {
   g_err[0] = 0;
   if (dt != ESEP_F16 && dt != ESEP_BF16)
     return fail(ESEP_EINVAL, "head_row_softmax: logits must be fp16 or bf16 (dtype code %d)", dt);
@@ -930,18 +931,82 @@ int esep_head_row_softmax(void* z, int64_t ld, const int64_t* target, const floa
                           (long long)V);
   if (rows == 0) return 0;
   if (z == nullptr || target == nullptr || lse == nullptr || tlogit == nullptr || ent == nullptr ||
-      amax == nullptr || (write_g && cew == nullptr))
+      (amax == nullptr && amax64 == nullptr) || (write_g && cew == nullptr))
     return fail(ESEP_EINVAL, "head_row_softmax: z, target, lse, tlogit, ent, amax (and cew with "
                              "write_g) are required");
   if (reinterpret_cast<uintptr_t>(z) & 1)
     return fail(ESEP_EALIGN, "head_row_softmax: z must be 2-byte aligned");
   const bool vec = aligned16(z) && (ld & 7) == 0 && (V & 7) == 0;
-  esep::HeadArgs a{z, target, cew, lse, tlogit, ent, amax, rows, ld, V, g_scale, write_g ? 1 : 0};
+  esep::HeadArgs a{z,  target, cew,     lse,             tlogit, ent,    amax, rows, ld,
+                   V,  g_scale, write_g ? 1 : 0, ce,     amax64, perm};
   bool sup = false;
   const hipError_t e =
       esep::launch_head_row(a, dt, vec, static_cast<hipStream_t>(stream), &sup);
   if (!sup) return fail(ESEP_EINVAL, "head_row_softmax: unsupported dtype");
   return e == hipSuccess ? 0 : hip_fail(e, "head_row_softmax launch");
+}
+}  // namespace
+
+int esep_head_row_softmax(void* z, int64_t ld, const int64_t* target, const float* cew,
+                          float* lse, float* tlogit, float* ent, int32_t* amax, int64_t rows,
+                          int64_t V, int write_g, float g_scale, int dt, void* stream) {
+  return head_rows(z, ld, target, cew, nullptr, lse, tlogit, nullptr, ent, amax, nullptr, rows, V,
+                   write_g, g_scale, dt, stream);
+}
+
+int esep_head_rows(void* z, int64_t ld, const int64_t* target, const float* cew,
+                   const int32_t* perm, float* lse, float* tlogit, float* ce, float* ent,
+                   int64_t* amax, int64_t rows, int64_t V, int write_g, float g_scale, int dt,
+                   void* stream) {
+  g_err[0] = 0;
+  if (ce == nullptr) return fail(ESEP_EINVAL, "head_rows: ce is required");
+  return head_rows(z, ld, target, cew, perm, lse, tlogit, ce, ent, nullptr, amax, rows, V, write_g,
+                   g_scale, dt, stream);
+}
+
+int esep_head_partition(const int64_t* target, const float* cew, int64_t N, int64_t V,
+                        int32_t* perm, int32_t* inv, int32_t* n_live, void* stream) {
+  g_err[0] = 0;
+  if (N < 1 || N > 0x7fffffffLL || V < 1)
+    return fail(ESEP_ESHAPE, "head_partition: N=%lld, V=%lld", (long long)N, (long long)V);
+  if (target == nullptr || cew == nullptr || perm == nullptr || inv == nullptr ||
+      n_live == nullptr)
+    return fail(ESEP_EINVAL, "head_partition: every pointer is required");
+  const hipError_t e = esep::launch_head_partition(target, cew, N, V, perm, inv, n_live,
+                                                   static_cast<hipStream_t>(stream));
+  return e == hipSuccess ? 0 : hip_fail(e, "head_partition launch");
+}
+
+int esep_head_loss(const int64_t* target, const float* cew, const float* ce, int64_t N, int64_t V,
+                   float* loss, void* stream) {
+  g_err[0] = 0;
+  if (N < 1 || V < 1)
+    return fail(ESEP_ESHAPE, "head_loss: N=%lld, V=%lld", (long long)N, (long long)V);
+  if (target == nullptr || cew == nullptr || ce == nullptr || loss == nullptr)
+    return fail(ESEP_EINVAL, "head_loss: every pointer is required");
+  const hipError_t e = esep::launch_head_loss(target, cew, ce, N, V, loss,
+                                              static_cast<hipStream_t>(stream));
+  return e == hipSuccess ? 0 : hip_fail(e, "head_loss launch");
+}
+
+int esep_head_dx(const float* prod, int64_t n_live, const int32_t* inv, const float* cew,
+                 const float* dloss, float g_scale, void* dx, int dx_dt, int64_t N, int64_t H,
+                 void* stream) {
+  g_err[0] = 0;
+  if (!float_dt(dx_dt)) return fail(ESEP_EINVAL, "head_dx: bad dtype code %d", dx_dt);
+  if (N < 1 || H < 8 || H % 8 != 0 || n_live < 0 || n_live > N || H > (1 << 24) ||
+      N * (H / 8) > (1LL << 38))
+    return fail(ESEP_ESHAPE, "head_dx: N=%lld, H=%lld, n_live=%lld", (long long)N, (long long)H,
+                (long long)n_live);
+  if ((n_live > 0 && prod == nullptr) || inv == nullptr || cew == nullptr || dloss == nullptr ||
+      dx == nullptr || g_scale == 0.f)
+    return fail(ESEP_EINVAL, "head_dx: every pointer and a nonzero scale are required");
+  if (!aligned16(prod) || !aligned16(dx))
+    return fail(ESEP_EALIGN, "head_dx: prod and dx need 16-byte alignment");
+  const hipError_t e =
+      esep::launch_head_dx(prod, n_live, inv, cew, dloss, 1.f / g_scale, dx, dx_dt, N, H,
+                           static_cast<hipStream_t>(stream));
+  return e == hipSuccess ? 0 : hip_fail(e, "head_dx launch");
 }
 
 }  // extern "C"

@@ -89,6 +89,7 @@ __global__ __launch_bounds__(kHeadThreads) void k_head_row(const HeadArgs a) {
   __shared__ float m_sh, log2s_sh;
   __shared__ int amin_sh;
   const int64_t row = blockIdx.x;
+  const int64_t at = a.perm != nullptr ? a.perm[row] : row;  // its place in the per-row arrays
   const int V = (int)a.V;
   const int nch = (V + 7) >> 3;
   const T* zrow = static_cast<const T*>(a.z) + row * a.ld;
@@ -149,10 +150,14 @@ __global__ __launch_bounds__(kHeadThreads) void k_head_row(const HeadArgs a) {
     RowState r = red[0];
     for (int w = 1; w < kHeadWaves; ++w) r = merge(r, red[w]);
     const float log2s = log2f(r.s);
-    a.lse[row] = fmaf(log2s, kLn2, r.m);
-    a.ent[row] = (log2s - r.t / r.s) * kLn2;
-    const int64_t tg = a.target[row];
-    a.tlogit[row] = (tg >= 0 && tg < a.V) ? Elt<T>::to_f(zrow[tg]) : 0.f;
+    const float lse = fmaf(log2s, kLn2, r.m);
+    a.lse[at] = lse;
+    a.ent[at] = (log2s - r.t / r.s) * kLn2;
+    const int64_t tg = a.target[at];
+    const bool has = tg >= 0 && tg < a.V;
+    const float tl = has ? Elt<T>::to_f(zrow[tg]) : 0.f;
+    a.tlogit[at] = tl;
+    if (a.ce != nullptr) a.ce[at] = has ? lse - tl : 0.f;
     m_sh = r.m;
     log2s_sh = log2s;
   }
@@ -173,13 +178,19 @@ __global__ __launch_bounds__(kHeadThreads) void k_head_row(const HeadArgs a) {
     atomicMin(&amin_sh, best);
   }
   __syncthreads();
-  if (tid == 0) a.amax[row] = amin_sh;
-  if (!a.write_g || a.cew[row] == 0.f) return;  // uniform over the block
+  if (tid == 0) {
+    if (a.amax64 != nullptr)
+      a.amax64[at] = amin_sh;
+    else
+      a.amax[at] = amin_sh;
+  }
+  if (!a.write_g || a.cew[at] == 0.f) return;  // uniform over the block
 
   // ---- pass 2: g = (softmax - onehot) * g_scale, in place ----
   const float l2s = log2s_sh;
   const float gs = a.g_scale;
-  const int64_t tg = a.target[row];
+  const int64_t tg = a.target[at];
+  if (a.ce != nullptr && !(tg >= 0 && tg < a.V)) return;
   const int tch = (tg >= 0 && tg < a.V) ? (int)(tg >> 3) : -1;
   for (int c0 = tid; c0 < nch; c0 += kStep) {
     const bool full = c0 - lane + (kWave - 1) + (kBatch - 1) * kHeadThreads < nch;
@@ -199,6 +210,92 @@ __global__ __launch_bounds__(kHeadThreads) void k_head_row(const HeadArgs a) {
       if (c < nch) Buf<T>::template store<VEC, kStream>(sp, (uint32_t)c * 16u, gv);
     }
   }
+}
+
+// One block: thread t owns the rows t per .. (t + 1) per - 1; their live counts are scanned over the
+// block, then every thread places its rows. A few thousand rows of 12 bytes: latency-bound, one
+// launch in place of the eleven (compare, nonzero twice, concatenate, sum, scatter, ...) that a
+// partition takes from tensor operations (N = 5000: about 60 us of kernels, here 9).
+constexpr int kPartThreads = 1024;
+
+__device__ __forceinline__ bool row_live(const int64_t* target, const float* cew, int64_t i,
+                                         int64_t V) {
+  const int64_t t = target[i];
+  return t >= 0 && t < V && cew[i] != 0.f;
+}
+
+__global__ __launch_bounds__(kPartThreads) void k_head_partition(const int64_t* target,
+                                                                 const float* cew, int64_t N,
+                                                                 int64_t V, int32_t* perm,
+                                                                 int32_t* inv, int32_t* n_live) {
+  __shared__ int wave_sum_sh[kPartThreads / kWave];
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), w = tid / kWave;
+  const int64_t per = (N + kPartThreads - 1) / kPartThreads;
+  const int64_t i0 = tid * per < N ? tid * per : N, i1 = i0 + per < N ? i0 + per : N;
+  int mine = 0;
+  for (int64_t i = i0; i < i1; ++i) mine += row_live(target, cew, i, V) ? 1 : 0;
+  int scan = mine;  // inclusive over the wavefront
+#pragma unroll
+  for (int h = 1; h < kWave; h <<= 1) {
+    const int o = __shfl_up(scan, h);
+    if (lane >= h) scan += o;
+  }
+  if (lane == kWave - 1) wave_sum_sh[w] = scan;
+  __syncthreads();
+  int before = 0, total = 0;
+  for (int v = 0; v < kPartThreads / kWave; ++v) {
+    if (v < w) before += wave_sum_sh[v];
+    total += wave_sum_sh[v];
+  }
+  int64_t live = before + scan - mine, dead = total + (i0 - live);
+  for (int64_t i = i0; i < i1; ++i) {
+    const int64_t at = row_live(target, cew, i, V) ? live++ : dead++;
+    perm[at] = (int32_t)i;
+    inv[i] = (int32_t)at;
+  }
+  if (tid == 0) *n_live = total;
+}
+
+// Fixed order: thread t sums rows t, t + 1024, ..., then the block's tree.
+__global__ __launch_bounds__(kPartThreads) void k_head_loss(const int64_t* target, const float* cew,
+                                                            const float* ce, int64_t N, int64_t V,
+                                                            float* loss) {
+  __shared__ float red[kPartThreads / kWave];
+  float s = 0.f;
+  for (int64_t i = threadIdx.x; i < N; i += kPartThreads) {
+    const int64_t t = target[i];
+    if (t >= 0 && t < V) s = fmaf(cew[i], ce[i], s);
+  }
+  s = wave_sum(s);
+  if ((threadIdx.x & (kWave - 1)) == 0) red[threadIdx.x / kWave] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    float r = 0.f;
+    for (int v = 0; v < kPartThreads / kWave; ++v) r += red[v];
+    *loss = r;
+  }
+}
+
+// The product's rows back in place, scaled and cast in one pass (8 columns per thread), where a
+// multiply, a gather, another multiply and a cast took four.
+template <typename O>
+__global__ __launch_bounds__(256) void k_head_dx(const float* prod, int64_t n_live,
+                                                 const int32_t* inv, const float* cew,
+                                                 const float* dloss, float inv_scale, O* dx,
+                                                 int64_t N, int per) {
+  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t i = e / per;
+  if (i >= N) return;
+  const int c = (int)(e % per);
+  const int64_t at = inv[i];
+  float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  if (at < n_live) {
+    Chunk<float>::load(prod + at * 8 * per + 8 * c, v);
+    const float s = cew[i] * inv_scale, d = *dloss;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = v[k] * s * d;
+  }
+  Chunk<O>::store(dx + i * 8 * per + 8 * c, v);
 }
 
 template <typename T>
@@ -223,6 +320,38 @@ hipError_t launch_head_row(const HeadArgs& a, int dt, bool vec, hipStream_t s, b
     *supported = false;
     return hipErrorInvalidValue;
   }
+  return hipGetLastError();
+}
+
+hipError_t launch_head_partition(const int64_t* target, const float* cew, int64_t N, int64_t V,
+                                 int32_t* perm, int32_t* inv, int32_t* n_live, hipStream_t s) {
+  hipLaunchKernelGGL(k_head_partition, dim3(1), dim3(kPartThreads), 0, s, target, cew, N, V, perm,
+                     inv, n_live);
+  return hipGetLastError();
+}
+
+hipError_t launch_head_loss(const int64_t* target, const float* cew, const float* ce, int64_t N,
+                            int64_t V, float* loss, hipStream_t s) {
+  hipLaunchKernelGGL(k_head_loss, dim3(1), dim3(kPartThreads), 0, s, target, cew, ce, N, V, loss);
+  return hipGetLastError();
+}
+
+hipError_t launch_head_dx(const float* prod, int64_t n_live, const int32_t* inv, const float* cew,
+                          const float* dloss, float inv_scale, void* dx, int dx_dt, int64_t N,
+                          int64_t H, hipStream_t s) {
+  const int per = (int)(H / 8);
+  const dim3 grid((unsigned)((N * per + 255) / 256));
+  auto go = [&](auto tag) {
+    using O = decltype(tag);
+    hipLaunchKernelGGL((k_head_dx<O>), grid, dim3(256), 0, s, prod, n_live, inv, cew, dloss,
+                       inv_scale, static_cast<O*>(dx), N, per);
+  };
+  if (dx_dt == 0)
+    go(float{});
+  else if (dx_dt == 1)
+    go(_Float16{});
+  else
+    go(__bf16{});
   return hipGetLastError();
 }
 

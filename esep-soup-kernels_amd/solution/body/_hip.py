@@ -62,6 +62,11 @@ SIGNATURES = {
     "esep_lora_grads_workspace": (_i64, [_i64, _i64, _i64, _i32]),
     "esep_lora_grads": (_i32, [_vp, _vp, _vp, _vp, _f32, _vp, _i32, _vp, _vp, _i64, _vp, _f32, _vp,
                                _vp, _i64, _i64, _i64, _i32, _i32, _vp]),
+    "esep_head_rows": (_i32, [_vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i32,
+                              _f32, _i32, _vp]),
+    "esep_head_partition": (_i32, [_vp, _vp, _i64, _i64, _vp, _vp, _vp, _vp]),
+    "esep_head_loss": (_i32, [_vp, _vp, _vp, _i64, _i64, _vp, _vp]),
+    "esep_head_dx": (_i32, [_vp, _i64, _vp, _vp, _vp, _f32, _vp, _i32, _i64, _i64, _vp]),
     "esep_gemm_pays": (_i32, [_i64, _i64, _i64, _i32]),
     "esep_gemm_workspace": (_i64, [_i64, _i64, _i64]),
     "esep_gemm": (_i32, [_vp, _i64, _vp, _i64, _i32, _vp, _vp, _i64, _i32, _vp, _i64, _i64, _i64,
@@ -613,16 +618,19 @@ def gemm(a, b, out, b_kn=False, bias=None, name="_gemm"):
     _record(name)
 
 
-def _no_cast(a):
-    return (not torch.is_autocast_enabled("cuda")
-            or torch.get_autocast_dtype("cuda") == a.dtype)
+def _plain(x):
+    """No cast and no graph is expected of a product with x (autocast to another dtype, a backward
+    pass that is itself recorded)."""
+    if torch.is_grad_enabled() and x.requires_grad:
+        return False
+    return not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == x.dtype
 
 
 def linear(x, w, bias=None):
-    """F.linear(x, w, bias) without autograd: esep_gemm where it takes the operands and pays, else
-    the vendor BLAS."""
+    """F.linear(x, w, bias) for autograd Functions: esep_gemm where it takes the operands and pays,
+    else the vendor BLAS (which also serves a recorded backward pass)."""
     x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
-    if (_no_cast(x) and gemm_takes(x2, w, False)
+    if (_plain(x) and gemm_takes(x2, w, False)
             and (bias is None or (bias.dtype == x.dtype and bias.dim() == 1 and bias.is_contiguous()
                                   and bias.data_ptr() % 16 == 0))):
         out = torch.empty((x2.shape[0], w.shape[0]), device=x.device, dtype=x.dtype)
@@ -632,10 +640,9 @@ def linear(x, w, bias=None):
 
 
 def matmul(x, w):
-    """x @ w for a 2-D w [K, N] without autograd: esep_gemm where it takes the operands and pays, else
-    the vendor BLAS."""
+    """x @ w for a 2-D w [K, N], as linear."""
     x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
-    if _no_cast(x) and gemm_takes(x2, w, True):
+    if _plain(x) and gemm_takes(x2, w, True):
         out = torch.empty((x2.shape[0], w.shape[1]), device=x.device, dtype=x.dtype)
         gemm(x2, w, out, b_kn=True)
         return out.view(*x.shape[:-1], w.shape[1])
@@ -706,22 +713,91 @@ def nf4_dequant_multi(items, name="_nf4_dequant_multi"):
     _record(name)
 
 
-def head_row_softmax(z, target, cew, lse, tlogit, ent, amax, write_g, g_scale,
+def head_row_softmax(z, target, cew, lse, tlogit, ent, amax, write_g, g_scale, perm=None, ce=None,
                      name="head_row_softmax_kernel"):
     """Softmax statistics of the logits chunk z [rows, V] (fp16 / bf16, unit column stride) and,
     with write_g, g = (softmax - onehot) * g_scale written over the rows whose cew is != 0
     (esep_head_row_softmax). target int64 [rows]; cew fp32 [rows]; lse / tlogit / ent fp32 and
-    amax int32 outputs of [rows]."""
-    dev = _dev(z, target, cew, lse, tlogit, ent, amax)
+    amax int32 outputs of [rows].
+    With ce (fp32), esep_head_rows: amax is int64, ce gets lse - tlogit (0 without a target), and g
+    is written only over rows that also have a target. perm (int32 [rows]): the chunk's row i is
+    row perm[i] of target, cew and the outputs, which are then of any (common) length."""
+    dev = _dev(z, target, cew, lse, tlogit, ent, amax, perm, ce)
     rows, V = z.shape
     ld = _rows_ld(z, V)
+    n = rows if perm is None else target.numel()
     for t, dt, nm in ((target, torch.int64, "target"), (cew, torch.float32, "cew"),
                       (lse, torch.float32, "lse"), (tlogit, torch.float32, "tlogit"),
-                      (ent, torch.float32, "ent"), (amax, torch.int32, "amax")):
-        if t.dtype != dt or t.numel() != rows or (rows > 1 and t.stride(0) != 1):
-            raise EsepError(f"{nm} must be a contiguous {dt} tensor of {rows} elements")
-    rc = lib().esep_head_row_softmax(_p(z), ld, _p(target), _p(cew), _p(lse), _p(tlogit), _p(ent),
-                                     _p(amax), rows, V, 1 if write_g else 0, float(g_scale),
-                                     dtype_code(z.dtype), _stream(dev))
+                      (ent, torch.float32, "ent"), (ce, torch.float32, "ce"),
+                      (amax, torch.int32 if ce is None else torch.int64, "amax")):
+        if t is not None and (t.dtype != dt or t.numel() != n or (n > 1 and t.stride(0) != 1)):
+            raise EsepError(f"{nm} must be a contiguous {dt} tensor of {n} elements")
+    if ce is None:
+        if perm is not None:
+            raise EsepError("perm needs ce")
+        rc = lib().esep_head_row_softmax(_p(z), ld, _p(target), _p(cew), _p(lse), _p(tlogit),
+                                         _p(ent), _p(amax), rows, V, 1 if write_g else 0,
+                                         float(g_scale), dtype_code(z.dtype), _stream(dev))
+    else:
+        if perm is not None and (perm.dtype != torch.int32 or perm.numel() != rows
+                                 or not perm.is_contiguous()):
+            raise EsepError(f"perm must be a contiguous int32 tensor of {rows} elements")
+        rc = lib().esep_head_rows(_p(z), ld, _p(target), _p(cew), _p(perm), _p(lse), _p(tlogit),
+                                  _p(ce), _p(ent), _p(amax), rows, V, 1 if write_g else 0,
+                                  float(g_scale), dtype_code(z.dtype), _stream(dev))
     _check(rc, "esep_head_row_softmax")
+    _record(name)
+
+
+def _head_rows_args(target, cew):
+    if (target.dtype != torch.int64 or cew.dtype != torch.float32 or target.dim() != 1
+            or target.shape != cew.shape or not target.is_contiguous() or not cew.is_contiguous()):
+        raise EsepError("target int64 [N] and cew fp32 [N], contiguous")
+
+
+def head_partition(target, cew, V, name="_head_partition"):
+    """(perm, inv, n_live): the rows with a target in [0, V) and a nonzero cew first, each part in
+    its order (esep_head_partition). perm[i] is the row at place i, inv its inverse (int32 [N]),
+    n_live int32 [1], all on the device."""
+    _head_rows_args(target, cew)
+    dev = _dev(target, cew)
+    N = target.numel()
+    perm, inv = (torch.empty(N, device=dev, dtype=torch.int32) for _ in range(2))
+    n_live = torch.empty(1, device=dev, dtype=torch.int32)
+    rc = lib().esep_head_partition(_p(target), _p(cew), N, int(V), _p(perm), _p(inv), _p(n_live),
+                                   _stream(dev))
+    _check(rc, "esep_head_partition")
+    _record(name)
+    return perm, inv, n_live
+
+
+def head_loss(target, cew, ce, V, name="_head_loss"):
+    """sum of cew * ce over the rows with a target in [0, V), a 0-dim fp32 tensor
+    (esep_head_loss)."""
+    _head_rows_args(target, cew)
+    dev = _dev(target, cew, ce)
+    if ce.dtype != torch.float32 or ce.shape != cew.shape or not ce.is_contiguous():
+        raise EsepError("ce must be a contiguous fp32 [N] tensor")
+    loss = torch.empty((), device=dev, dtype=torch.float32)
+    rc = lib().esep_head_loss(_p(target), _p(cew), _p(ce), ce.numel(), int(V), _p(loss),
+                              _stream(dev))
+    _check(rc, "esep_head_loss")
+    _record(name)
+    return loss
+
+
+def head_dx(prod, inv, cew, dloss, g_scale, dx, name="_head_dx"):
+    """dx[i] = prod[inv[i]] * (cew[i] / g_scale) * dloss for the rows with inv[i] < len(prod), else 0
+    (esep_head_dx). prod fp32 [n_live, H], inv int32 [N], cew fp32 [N], dloss one fp32 on the device,
+    dx [N, H] of a float dtype; all contiguous, H a multiple of 8."""
+    dev = _dev(prod, inv, cew, dloss, dx)
+    N, H = dx.shape
+    if (prod.dtype != torch.float32 or prod.dim() != 2 or prod.shape[1] != H or H % 8
+            or inv.dtype != torch.int32 or inv.numel() != N or cew.dtype != torch.float32
+            or cew.numel() != N or dloss.dtype != torch.float32 or dloss.numel() != 1
+            or not all(t.is_contiguous() for t in (prod, inv, cew, dx))):
+        raise EsepError("head_dx: operands do not match dx [N, H]")
+    rc = lib().esep_head_dx(_p(prod), prod.shape[0], _p(inv), _p(cew), _p(dloss), float(g_scale),
+                            _p(dx), dtype_code(dx.dtype), N, H, _stream(dev))
+    _check(rc, "esep_head_dx")
     _record(name)

@@ -124,7 +124,8 @@ def lora_down_bwd(x, a16, dxa, key, p, need_dx=True, dx_accum=None):
     """Backward of lora_down_fwd: (dx or None, dA fp32 [r, in]). With dx_accum (a dense
     [T, in] buffer, e.g. the base projection's dx) the LoRA part of dx is added into it in
     place and it is returned as dx."""
-    if _grads_fused(x, a16, dxa) and (not need_dx or dx_accum is None or _dense(dx_accum, x)):
+    if (not (torch.is_grad_enabled() and dxa.requires_grad) and _grads_fused(x, a16, dxa)
+            and (not need_dx or dx_accum is None or _dense(dx_accum, x))):
         dx = None
         if need_dx:
             dx = torch.empty_like(x) if dx_accum is None else dx_accum
@@ -160,7 +161,7 @@ def lora_delta(xa, b16, scaling):
 
 def lora_up_bwd(dout, xa, b16, scaling):
     """(dxa [T, r], dB fp32 [out, r]) for the term's gradient dout."""
-    if _up_bwd_fused(dout, xa, b16):
+    if not (torch.is_grad_enabled() and dout.requires_grad) and _up_bwd_fused(dout, xa, b16):
         db = torch.empty(b16.shape, device=dout.device, dtype=torch.float32)
         _hip.lora_grads(dterm=dout, xa=xa, scale=scaling, db=db)
         return _dxa(dout, b16, scaling), db
@@ -211,7 +212,8 @@ class _LoRATerm:
         x2, xa, a16, b16, key = ctx.saved_tensors
         need = ctx.needs_input_grad
         dt2 = _rows_mm(dterm, ctx.dtype)
-        if ctx.fused and _fused(b16.shape[1], dt2):
+        recorded = torch.is_grad_enabled() and dt2.requires_grad  # a pass with create_graph
+        if ctx.fused and not recorded and _fused(b16.shape[1], dt2):
             # dx, dA and dB in one launch after dxa
             dxa = _dxa(dt2, b16, ctx.scaling)
             dx = torch.empty_like(x2) if need[x_index] else None

@@ -50,48 +50,53 @@ def warmup(device=None, vocab=VOCAB):
 
 
 class _RowOrder:
-    """A stable partition of the rows: those with a nonzero loss weight first, in their
-    original order, then the rest. `take` permutes per-row tensors into that order and `undo`
-    brings results back. The identity (no copy) when no gradient pass is wanted."""
+    """The order the rows go through in: with a gradient, those that carry a loss first (a stable
+    partition made on the device), else as they are. The number of live rows sizes the dX product, so
+    the host needs it: its copy is queued at once and read only when the first chunk's logits
+    and statistics are queued behind it, so the GPU does not idle for it."""
 
-    def __init__(self, cew, partition):
-        self.perm = self.inv = None
-        self.n_live = 0
+    def __init__(self, target, cew, vocab, partition):
+        self.perm = self.inv = self._event = None
+        self._live = 0
         if partition:
-            live = cew != 0
-            self.perm = torch.cat((live.nonzero().squeeze(1), (~live).nonzero().squeeze(1)))
-            self.n_live = int(live.sum())  # the one host sync of the call
-            self.inv = torch.empty_like(self.perm)
-            self.inv[self.perm] = torch.arange(self.perm.numel(), device=self.perm.device)
+            self.perm, self.inv, n_live = _hip.head_partition(target, cew, vocab)
+            self._host = torch.empty(1, dtype=torch.int32, pin_memory=True)
+            self._host.copy_(n_live, non_blocking=True)
+            self._event = torch.cuda.Event()
+            self._event.record()
+
+    def n_live(self):
+        if self._event is not None:
+            self._event.synchronize()
+            self._live, self._event = int(self._host[0]), None
+        return self._live
 
     def take(self, t):
         return t.contiguous() if self.perm is None else t.index_select(0, self.perm)
 
-    def undo(self, t):
-        return t if self.inv is None else t.index_select(0, self.inv)
-
 
 class _Chunks:
-    """Statistics (and dX) of rows already in partition order, chunk by chunk."""
+    """Statistics (in the rows' own order) and the dX product (in the partition's order) of rows
+    x16 already in the partition's order, chunk by chunk."""
 
-    def __init__(self, x16, w16, target, cew, n_live, want_dx, chunk_rows):
+    def __init__(self, x16, w16, target, cew, order, want_dx, chunk_rows):
         self.x16, self.w16, self.target, self.cew = x16, w16, target, cew
-        self.n_live, self.want_dx = n_live, want_dx
-        n, h = x16.shape
+        self.order, self.want_dx = order, want_dx
+        n = x16.shape[0]
         dev = x16.device
         self.rows = max(1, min(chunk_rows, n))
         self.z = torch.empty(self.rows, w16.shape[0], device=dev, dtype=w16.dtype)
-        self.lse, self.tlogit, self.ent = (torch.empty(n, device=dev, dtype=torch.float32)
-                                           for _ in range(3))
-        self.amax = torch.empty(n, device=dev, dtype=torch.int32)
-        self.dx = torch.zeros(n, h, device=dev, dtype=torch.float32) if want_dx else None
+        self.lse, self.tlogit, self.ce, self.ent = (
+            torch.empty(n, device=dev, dtype=torch.float32) for _ in range(4))
+        self.amax = torch.empty(n, device=dev, dtype=torch.int64)
+        self.prod = None
         self._full = None  # dX product over a whole chunk (see _dx)
 
     def run(self):
         n = self.x16.shape[0]
         for r0 in range(0, n, self.rows):
             self._chunk(r0, min(self.rows, n - r0))
-        return self.lse, self.tlogit, self.ent, self.amax, self.dx
+        return self.lse, self.tlogit, self.ce, self.ent, self.amax, self.prod
 
     def _chunk(self, r0, nr):
         rows = slice(r0, r0 + nr)
@@ -100,19 +105,27 @@ class _Chunks:
             _hip.gemm(self.x16[rows], self.w16, z)
         else:
             torch.mm(self.x16[rows], self.w16.t(), out=z)
-        _hip.head_row_softmax(z, self.target[rows], self.cew[rows], self.lse[rows],
-                              self.tlogit[rows], self.ent[rows], self.amax[rows],
-                              self.want_dx, G_SCALE)
-        live = max(0, min(self.n_live - r0, nr))
-        if self.want_dx and live:
-            self._dx(r0, nr, live)
+        perm = self.order.perm
+        if perm is None:  # without a partition the chunk's rows are a slice of each array
+            _hip.head_row_softmax(z, self.target[rows], self.cew[rows], self.lse[rows],
+                                  self.tlogit[rows], self.ent[rows], self.amax[rows],
+                                  self.want_dx, G_SCALE, ce=self.ce[rows])
+        else:
+            _hip.head_row_softmax(z, self.target, self.cew, self.lse, self.tlogit, self.ent,
+                                  self.amax, self.want_dx, G_SCALE, perm=perm[rows], ce=self.ce)
+        if not self.want_dx:
+            return
+        if self.prod is None:
+            self.prod = torch.empty(self.order.n_live(), self.x16.shape[1], device=z.device,
+                                    dtype=torch.float32)
+        live = max(0, min(self.order.n_live() - r0, nr))
+        if live:
+            self._dx(r0, live)
 
-    def _dx(self, r0, nr, live):
-        scale = (self.cew[r0:r0 + live] * (1.0 / G_SCALE)).unsqueeze(1)
-        out = self.dx[r0:r0 + live]
+    def _dx(self, r0, live):
+        out = self.prod[r0:r0 + live]
         if _hip.gemm_takes(self.z[:live], self.w16, True):
             _hip.gemm(self.z[:live], self.w16, out, b_kn=True)
-            out.mul_(scale)
         elif live < self.rows <= 2 * live:
             # hipBLASLt runs this product much faster at the chunk's full row count than at a
             # ragged one (MI355X, K = 151936, N = 1536: M = 2925 2.06 ms, M = 4096 1.67 ms), so
@@ -122,27 +135,24 @@ class _Chunks:
                 self._full = torch.empty(self.rows, self.x16.shape[1], device=self.x16.device,
                                          dtype=torch.float32)
             torch.mm(self.z, self.w16, out_dtype=torch.float32, out=self._full)
-            torch.mul(self._full[:live], scale, out=out)
+            out.copy_(self._full[:live])
         else:
             torch.mm(self.z[:live], self.w16, out_dtype=torch.float32, out=out)
-            out.mul_(scale)
 
 
 def _forward(x, w16, target, ce_weight, want_dx, chunk_rows):
-    """(loss, stats tuple in _KEYS order, dX fp32 or None) for the given rows."""
+    """(loss, stats tuple in _KEYS order, (dX product fp32 [n_live, H], inv, cew) or None) for the
+    given rows. The per-row work around the two products is one launch each: the partition, the
+    row kernel (statistics straight into the rows' places), the loss, and in backward the scaled
+    dX; from tensor operations it took about forty (5000 rows: 230 us of kernels, now 40)."""
     vocab = w16.shape[0]
-    has_target = (target >= 0) & (target < vocab)
-    cew = torch.where(has_target, ce_weight.to(torch.float32), 0.0)
-    tgt = torch.where(has_target, target, -1)
-    order = _RowOrder(cew, want_dx)
-    lse, tlogit, ent, amax, dx = _Chunks(order.take(x.to(w16.dtype)), w16, order.take(tgt),
-                                         order.take(cew), order.n_live, want_dx,
-                                         chunk_rows).run()
-    lse, tlogit, ent, amax = (order.undo(t) for t in (lse, tlogit, ent, amax))
-    dx = order.undo(dx) if dx is not None else None
-    tlogit = torch.where(has_target, tlogit, 0.0)
-    ce = torch.where(has_target, lse - tlogit, 0.0)
-    return (cew * ce).sum(), (lse, tlogit, ce, ent, amax.to(torch.int64)), dx
+    target = target.contiguous()
+    cew = ce_weight.detach().to(torch.float32).contiguous()
+    order = _RowOrder(target, cew, vocab, want_dx)
+    lse, tlogit, ce, ent, amax, prod = _Chunks(order.take(x.to(w16.dtype)), w16, target, cew, order,
+                                               want_dx, chunk_rows).run()
+    loss = _hip.head_loss(target, cew, ce, vocab)
+    return loss, (lse, tlogit, ce, ent, amax), (prod, order.inv, cew) if want_dx else None
 
 
 class FusedLinearCE(torch.autograd.Function):
@@ -151,15 +161,26 @@ class FusedLinearCE(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, w16, target, ce_weight, chunk_rows):
-        loss, stats, dx = _forward(x, w16, target, ce_weight, True, chunk_rows)
-        ctx.save_for_backward(dx)
-        ctx.x_dtype = x.dtype
+        loss, stats, saved = _forward(x, w16, target, ce_weight, True, chunk_rows)
+        ctx.save_for_backward(*saved)
+        ctx.x_dtype, ctx.x_shape = x.dtype, x.shape
         ctx.mark_non_differentiable(*stats)
+        ctx.set_materialize_grads(False)  # no zero gradients for the statistics
         return (loss, *stats)
 
     @staticmethod
     def backward(ctx, dloss, *_stat_grads):
-        (dx,) = ctx.saved_tensors
+        if dloss is None:
+            return None, None, None, None, None
+        prod, inv, cew = ctx.saved_tensors
+        n, h = ctx.x_shape
+        if h % 8 == 0 and not (torch.is_grad_enabled() and dloss.requires_grad):
+            dx = torch.empty((n, h), device=prod.device, dtype=ctx.x_dtype)
+            _hip.head_dx(prod, inv, cew, dloss, G_SCALE, dx)
+            return dx, None, None, None, None
+        dx = torch.zeros(n, h, device=prod.device, dtype=torch.float32)
+        rows = torch.argsort(inv)[:prod.shape[0]]
+        dx[rows] = prod * (cew[rows] * (1.0 / G_SCALE)).unsqueeze(1)
         return (dx * dloss).to(ctx.x_dtype), None, None, None, None
 
 

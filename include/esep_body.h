@@ -394,6 +394,33 @@ int esep_head_row_softmax(void* z, int64_t ld, const int64_t* target, const floa
                           float* lse, float* tlogit, float* ent, int32_t* amax, int64_t rows,
                           int64_t V, int write_g, float g_scale, int dt, void* stream);
 
+/*
+ * The rest of the fused head's row work, as single launches (the reference composes it from tensor
+ * operations, solution/head/op.py:63-140).
+ *   esep_head_rows       esep_head_row_softmax that also writes ce[i] = lse - tlogit (0 without a
+ *                        target) and the argmax as int64, and writes g only over rows with a target;
+ *                        perm (int32 [rows] or NULL): the chunk's row i is row perm[i] of target,
+ *                        cew and every output
+ *   esep_head_partition  perm: the rows with a target in [0, V) and cew != 0, then the others, each
+ *                        in order; inv its inverse (int32 [N]); *n_live the first part's length
+ *   esep_head_loss       *loss = sum of cew * ce over the rows with a target in [0, V), fixed order
+ *   esep_head_dx         dx[i, :] = prod[inv[i], :] * (cew[i] / g_scale) * *dloss for inv[i] < n_live,
+ *                        else 0: prod fp32 [n_live, H], dx [N, H] of dx_dt; H a multiple of 8,
+ *                        prod and dx 16-byte aligned
+ * 1 <= N < 2^31. No host synchronization.
+ */
+int esep_head_rows(void* z, int64_t ld, const int64_t* target, const float* cew,
+                   const int32_t* perm, float* lse, float* tlogit, float* ce, float* ent,
+                   int64_t* amax, int64_t rows, int64_t V, int write_g, float g_scale, int dt,
+                   void* stream);
+int esep_head_partition(const int64_t* target, const float* cew, int64_t N, int64_t V,
+                        int32_t* perm, int32_t* inv, int32_t* n_live, void* stream);
+int esep_head_loss(const int64_t* target, const float* cew, const float* ce, int64_t N, int64_t V,
+                   float* loss, void* stream);
+int esep_head_dx(const float* prod, int64_t n_live, const int32_t* inv, const float* cew,
+                 const float* dloss, float g_scale, void* dx, int dx_dt, int64_t N, int64_t H,
+                 void* stream);
+
 #ifdef __cplusplus
 }
 #endif
