@@ -286,23 +286,15 @@ __device__ __forceinline__ int xcd_order(int b, int C) {
 inline int64_t xcd_grid(int64_t C, int64_t groups) { return (groups + 7) / 8 * 8 * C; }
 
 // xcd_order with each XCD running its groups tile-major: tile 0 of every group it holds, then
-// tile 1, and so on, in the order the hardware dispatches its workgroups. The kernels number a
-// group's tiles heaviest first (causal: the query tile with the most keys, the key tile with
-// the most queries), so every XCD starts its longest blocks before its short ones
-// (longest-processing-time first); groups stay whole on one XCD as with xcd_order. It pays when
-// the grid is resident in about one round (short inputs: the longest blocks set the kernel's
-// time); on long inputs the group-by-group order of xcd_order keeps a group's K / V (or Q / dO)
-// reads close together in time in its XCD's L2 and is faster (block_order picks).
+// tile 1, and so on, in the order the hardware dispatches its workgroups; groups stay whole on one
+// XCD as with xcd_order. The kernels number a group's tiles heaviest first (causal: the query tile
+// with the most keys, the key tile with the most queries), so every XCD starts its longest blocks
+// before its short ones. It serves short inputs of more than 64 sequences (level_order the others).
 __device__ __forceinline__ int xcd_order_lpt(int b, int C, int groups) {
   const int xcd = b % 8, slot = b / 8;
   const int per_xcd = (groups + 7) / 8;
   return (xcd + 8 * (slot % per_xcd)) * C + slot / per_xcd;
 }
-// Whether a grid of `blocks` workgroups of a kernel that keeps `per_cu` of them resident on each
-// of MI355X's 256 CUs runs longest-first (xcd_order_lpt): at most two rounds of residency.
-constexpr int64_t kAttnCUs = 256;
-inline int use_lpt(int64_t blocks, int per_cu) { return blocks <= 2 * kAttnCUs * per_cu ? 1 : 0; }
-
 // Sequence s's token range [start, end), clamped into [0, T].
 __device__ __forceinline__ void seq_bounds(const int32_t* cu, int s, int64_t T, int* start,
                                            int* end) {
@@ -332,24 +324,68 @@ __device__ __forceinline__ int seq_of_rank(const int32_t* cu, int n_seq, int64_t
   return hit != 0 ? (int)__builtin_ctzll(hit) : n_seq;
 }
 
-// Block orders of the D = 128 attention kernels, chosen per launch (attn_order):
+// Longest blocks first over the whole launch (n_seq <= 64): what is started last is short, and the
+// CUs end with near-equal work. A block's work
+// is its tile's level (a query tile's keys, a key tile's queries, in 128-row tiles: 1 .. the
+// sequence's tile count), so the (sequence, tile) pairs are walked level by level from the
+// longest sequence's down, each pair's gps blocks (heads) in a row, and every wavefront finds its
+// pair with a ballot per level. Each second run of 256 places is reversed: the hardware deals
+// blocks breadth-first over the 256 CUs, so a CU that got one of the longest blocks of a run gets
+// one of the shortest of the next. The heads of a kv head then lie on different XCDs: an input of up
+// to a few rounds of blocks fits their L2s and the Infinity Cache.
+// Against xcd_order_lpt / the sorted order (bf16, us): dK / dV 123 -> 98, dQ 79 -> 65, forward 65 ->
+// 48 at 12011 tokens in 9 sequences, 14 / 2 heads, D = 64; dK / dV 98 -> 87, dQ 72 -> 68, forward 48 ->
+// 46 at 8 x 1024, 12 / 2 heads, D = 128. Without the reversal dQ of 5933 tokens is 46.0 against
+// 43.5. On long inputs dK / dV, whose few key tiles differ most, still gain (65536 tokens in 29
+// sequences, 28 / 4 heads, D = 128: 2537 -> 2276), while the forward and dQ lose the K / V reuse of
+// the sorted order (forward 1297 -> 1401).
+__device__ __forceinline__ int level_order(int b, int nblk, int C, int groups, int gps,
+                                           const int32_t* cu, int n_seq, int64_t T) {
+  const int lane = (int)(threadIdx.x & 63);
+  const int run = b >> 8;
+  const int p = (run & 1) && (run + 1) << 8 <= nblk ? (run << 8) + 255 - (b & 255) : b;
+  int tiles = 0;
+  if (lane < n_seq) {
+    int s, e;
+    seq_bounds(cu, lane, T, &s, &e);
+    tiles = (e - s + kAttnBM - 1) / kAttnBM;
+  }
+  int pair = p / gps, level = C;
+  uint64_t has = 0;
+  for (; level >= 1; --level) {
+    has = __ballot(tiles >= level);
+    const int n = __popcll(has);
+    if (pair < n) break;
+    pair -= n;
+  }
+  if (level < 1) return groups * C;
+  const int rank = __popcll(has & ((1ull << lane) - 1));
+  const uint64_t hit = __ballot(tiles >= level && rank == pair);
+  const int seq = (int)__builtin_ctzll(hit);
+  return (seq * gps + p % gps) * C + __builtin_amdgcn_readlane(tiles, seq) - level;
+}
+
+// Block orders of the attention kernels, chosen per launch (attn_order):
 //   kOrderGroups  xcd_order: each XCD runs its groups one after another;
-//   kOrderLpt     xcd_order_lpt: each XCD runs its groups tile-major, longest tiles first (grids
-//                 resident in at most two rounds);
+//   kOrderLpt     grids of a few rounds of residency: level_order, or xcd_order_lpt past 64
+//                 sequences;
 //   kOrderSorted  the groups (gps per sequence, sequence-major) sorted by their sequence's
 //                 length, longest first, and dealt to the 8 XCDs in snake order (XCD 0..7, then
 //                 7..0, ...): every XCD gets a near-equal share of the work and runs its groups
 //                 heaviest first, each group whole with its tiles in a row as with xcd_order
-//                 (n_seq <= 64). Dealing groups round-robin in index order instead put a
+//                 (n_seq <= 64), which keeps a group's K / V (or Q / dO) reads close together in its
+//                 XCD's L2. Dealing groups round-robin in index order instead put a
 //                 sequence's 4 kv-head groups of config 5's dK / dV on XCDs 0-3 or 4-7 by the
 //                 sequence's parity, and the two halves' work differed by 38%.
-// The result is the block's index in the group-major order (group * C + tile); a padding block
-// gets an index past the last group and exits.
+// The result is the block's index in the group-major order (group * C + tile, C tiles of 128 rows);
+// a padding block gets an index past the last group and exits.
 constexpr int kOrderGroups = 0, kOrderLpt = 1, kOrderSorted = 2;
 __device__ __forceinline__ int block_order(int b, int C, int groups, int mode, int gps,
                                            const int32_t* cu, int n_seq, int64_t T) {
   if (mode == kOrderGroups) return xcd_order(b, C);
-  if (mode == kOrderLpt) return xcd_order_lpt(b, C, groups);
+  if (mode == kOrderLpt)
+    return n_seq <= 64 ? level_order(b, (int)gridDim.x, C, groups, gps, cu, n_seq, T)
+                       : xcd_order_lpt(b, C, groups);
   const int xcd = b % 8, slot = b / 8;
   const int j = slot / C, tile = slot % C;
   const int p = 8 * j + ((j & 1) ? 7 - xcd : xcd);  // position in the sorted group list
@@ -358,11 +394,14 @@ __device__ __forceinline__ int block_order(int b, int C, int groups, int mode, i
   return (seq * gps + p % gps) * C + tile;
 }
 
-// The order a grid of `blocks` workgroups takes when `per_cu` of them stay resident per CU.
-inline int attn_order(int64_t blocks, int per_cu, int n_seq) {
-  if (use_lpt(blocks, per_cu)) return kOrderLpt;
+// The order a grid of `blocks` workgroups takes when `per_cu` of them stay resident on each of
+// MI355X's 256 CUs: longest first up to `rounds` rounds of residency (two past 64 sequences).
+constexpr int64_t kAttnCUs = 256;
+inline int attn_order(int64_t blocks, int per_cu, int n_seq, int rounds) {
+  if (blocks <= (n_seq <= 64 ? rounds : 2) * kAttnCUs * per_cu) return kOrderLpt;
   return n_seq <= 64 ? kOrderSorted : kOrderGroups;
 }
+constexpr int kRoundsQ = 4, kRoundsKV = 16;  // forward and dQ; dK / dV (level_order's figures)
 
 // A [ROWS x D] tile (token rows r0 .. r0 + ROWS - 1 below rend; the rest reads as 0) moved
 // through registers into a swizzled LDS tile. load() issues every global read of the thread

@@ -108,7 +108,7 @@ constexpr int kDkdvPerCU = 2;
 // dQ with the K / V tiles moved as the forward moves them: swizzled BN-key tiles filled by dwordx4
 // LDS DMA through a ring of two buffers (tile t + 1 in flight while tile t is consumed, one
 // barrier per tile). At D = 64 (the dK / dV kernel's sizes below) 78 us, against 133 staged through
-// registers into padded tiles in the hardware's block order.
+// registers into padded tiles in the hardware's block order (65 in level_order).
 template <typename T, int D, int BN, int NW>
 __global__ __launch_bounds__(64 * NW, kDqPerCU<D>) void k_attn_bwd_dq_dma(const AttnBwdArgs b,
                                                                           int qtiles, int order) {
@@ -118,7 +118,6 @@ __global__ __launch_bounds__(64 * NW, kDqPerCU<D>) void k_attn_bwd_dq_dma(const 
   constexpr int BM = 32 * NW;  // queries per block
   __shared__ __align__(1024) char kv[2][2][BN * RB];  // [buffer][K, V][swizzled tile]
 
-  // XCD-aware order: the query tiles of one (sequence, head) run on one XCD
   const int lin = block_order((int)blockIdx.x, qtiles, a.HQ * a.n_seq, order, a.HQ, a.cu, a.n_seq,
                               a.T);
   const int bx = lin % qtiles, rest = lin / qtiles;
@@ -218,7 +217,7 @@ __global__ __launch_bounds__(64 * NW, kDqPerCU<D>) void k_attn_bwd_dq_dma(const 
 // heads split six ways). At D = 64 (12011 tokens in 9 sequences, 14 / 2 heads, bf16) this kernel
 // takes 119 us, with 64-query tiles 130, at a bound of three blocks per CU 124 (64-query tiles: 10
 // spilled registers, 134), with V's operands in registers 119 .. 131; staged through registers into
-// padded tiles it took 144.
+// padded tiles it took 144. (All in the sorted order; level_order then took it to 98.)
 template <typename T, int D, int NW, int BQ>
 __global__ __launch_bounds__(64 * NW, kDkdvPerCU) void k_attn_bwd_dkdv(const AttnBwdArgs b,
                                                                         int ktiles, int order) {
@@ -236,8 +235,6 @@ __global__ __launch_bounds__(64 * NW, kDkdvPerCU) void k_attn_bwd_dkdv(const Att
   __shared__ __align__(16) float ld_s[NB][2 * BQ];  // lse, then delta
   __shared__ __align__(1024) char vsm[BK * ROWB];  // this block's V rows (B operands of dP)
 
-  // XCD-aware order: the key tiles of one (sequence, kv head, part) run on one XCD (they read
-  // the same Q / dO rows)
   const int split = b.split;                 // query-head groups per kv head
   const int lin = block_order((int)blockIdx.x, ktiles, a.HK * split * a.n_seq, order, a.HK * split,
                               a.cu, a.n_seq, a.T);
@@ -475,7 +472,7 @@ hipError_t bwd_run(const AttnBwdArgs& b, int max_seqlen, hipStream_t s) {
   const int64_t nq = xcd_grid(gq.x, (int64_t)gq.y * gq.z);
   if (nq > 0x7fffffff) return hipErrorInvalidValue;
   hipLaunchKernelGGL((k_attn_bwd_dq_dma<T, D, D == 128 ? 32 : 64, QW>), dim3((unsigned)nq),
-                     dim3(64 * QW), 0, s, b, (int)gq.x, attn_order(nq, kDqPerCU<D>, b.f.n_seq));
+                     dim3(64 * QW), 0, s, b, (int)gq.x, attn_order(nq, kDqPerCU<D>, b.f.n_seq, kRoundsQ));
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   constexpr int NW = 4, BQ = 32;
@@ -483,7 +480,7 @@ hipError_t bwd_run(const AttnBwdArgs& b, int max_seqlen, hipStream_t s) {
   const int64_t nk = xcd_grid(ktiles, (int64_t)b.f.HK * b.split * b.f.n_seq);
   if (nk > 0x7fffffff) return hipErrorInvalidValue;
   hipLaunchKernelGGL((k_attn_bwd_dkdv<T, D, NW, BQ>), dim3((unsigned)nk), dim3(64 * NW), 0, s, b,
-                     (int)ktiles, attn_order(nk, kDkdvPerCU, b.f.n_seq));
+                     (int)ktiles, attn_order(nk, kDkdvPerCU, b.f.n_seq, kRoundsKV));
   e = hipGetLastError();
   if (e != hipSuccess || b.split == 1) return e;
   const int64_t quads = b.f.T * b.f.HK * D / 4;

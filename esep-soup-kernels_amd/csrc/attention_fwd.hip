@@ -108,7 +108,8 @@ constexpr int kFwdPerCU = D == 128 ? 3 : 4;
 // buffers filled by LDS DMA (tile t + 1 in flight while tile t is consumed, one barrier per tile
 // publishing it and freeing the buffer consumed before). At D = 64 (rows of 128 bytes, 64-key tiles:
 // half the barriers) 12011 tokens in 9 sequences, 14 / 2 heads, bf16, take 64 us, against 121 with K
-// and V staged through registers into padded tiles in the hardware's block order.
+// and V staged through registers into padded tiles in the hardware's block order (48 in
+// level_order).
 template <typename T, int D, int BN, int NBUF>
 __global__ __launch_bounds__(kAttnThreads, kFwdPerCU<D>) void k_attn_fwd_swz(const AttnArgs a,
                                                                              int qtiles,
@@ -118,7 +119,6 @@ __global__ __launch_bounds__(kAttnThreads, kFwdPerCU<D>) void k_attn_fwd_swz(con
   using V8 = typename Mfma<T>::v8;
   __shared__ __align__(1024) char kv[NBUF][2][TILE];  // [buffer][K, V][swizzled rows]
 
-  // XCD-aware order (xcd_order): the query tiles of one (sequence, head) run on one XCD.
   const int lin = block_order((int)blockIdx.x, qtiles, a.HQ * a.n_seq, order, a.HQ, a.cu, a.n_seq,
                               a.T);
   const int bx = lin % qtiles, rest = lin / qtiles;
@@ -209,7 +209,7 @@ hipError_t fwd_run(const AttnArgs& a, dim3 grid, hipStream_t s) {
   const int64_t n = xcd_grid(grid.x, (int64_t)grid.y * grid.z);
   if (n > 0x7fffffff) return hipErrorInvalidValue;
   hipLaunchKernelGGL((k_attn_fwd_swz<T, D, BN, 2>), dim3((unsigned)n), dim3(kAttnThreads), 0, s, a,
-                     (int)grid.x, attn_order(n, kFwdPerCU<D>, a.n_seq));
+                     (int)grid.x, attn_order(n, kFwdPerCU<D>, a.n_seq, kRoundsQ));
   return hipGetLastError();
 }
 
