@@ -349,6 +349,7 @@ __device__ __forceinline__ int level_order(int b, int nblk, int C, int groups, i
     int s, e;
     seq_bounds(cu, lane, T, &s, &e);
     tiles = (e - s + kAttnBM - 1) / kAttnBM;
+    if (tiles > C) tiles = C;  // a sequence past max_seqlen: the tiles the grid holds, as elsewhere
   }
   int pair = p / gps, level = C;
   uint64_t has = 0;

@@ -93,9 +93,11 @@ int64_t bwd_partials(int64_t rows, int64_t n) {
 // would leave the GPU short of work. The rule counts 256-token key spans per kv head and takes
 // the smallest divisor s of HQ / HK with spans * s >= 384 (768 of the kernel's 128-key blocks,
 // one and a half rounds of its two blocks per CU); it depends on the shape only. The partials
-// cost traffic (at config 4 a 6-way split writes and re-reads 100 MB), but with the
-// longest-first block order (xcd_order_lpt) the finer split balances better: config 4 backward
-// 0.182 ms with split 3, 0.171 ms with 6.
+// cost traffic (8192 tokens, 12 / 2 heads, D = 128: a 6-way split writes and re-reads 100 MB), but
+// with the blocks started longest first (level_order) the finer split balances better. dK / dV and
+// its reduction in us, bf16: that size 84 + 17 with split 6, 119 + 10 with 3; 14000 tokens, 28 / 4
+// heads: 497 + 85 with split 7, 655 unsplit. Half, a quarter and an eighth of 384 are no better at
+// any size tried.
 int attn_split(int64_t T, int HQ, int HK) {
   const int G = HQ / HK;
   const int64_t blocks = ((T + 255) / 256) * HK;  // 256-token key spans

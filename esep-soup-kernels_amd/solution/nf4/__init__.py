@@ -95,7 +95,8 @@ class NF4Linear(torch.autograd.Function):
     """y = x W^T + bias with W dequantized from NF4 in forward and again in backward (frozen
     weight: nothing of W is kept; dx = dy W) (reference autograd.py:24-48). x and W in x's
     16-bit dtype (fp16 as the reference; an fp32 x computes with an fp16 W and returns fp16);
-    the bias gets its gradient (the sum of dy over the rows, in the bias dtype) when it needs one."""
+    the bias gets its gradient (the sum of dy over the rows, in the bias dtype) when it needs one.
+    Each product runs on esep_gemm where that is expected to be faster, else on the vendor BLAS."""
 
     @staticmethod
     def forward(ctx, x, packed, bias, quant_state):
