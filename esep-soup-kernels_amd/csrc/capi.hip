@@ -873,9 +873,14 @@ int esep_nf4_dequant(const void* packed, const uint8_t* absmax, const float* abs
     return fail(ESEP_EINVAL, "nf4_dequant: every pointer is required");
   if ((reinterpret_cast<uintptr_t>(packed) & 7) || !aligned16(out))
     return fail(ESEP_EALIGN, "nf4_dequant: packed needs 8-byte and out 16-byte alignment");
-  esep::Nf4Args a{packed, absmax, absmax2, code2, offset, nf4, out, n_blocks};
+  if (n_blocks > (int64_t{1} << 36))  // 4 TiB of packed bytes: past every memory, and the grid's limit
+    return fail(ESEP_ESHAPE, "nf4_dequant: too many blocks for one launch");
+  esep::Nf4Multi m{};
+  m.n = 1;
+  m.w[0] = esep::Nf4Args{packed, absmax, absmax2, code2, offset, nf4, out, n_blocks};
+  for (int i = 0; i < esep::kNf4MultiMax; ++i) m.u0[i + 1] = 8 * n_blocks;
   bool sup = false;
-  const hipError_t e = esep::launch_nf4_dequant(a, out_dt, static_cast<hipStream_t>(stream), &sup);
+  const hipError_t e = esep::launch_nf4_dequant(m, out_dt, static_cast<hipStream_t>(stream), &sup);
   if (!sup) return fail(ESEP_EINVAL, "nf4_dequant: unsupported output dtype");
   return e == hipSuccess ? 0 : hip_fail(e, "nf4_dequant launch");
 }
@@ -892,7 +897,7 @@ int esep_nf4_dequant_multi(const esep_nf4_weight* weights, int n_weights, int ou
                 n_weights);
   esep::Nf4Multi m{};
   m.n = n_weights;
-  m.q0[0] = 0;
+  m.u0[0] = 0;
   for (int i = 0; i < n_weights; ++i) {
     const esep_nf4_weight& w = weights[i];
     if (w.n_blocks < 0 || w.n_blocks > (int64_t{1} << 40))
@@ -906,14 +911,14 @@ int esep_nf4_dequant_multi(const esep_nf4_weight* weights, int n_weights, int ou
                   "nf4_dequant_multi: weight %d: packed needs 8-byte and out 16-byte alignment", i);
     m.w[i] = esep::Nf4Args{w.packed, w.absmax, w.absmax2, w.code2, w.offset, w.nf4, w.out,
                            w.n_blocks};
-    m.q0[i + 1] = m.q0[i] + 4 * w.n_blocks;
+    m.u0[i + 1] = m.u0[i] + 8 * w.n_blocks;
   }
-  for (int i = n_weights; i < esep::kNf4MultiMax; ++i) m.q0[i + 1] = m.q0[n_weights];
-  if (m.q0[n_weights] / 256 >= 0x7fffffffLL)
+  for (int i = n_weights; i < esep::kNf4MultiMax; ++i) m.u0[i + 1] = m.u0[n_weights];
+  if (m.u0[n_weights] / 512 >= 0x7fffffffLL)
     return fail(ESEP_ESHAPE, "nf4_dequant_multi: too many blocks for one launch");
   bool sup = false;
   const hipError_t e =
-      esep::launch_nf4_dequant_multi(m, out_dt, static_cast<hipStream_t>(stream), &sup);
+      esep::launch_nf4_dequant(m, out_dt, static_cast<hipStream_t>(stream), &sup);
   if (!sup) return fail(ESEP_EINVAL, "nf4_dequant_multi: unsupported output dtype");
   return e == hipSuccess ? 0 : hip_fail(e, "nf4_dequant_multi launch");
 }

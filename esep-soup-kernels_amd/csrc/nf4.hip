@@ -6,12 +6,16 @@
 // Every step is rounded separately (contraction into fused multiply-adds is switched off in the
 // kernel), which is what makes the result bit-exact with the format's reference decoder.
 //
-// Mapping: a thread decodes 8 packed bytes (16 elements, a quarter of one 64-element scale
-// block) per step (k_nf4_dequant: grid-strided; k_nf4_dequant_multi: one quarter per thread over
-// several weights laid end to end, the reference's multi-weight kernel, dequant.py:129-166):
-// 8-byte loads, two 16-byte (fp16 / bf16) or four 16-byte (fp32) stores. The 16-entry NF4 tables
-// sit in LDS. (8 elements per thread, for wavefront-contiguous 16-byte stores, measured slower:
-// 32 vs 28.6 us for one layer's seven weights.)
+// Bound by bytes: 0.5 read and 2 (fp32: 4) written per element. A thread decodes units of 4 packed
+// bytes (8 elements), consecutive threads consecutive units, so that a wavefront's loads (256
+// bytes) and its 16-byte stores (1 KiB) are each one contiguous run, and takes several units 256
+// apart, all requested before any is decoded. The 16-entry NF4 tables sit in LDS. 16 elements per
+// thread left every store of a wavefront a stride of 32 bytes (fp32: 64) apart. Before -> now in us:
+// 17920 x 1536 in fp32 86 -> 35 by k_nf4_dequant_one; in fp16 20 -> 19.5 by it, two weights of half that size
+// 19.7 -> 18 by k_nf4_dequant_multi (69 MB: 3.8 TB/s). The stores are plain: past the caches
+// (non-temporal) the same kernels take 18.7 and 16.7, but the GEMM that reads the weight next
+// loses more than that (1031 x 17920 x 1536: 64.5 -> 61 with the weight in the caches, its dX
+// 69.5 -> 68; 3001 x 8960 x 1536: 100 -> 92).
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -23,36 +27,34 @@ namespace esep {
 namespace {
 
 constexpr int kNf4Threads = 256;
+// Units from which a block of k_nf4_dequant_multi takes 4 runs of units instead of 2: 1024 blocks,
+// 4 per CU. Below, fewer blocks leave CUs idle (2 runs against 4 in us: 5.6 / 6.9 at 295 k units,
+// 7.4 / 8.3 at 688 k; 14.4 / 12.1 at 1.7 M, 26.8 / 23.2 at 3.4 M).
+constexpr int64_t kNf4Wide = 1 << 20;
 
-// Decode quarter i (8 packed bytes, 16 elements) of one weight with its block scale; tab = the
-// weight's NF4 table (LDS).
+// Decode one unit (4 packed bytes, 8 elements, low byte first) with its block's scale into o;
+// tab = the weight's NF4 table (LDS).
 template <typename TO>
-__device__ __forceinline__ void nf4_decode(uint2 raw, float scale, const float* tab,
-                                           TO* __restrict__ out, int64_t i) {
+__device__ __forceinline__ void nf4_decode(uint32_t raw, float scale, const float* tab,
+                                           TO* __restrict__ o) {
 #pragma clang fp contract(off)
-  float v[16];
+  float v[8];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const uint32_t byte = ((j < 4 ? raw.x : raw.y) >> (8 * (j & 3))) & 0xffu;
+  for (int j = 0; j < 4; ++j) {
+    const uint32_t byte = (raw >> (8 * j)) & 0xffu;
     v[2 * j] = tab[byte >> 4] * scale;
     v[2 * j + 1] = tab[byte & 15u] * scale;
   }
-  TO* o = out + 16 * i;
   if constexpr (sizeof(TO) == 2) {
     typedef TO v8t __attribute__((ext_vector_type(8)));
+    v8t e;
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      v8t e;
-#pragma unroll
-      for (int k = 0; k < 8; ++k) e[k] = Elt<TO>::from_f(v[8 * h + k]);
-      __builtin_nontemporal_store(__builtin_bit_cast(u32x4, e), reinterpret_cast<u32x4*>(o) + h);
-    }
+    for (int k = 0; k < 8; ++k) e[k] = Elt<TO>::from_f(v[k]);
+    *reinterpret_cast<v8t*>(o) = e;
   } else {
 #pragma unroll
-    for (int h = 0; h < 4; ++h) {
-      const f32x4 e = {v[4 * h], v[4 * h + 1], v[4 * h + 2], v[4 * h + 3]};
-      __builtin_nontemporal_store(e, reinterpret_cast<f32x4*>(o) + h);
-    }
+    for (int h = 0; h < 2; ++h)
+      reinterpret_cast<f32x4*>(o)[h] = f32x4{v[4 * h], v[4 * h + 1], v[4 * h + 2], v[4 * h + 3]};
   }
 }
 
@@ -68,101 +70,107 @@ __device__ __forceinline__ float nf4_scale(const uint8_t* __restrict__ absmax,
   return prod + off;
 }
 
-template <typename TO>
-__global__ __launch_bounds__(kNf4Threads) void k_nf4_dequant(const uint8_t* __restrict__ packed,
-                                                             const uint8_t* __restrict__ absmax,
-                                                             const float* __restrict__ absmax2,
-                                                             const float* __restrict__ code2,
-                                                             const float* __restrict__ offset,
-                                                             const float* __restrict__ nf4,
-                                                             TO* __restrict__ out,
-                                                             int64_t n_blocks) {
-  __shared__ float tab[16];
-  if (threadIdx.x < 16) tab[threadIdx.x] = nf4[threadIdx.x];
-  __syncthreads();
-  const float off = *offset;
-  const int64_t quarters = 4 * n_blocks;
-  const int64_t stride = (int64_t)gridDim.x * kNf4Threads;
-  for (int64_t i = (int64_t)blockIdx.x * kNf4Threads + threadIdx.x; i < quarters; i += stride) {
-    const uint2 raw = *reinterpret_cast<const uint2*>(packed + 8 * i);
-    nf4_decode<TO>(raw, nf4_scale(absmax, absmax2, code2, off, i >> 2), tab, out, i);
-  }
-}
-
-// Several weights, one quarter per thread over their concatenation (a weight is whole scale
-// blocks, so the 4 quarters of a scale block share a weight). The packed bytes are requested
-// first; meanwhile 64 threads resolve the block's 64 scales (absmax -> code2 is a dependent pair
-// of loads) into LDS, so only a quarter of the threads wait on that chain. The NF4 tables of
-// every weight sit in LDS.
-template <typename TO>
+// Several weights, their units laid end to end (weight w: units [u0[w], u0[w + 1]), whole scale
+// blocks). A block takes U runs of 256 units. While the packed bytes are on their way, one thread per
+// scale block resolves its scale (absmax -> code2 is a dependent pair of loads) into LDS, so the
+// search for the weight and that chain are paid once per 8 units.
+template <typename TO, int U>
 __global__ __launch_bounds__(kNf4Threads) void k_nf4_dequant_multi(const Nf4Multi m) {
+  constexpr int kScales = kNf4Threads * U / 8;
   __shared__ float tab[kNf4MultiMax][16];
-  __shared__ float scl[kNf4Threads / 4];
+  __shared__ float scl[kScales];
   const int tid = threadIdx.x;
-  const int64_t g0 = (int64_t)blockIdx.x * kNf4Threads;
-  const int64_t total = m.q0[m.n];
-  auto weight_of = [&](int64_t q) {
+  const int64_t g0 = (int64_t)blockIdx.x * (kNf4Threads * U);
+  const int64_t total = m.u0[m.n];
+  auto weight_of = [&](int64_t u) {
     int wi = 0;
 #pragma unroll
     for (int k = 1; k < kNf4MultiMax; ++k)
-      if (k < m.n && q >= m.q0[k]) wi = k;
+      if (k < m.n && u >= m.u0[k]) wi = k;
     return wi;
   };
-  const int64_t g = g0 + tid;
-  const bool live = g < total;
-  const int wi = live ? weight_of(g) : 0;
-  const int64_t i = g - m.q0[wi];  // quarter within the weight
-  uint2 raw = make_uint2(0, 0);
-  if (live) raw = *reinterpret_cast<const uint2*>(static_cast<const uint8_t*>(m.w[wi].packed) + 8 * i);
+  uint32_t raw[U];
+  int wi[U];
+#pragma unroll
+  for (int t = 0; t < U; ++t) {
+    const int64_t g = g0 + t * kNf4Threads + tid;
+    wi[t] = g < total ? weight_of(g) : 0;
+    raw[t] = g < total ? static_cast<const uint32_t*>(m.w[wi[t]].packed)[g - m.u0[wi[t]]] : 0u;
+  }
   if (tid < 16 * m.n) tab[tid >> 4][tid & 15] = m.w[tid >> 4].nf4[tid & 15];
-  if (tid < kNf4Threads / 4) {
-    const int64_t gs = g0 + 4 * tid;  // first quarter of this scale block
+  if (tid < kScales) {
+    const int64_t gs = g0 + 8 * tid;  // first unit of this scale block
     if (gs < total) {
       const int ws = weight_of(gs);
       const Nf4Args& w = m.w[ws];
-      scl[tid] = nf4_scale(w.absmax, w.absmax2, w.code2, *w.offset, (gs - m.q0[ws]) >> 2);
+      scl[tid] = nf4_scale(w.absmax, w.absmax2, w.code2, *w.offset, (gs - m.u0[ws]) >> 3);
     }
   }
   __syncthreads();
-  if (live) nf4_decode<TO>(raw, scl[tid >> 2], tab[wi], static_cast<TO*>(m.w[wi].out), i);
+#pragma unroll
+  for (int t = 0; t < U; ++t) {
+    const int64_t g = g0 + t * kNf4Threads + tid;
+    if (g < total)
+      nf4_decode<TO>(raw[t], scl[(t * kNf4Threads + tid) >> 3], tab[wi[t]],
+                     static_cast<TO*>(m.w[wi[t]].out) + 8 * (g - m.u0[wi[t]]));
+  }
+}
+
+// One weight: every thread reads its own scales (8 threads the same ones), no wait between them and the
+// packed bytes: 5.2 us at 1536 x 1536 against 5.6 through LDS, 10.7 against 14.4 at 1536 x 8960. Two
+// runs of units per block: four take 10.3 there but 5.8 at 1536 x 1536, one 12.5 and 5.2.
+template <typename TO, int U>
+__global__ __launch_bounds__(kNf4Threads) void k_nf4_dequant_one(const Nf4Args w) {
+  __shared__ float tab[16];
+  const int tid = threadIdx.x;
+  const int64_t g0 = (int64_t)blockIdx.x * (kNf4Threads * U) + tid;
+  const int64_t total = 8 * w.n_blocks;
+  uint32_t raw[U];
+  float scale[U];
+  const float off = *w.offset;
+#pragma unroll
+  for (int t = 0; t < U; ++t) {
+    const int64_t g = g0 + t * kNf4Threads;
+    const bool live = g < total;
+    raw[t] = live ? static_cast<const uint32_t*>(w.packed)[g] : 0u;
+    scale[t] = live ? nf4_scale(w.absmax, w.absmax2, w.code2, off, g >> 3) : 0.f;
+  }
+  if (tid < 16) tab[tid] = w.nf4[tid];
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < U; ++t) {
+    const int64_t g = g0 + t * kNf4Threads;
+    if (g < total) nf4_decode<TO>(raw[t], scale[t], tab, static_cast<TO*>(w.out) + 8 * g);
+  }
+}
+
+template <typename TO>
+void launch(const Nf4Multi& m, hipStream_t s) {
+  const int64_t units = m.u0[m.n];
+  auto grid = [&](int u) {
+    const int64_t per = (int64_t)kNf4Threads * u;
+    return dim3((unsigned)((units + per - 1) / per));
+  };
+  const dim3 block(kNf4Threads);
+  if (m.n == 1)
+    hipLaunchKernelGGL((k_nf4_dequant_one<TO, 2>), grid(2), block, 0, s, m.w[0]);
+  else if (units < kNf4Wide)
+    hipLaunchKernelGGL((k_nf4_dequant_multi<TO, 2>), grid(2), block, 0, s, m);
+  else
+    hipLaunchKernelGGL((k_nf4_dequant_multi<TO, 4>), grid(4), block, 0, s, m);
 }
 
 }  // namespace
 
-hipError_t launch_nf4_dequant_multi(const Nf4Multi& m, int out_dt, hipStream_t s, bool* sup) {
+hipError_t launch_nf4_dequant(const Nf4Multi& m, int out_dt, hipStream_t s, bool* sup) {
   *sup = true;
-  const int64_t blocks = (m.q0[m.n] + kNf4Threads - 1) / kNf4Threads;
-  if (blocks == 0) return hipSuccess;
-  const dim3 grid((unsigned)blocks), block(kNf4Threads);
+  if (m.u0[m.n] == 0) return hipSuccess;
   if (out_dt == 0)
-    hipLaunchKernelGGL(k_nf4_dequant_multi<float>, grid, block, 0, s, m);
+    launch<float>(m, s);
   else if (out_dt == 1)
-    hipLaunchKernelGGL(k_nf4_dequant_multi<_Float16>, grid, block, 0, s, m);
+    launch<_Float16>(m, s);
   else if (out_dt == 2)
-    hipLaunchKernelGGL(k_nf4_dequant_multi<__bf16>, grid, block, 0, s, m);
-  else {
-    *sup = false;
-    return hipErrorInvalidValue;
-  }
-  return hipGetLastError();
-}
-
-hipError_t launch_nf4_dequant(const Nf4Args& a, int out_dt, hipStream_t s, bool* sup) {
-  *sup = true;
-  int64_t blocks = (4 * a.n_blocks + kNf4Threads - 1) / kNf4Threads;
-  if (blocks > 256 * 16) blocks = 256 * 16;
-  if (blocks < 1) blocks = 1;
-  const dim3 grid((unsigned)blocks), block(kNf4Threads);
-  const uint8_t* pk = static_cast<const uint8_t*>(a.packed);
-  if (out_dt == 0)
-    hipLaunchKernelGGL(k_nf4_dequant<float>, grid, block, 0, s, pk, a.absmax, a.absmax2, a.code2,
-                       a.offset, a.nf4, static_cast<float*>(a.out), a.n_blocks);
-  else if (out_dt == 1)
-    hipLaunchKernelGGL(k_nf4_dequant<_Float16>, grid, block, 0, s, pk, a.absmax, a.absmax2, a.code2,
-                       a.offset, a.nf4, static_cast<_Float16*>(a.out), a.n_blocks);
-  else if (out_dt == 2)
-    hipLaunchKernelGGL(k_nf4_dequant<__bf16>, grid, block, 0, s, pk, a.absmax, a.absmax2, a.code2,
-                       a.offset, a.nf4, static_cast<__bf16*>(a.out), a.n_blocks);
+    launch<__bf16>(m, s);
   else {
     *sup = false;
     return hipErrorInvalidValue;

@@ -1,0 +1,63 @@
+"""NF4 dequantization at the edges of its launches (a block covers 64 scale blocks of one weight, 64
+or, from 131072 scale blocks in all, 128 of several): the same bits as the oracle, and as one
+launch per weight, and nothing written past the output."""
+
+import numpy as np
+import pytest
+import torch
+
+from _util import DEV
+from oracle import nf4_ref as ref
+
+pytestmark = pytest.mark.gpu
+
+
+def _weight(nb, seed, dtype):
+    """Raw state of nb scale blocks and its device form with a guarded output buffer."""
+    rng = np.random.default_rng(seed)
+    raw = (rng.integers(0, 256, nb * 32, dtype=np.uint8), rng.integers(0, 256, nb, dtype=np.uint8),
+           (rng.random((nb + 255) // 256) * 0.1 + 0.01).astype(np.float32),
+           np.sort(rng.standard_normal(256)).astype(np.float32), np.float32(rng.random() * 0.05))
+    table = ref.NF4 if seed % 2 else (ref.NF4[::-1] * 0.5).astype(np.float32)
+    buf = torch.full((nb * 64 + 64,), 7.0, device=DEV, dtype=dtype)
+    dev = [torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
+           for a in (*raw[:4], np.array([raw[4]], dtype=np.float32), table)]
+    return raw, table, dev, buf
+
+
+def _want(raw, table, dtype):
+    """The oracle's formula with the weight's own table: fp32 scale in two roundings, one product,
+    one rounding to the output type."""
+    packed, absmax, absmax2, code2, offset = raw
+    prod = (code2[absmax] * absmax2[np.arange(absmax.size) // 256]).astype(np.float32)
+    scale = (prod + offset).astype(np.float32)
+    nib = np.stack([packed >> 4, packed & 15], 1).reshape(-1)
+    return torch.from_numpy((table[nib] * np.repeat(scale, 64)).astype(np.float32)).to(dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32],
+                         ids=["fp16", "bf16", "fp32"])
+@pytest.mark.parametrize("nb", [1, 63, 64, 65, 257])
+def test_one_weight(nb, dtype):
+    from solution.body import _hip
+
+    raw, table, dev, buf = _weight(nb, 1, dtype)
+    _hip.nf4_dequant(*dev, buf[:nb * 64].view(nb, 64))
+    assert torch.equal(buf[:nb * 64].cpu(), _want(raw, table, dtype))
+    assert np.array_equal(_want(raw, table, torch.float32).numpy(),
+                          ref.dequantize_nf4(*raw, out_dtype=np.float32).reshape(-1))
+    assert (buf[nb * 64:] == 7).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32], ids=["fp16", "fp32"])
+@pytest.mark.parametrize("sizes", [(1, 1), (63, 1, 64), (65, 127, 2, 1, 1, 30, 128, 5),
+                                   (70000, 61071), (70001, 61071), (131072, 3, 128)])
+def test_several_weights(sizes, dtype):
+    from solution.body import _hip
+
+    ws = [_weight(nb, 2 + i, dtype) for i, nb in enumerate(sizes)]
+    _hip.nf4_dequant_multi([(*dev, buf[:nb * 64].view(nb, 64))
+                            for nb, (_, _, dev, buf) in zip(sizes, ws)])
+    for nb, (raw, table, dev, buf) in zip(sizes, ws):
+        assert torch.equal(buf[:nb * 64].cpu(), _want(raw, table, dtype))
+        assert (buf[nb * 64:] == 7).all()
