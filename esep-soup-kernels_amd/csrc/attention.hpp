@@ -132,9 +132,14 @@ typedef short s16x8 __attribute__((ext_vector_type(8)));
 // tile). The LDS address goes in M0 through the "{m0}" operand constraint: the compiler itself
 // loads M0 before the instruction and knows what M0 holds afterwards (the asm only reads it),
 // so no M0 value of the compiler's own is ever overwritten behind its back.
+//
+// The compiler's hazard pass does not look into asm, so the wait states are part of it (the s_nop
+// before the load in each form): one between a scalar write of M0 and an LDS DMA, which the
+// compiler otherwise puts back to back, and five between a VALU write of an SGPR (v_readfirstlane
+// of a base it holds in VGPRs) and the VMEM instruction that reads it as its base.
 __device__ __forceinline__ void lds_dma_dword(const void* g, const void* lds) {
   const uint32_t m = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds);
-  asm volatile("global_load_lds_dword %0, off" ::"v"(g), "{m0}"(m) : "memory");
+  asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(g), "{m0}"(m) : "memory");
 }
 
 // s_waitcnt vmcnt(0) (expcnt, lgkmcnt left at their maxima): through the builtin, so that the
@@ -156,11 +161,11 @@ constexpr int kWaitVm0 = 0x0F70;
 // ---------------------------------------------------------------------------------------
 __device__ __forceinline__ void lds_dma_x4_s(const void* base, uint32_t voff, const void* lds) {
   const uint32_t m = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds);
-  asm volatile("global_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(base), "{m0}"(m) : "memory");
+  asm volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(base), "{m0}"(m) : "memory");
 }
 __device__ __forceinline__ void lds_dma_x4(const void* g, const void* lds) {
   const uint32_t m = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds);
-  asm volatile("global_load_lds_dwordx4 %0, off" ::"v"(g), "{m0}"(m) : "memory");
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "{m0}"(m) : "memory");
 }
 
 template <int RB>

@@ -36,17 +36,12 @@ constexpr int kBK = 64;  // contraction depth of one LDS tile: 128-byte rows
 // s_waitcnt vmcnt(0) lgkmcnt(0)
 constexpr int kWaitVmLgkm0 = 0x0070;
 
-// One LDS DMA instruction as lds_dma_x4_s, from any wavefront-uniform base. Where the compiler
-// holds the base in VGPRs it copies it to SGPRs with v_readfirstlane right before the asm, whose
-// VMEM use of an SGPR needs five wait states after a VALU write of it; the compiler's hazard
-// pass does not look into the asm, so the s_nop is part of it.
+// lds_dma_x4_s from any wavefront-uniform base, also one that the compiler holds in VGPRs.
 __device__ __forceinline__ void lds_dma(const char* base, uint32_t voff, const void* lds) {
   const uint64_t v = reinterpret_cast<uint64_t>(base);
   const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
   const uint32_t up = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-  const uint64_t sbase = ((uint64_t)up << 32) | lo;
-  const uint32_t m = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds);
-  asm volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "{m0}"(m) : "memory");
+  lds_dma_x4_s(reinterpret_cast<const void*>(((uint64_t)up << 32) | lo), voff, lds);
 }
 
 template <int WM, int WN, int TM, int TN>
