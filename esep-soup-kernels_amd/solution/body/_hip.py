@@ -19,6 +19,7 @@ import threading
 from pathlib import Path
 
 import torch
+from torch.autograd import forward_ad
 
 LIB_PATH = Path(__file__).resolve().with_name("libesep_body.so")
 ABI_VERSION = 1
@@ -180,6 +181,19 @@ except AttributeError:  # a torch without it (or without a GPU build)
 
 def _stream(dev):
     return _current_stream(dev) if _raw_stream is None else _raw_stream(dev.index)
+
+
+def recorded(*tensors):
+    """Torch has to see the operations on these tensors as its own (a kernel would fill a buffer behind
+    its back): one requires grad in grad mode, carries a forward-mode tangent, or is a functorch
+    wrapper (vmap, batched gradients, torch.func), which has no memory of its own."""
+    tensors = [t for t in tensors if t is not None]
+    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
+        return True
+    if any(map(torch._C._functorch.is_functorch_wrapped_tensor, tensors)):
+        return True
+    return forward_ad._current_level >= 0 and any(
+        forward_ad.unpack_dual(t).tangent is not None for t in tensors)
 
 
 def _rows_ld(t, n):

@@ -91,7 +91,8 @@ def _mm_fp32(a, b):
 
 def lora_down_fwd(x, a16, key, p):
     """xa = drop(x) @ A^T for a dense x [T, in] (no dropout when p == 0)."""
-    if _fused(a16.shape[0], x, a16) and x.is_contiguous() and a16.is_contiguous():
+    if (not _hip.recorded(x, a16) and _fused(a16.shape[0], x, a16) and x.is_contiguous()
+            and a16.is_contiguous()):
         xa = torch.empty((x.shape[0], a16.shape[0]), device=x.device, dtype=x.dtype)
         _hip.lora_down(x, a16, xa, key=key if p > 0.0 else None, p=p)
         return xa
@@ -150,8 +151,8 @@ def lora_down_bwd(x, a16, dxa, key, p, need_dx=True, dx_accum=None):
 
 def lora_delta(xa, b16, scaling):
     """The term scaling * xa @ B^T on its own."""
-    if _fused(b16.shape[1], xa, b16) and xa.is_contiguous() and b16.is_contiguous() \
-            and b16.shape[0] % 8 == 0:
+    if (not _hip.recorded(xa, b16) and _fused(b16.shape[1], xa, b16) and xa.is_contiguous()
+            and b16.is_contiguous() and b16.shape[0] % 8 == 0):
         term = torch.empty((xa.shape[0], b16.shape[0]), device=xa.device, dtype=xa.dtype)
         _hip.lora_up(xa, b16, term, scaling)
         return term

@@ -1,0 +1,117 @@
+"""Calls that torch has to see as its own operations (a graph through the public product functions, a
+recorded backward pass, forward-mode tangents, vmap and batched gradients) keep them: the fused
+kernels fill buffers behind torch's back. Results against the same products written in torch."""
+
+import pytest
+import torch
+import torch.autograd.forward_ad as fwd
+
+from _util import DEV
+
+pytestmark = pytest.mark.gpu
+
+T, K, N, R, S = 40, 64, 128, 16, 2.0
+# products of fp16 operands of up to 128 terms, results rounded once or twice (2^-11 each)
+TOL = dict(rtol=4e-3, atol=4e-3)
+
+
+def _rnd(*shape, seed=0):
+    g = torch.Generator(device=DEV).manual_seed(seed + sum(shape))
+    return (torch.randn(*shape, generator=g, device=DEV) * 0.5).half()
+
+
+def _same(got, want):
+    got, want = (t if isinstance(t, tuple) else (t,) for t in (got, want))
+    assert len(got) == len(want)
+    for a, b in zip(got, want):
+        assert (a is None) == (b is None)
+        if a is not None:
+            torch.testing.assert_close(a.float(), b.float(), **TOL)
+
+
+def _ref_delta(xa, b):
+    return S * (xa @ b.t())
+
+
+def _ref_down(x, a):
+    return x @ a.t()
+
+
+def _ref_up_bwd(dout, xa, b):
+    return S * (dout @ b), S * (dout.t() @ xa).float()
+
+
+def _ref_down_bwd(x, a, dxa):
+    return dxa @ a, (dxa.t() @ x).float()
+
+
+def _functions():
+    """(function, torch's form, operands); p = 0 throughout."""
+    from solution.body import lora as L
+
+    x, a, xa, b, d, dxa = _rnd(T, K), _rnd(R, K), _rnd(T, R), _rnd(N, R), _rnd(T, N), _rnd(T, R, seed=1)
+    return {
+        "delta": (lambda xa, b: L.lora_delta(xa, b, S), _ref_delta, (xa, b)),
+        "down_fwd": (lambda x, a: L.lora_down_fwd(x, a, None, 0.0), _ref_down, (x, a)),
+        "up_bwd": (lambda d, xa, b: L.lora_up_bwd(d, xa, b, S), _ref_up_bwd, (d, xa, b)),
+        "down_bwd": (lambda x, a, dxa: L.lora_down_bwd(x, a, dxa, None, 0.0), _ref_down_bwd, (x, a, dxa)),
+    }
+
+
+@pytest.fixture(autouse=True)
+def _fp32_products(monkeypatch):
+    """lora._mm_fp32 gives up torch's out_dtype for good where torch refuses it (forward mode)."""
+    from solution.body import lora as L
+
+    monkeypatch.setattr(L, "_OUT_DTYPE_OK", L._OUT_DTYPE_OK)
+
+
+@pytest.mark.parametrize("name", ["delta", "down_fwd"])
+@pytest.mark.parametrize("which", [0, 1])
+def test_graph_of_the_forward_products(name, which):
+    f, ref, ops = _functions()[name]
+    grads = []
+    for fn in (f, ref):
+        ins = [t.clone().requires_grad_(i == which) for i, t in enumerate(ops)]
+        out = fn(*ins)
+        grads.append(torch.autograd.grad(out, ins[which], torch.ones_like(out))[0])
+    _same(*grads)
+    with torch.no_grad():  # the kernels' own result
+        _same(f(*ops), ref(*ops))
+
+
+def test_graph_of_the_dropped_product():
+    """With dropout on, the product's other operand still gets its gradient."""
+    from solution.body import lora as L
+
+    x, key = _rnd(T, K), torch.tensor([77], device=DEV)
+    a = _rnd(R, K).requires_grad_()
+    out = L.lora_down_fwd(x, a, key, 0.25)
+    (da,) = torch.autograd.grad(out, a, torch.ones_like(out))
+    want = torch.ones_like(out).t() @ L.lora_dropout(x, key, 0.25)
+    _same(da, want)
+
+
+@pytest.mark.parametrize("name", ["delta", "down_fwd"])
+def test_forward_mode(name):
+    f, ref, ops = _functions()[name]
+    which = len(ops) - 1
+    tangents = []
+    for fn in (f, ref):
+        with fwd.dual_level():
+            ins = list(ops)
+            ins[which] = fwd.make_dual(ops[which], _rnd(*ops[which].shape, seed=5))
+            out = fn(*ins)
+            tangents.append(tuple(fwd.unpack_dual(o).tangent
+                                  for o in (out if isinstance(out, tuple) else (out,))))
+    _same(*tangents)
+
+
+@pytest.mark.parametrize("name", ["delta", "down_fwd"])
+@pytest.mark.filterwarnings("ignore:There is a performance drop")
+def test_vmap(name):
+    f, ref, ops = _functions()[name]
+    dims = [None] * len(ops)
+    dims[-1] = 0
+    ins = (*ops[:-1], torch.stack([ops[-1], -ops[-1], 2 * ops[-1]]))
+    _same(torch.vmap(f, tuple(dims))(*ins), torch.vmap(ref, tuple(dims))(*ins))
