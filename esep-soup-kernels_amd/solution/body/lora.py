@@ -125,7 +125,7 @@ def lora_down_bwd(x, a16, dxa, key, p, need_dx=True, dx_accum=None):
     """Backward of lora_down_fwd: (dx or None, dA fp32 [r, in]). With dx_accum (a dense
     [T, in] buffer, e.g. the base projection's dx) the LoRA part of dx is added into it in
     place and it is returned as dx."""
-    if (not (torch.is_grad_enabled() and dxa.requires_grad) and _grads_fused(x, a16, dxa)
+    if (not _hip.recorded(x, a16, dxa, dx_accum) and _grads_fused(x, a16, dxa)
             and (not need_dx or dx_accum is None or _dense(dx_accum, x))):
         dx = None
         if need_dx:
@@ -162,7 +162,7 @@ def lora_delta(xa, b16, scaling):
 
 def lora_up_bwd(dout, xa, b16, scaling):
     """(dxa [T, r], dB fp32 [out, r]) for the term's gradient dout."""
-    if not (torch.is_grad_enabled() and dout.requires_grad) and _up_bwd_fused(dout, xa, b16):
+    if not _hip.recorded(dout, xa, b16) and _up_bwd_fused(dout, xa, b16):
         db = torch.empty(b16.shape, device=dout.device, dtype=torch.float32)
         _hip.lora_grads(dterm=dout, xa=xa, scale=scaling, db=db)
         return _dxa(dout, b16, scaling), db

@@ -92,7 +92,28 @@ def test_graph_of_the_dropped_product():
     _same(da, want)
 
 
-@pytest.mark.parametrize("name", ["delta", "down_fwd"])
+@pytest.mark.parametrize("name,which,out", [("up_bwd", 2, 0), ("down_bwd", 1, 0)])
+def test_graph_of_the_backward_products(name, which, out):
+    """Their 16-bit results are differentiable in every operand, not in the incoming gradient alone."""
+    f, ref, ops = _functions()[name]
+    grads = []
+    for fn in (f, ref):
+        ins = [t.clone().requires_grad_(i == which) for i, t in enumerate(ops)]
+        o = fn(*ins)[out]
+        grads.append(torch.autograd.grad(o, ins[which], torch.ones_like(o))[0])
+    _same(*grads)
+
+
+@pytest.mark.parametrize("name,which", [("up_bwd", 1), ("down_bwd", 0)])
+def test_fp32_results_are_on_the_graph(name, which):
+    """The fp32 results stand on the graph of an operand that requires grad (torch then says itself
+    that it has no derivative for them), instead of passing for constants."""
+    f, _, ops = _functions()[name]
+    ins = [t.clone().requires_grad_(i == which) for i, t in enumerate(ops)]
+    assert f(*ins)[1].requires_grad
+
+
+@pytest.mark.parametrize("name", ["delta", "down_fwd", "up_bwd", "down_bwd"])
 def test_forward_mode(name):
     f, ref, ops = _functions()[name]
     which = len(ops) - 1
@@ -107,7 +128,7 @@ def test_forward_mode(name):
     _same(*tangents)
 
 
-@pytest.mark.parametrize("name", ["delta", "down_fwd"])
+@pytest.mark.parametrize("name", ["delta", "down_fwd", "up_bwd", "down_bwd"])
 @pytest.mark.filterwarnings("ignore:There is a performance drop")
 def test_vmap(name):
     f, ref, ops = _functions()[name]
