@@ -213,7 +213,8 @@ class _LoRATerm:
         x2, xa, a16, b16, key = ctx.saved_tensors
         need = ctx.needs_input_grad
         dt2 = _rows_mm(dterm, ctx.dtype)
-        recorded = torch.is_grad_enabled() and dt2.requires_grad  # a pass with create_graph
+        # torch's products for a pass with create_graph, under vmap (is_grads_batched), with a tangent
+        recorded = _hip.recorded(dt2, x2, xa, a16, b16)
         if ctx.fused and not recorded and _fused(b16.shape[1], dt2):
             # dx, dA and dB in one launch after dxa
             dxa = _dxa(dt2, b16, ctx.scaling)

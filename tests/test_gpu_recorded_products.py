@@ -136,3 +136,44 @@ def test_vmap(name):
     dims[-1] = 0
     ins = (*ops[:-1], torch.stack([ops[-1], -ops[-1], 2 * ops[-1]]))
     _same(torch.vmap(f, tuple(dims))(*ins), torch.vmap(ref, tuple(dims))(*ins))
+
+
+def _lora_function(name, x, a, b):
+    from solution.body import lora as L
+
+    if name == "delta":
+        return L.LoRADeltaFunction.apply(x, a, b, 0.0, S)
+    return L.LoRAFunction.apply(x, torch.zeros(T, N, device=DEV).half(), a, b, 0.0, S)
+
+
+@pytest.mark.parametrize("name", ["delta", "added"])
+@pytest.mark.filterwarnings("ignore:There is a performance drop")
+def test_batched_gradients_of_the_term(name):
+    """torch.autograd.grad(is_grads_batched=True) runs the backward pass under vmap."""
+    ops = [t.clone().requires_grad_() for t in (_rnd(T, K), _rnd(R, K).float(), _rnd(N, R).float())]
+    out = _lora_function(name, *ops)
+    d = torch.stack([_rnd(T, N), _rnd(T, N, seed=3)])
+    got = torch.autograd.grad(out, ops, d, is_grads_batched=True, retain_graph=True)
+    for i in range(2):
+        want = torch.autograd.grad(out, ops, d[i], retain_graph=True)
+        _same(tuple(g[i] for g in got), want)
+
+
+@pytest.mark.parametrize("name", ["delta", "added"])
+def test_tangent_of_the_incoming_gradient(name):
+    ops = [t.clone().requires_grad_() for t in (_rnd(T, K), _rnd(R, K).float(), _rnd(N, R).float())]
+    out = _lora_function(name, *ops)
+    d, t = _rnd(T, N), _rnd(T, N, seed=3)
+    with fwd.dual_level():
+        got = torch.autograd.grad(out, ops, fwd.make_dual(d, t), retain_graph=True)
+        got = tuple(fwd.unpack_dual(g).tangent for g in got)
+    _same(got, torch.autograd.grad(out, ops, t))  # the backward pass is linear in it
+
+
+def test_recorded_pass_over_a_constant_gradient():
+    """create_graph with an incoming gradient that is a constant: what the backward pass computes from
+    tensors on the graph is on it."""
+    ops = [t.clone().requires_grad_() for t in (_rnd(T, K), _rnd(R, K).float(), _rnd(N, R).float())]
+    out = _lora_function("delta", *ops)
+    _, da, _ = torch.autograd.grad(out, ops, torch.ones_like(out), create_graph=True)
+    assert da.requires_grad  # dA is a product with x
