@@ -632,10 +632,10 @@ def gemm(a, b, out, b_kn=False, bias=None, name="_gemm"):
     _record(name)
 
 
-def _plain(x):
-    """No cast and no graph is expected of a product with x (autocast to another dtype, a backward
-    pass that is itself recorded)."""
-    if torch.is_grad_enabled() and x.requires_grad:
+def _plain(x, w, bias=None):
+    """No cast and no graph is expected of a product of these (autocast to another dtype; a backward
+    pass that is itself recorded, batched or carries tangents)."""
+    if recorded(x, w, bias):
         return False
     return not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == x.dtype
 
@@ -644,7 +644,7 @@ def linear(x, w, bias=None):
     """F.linear(x, w, bias) for autograd Functions: esep_gemm where it takes the operands and pays,
     else the vendor BLAS (which also serves a recorded backward pass)."""
     x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
-    if (_plain(x) and gemm_takes(x2, w, False)
+    if (_plain(x, w, bias) and gemm_takes(x2, w, False)
             and (bias is None or (bias.dtype == x.dtype and bias.dim() == 1 and bias.is_contiguous()
                                   and bias.data_ptr() % 16 == 0))):
         out = torch.empty((x2.shape[0], w.shape[0]), device=x.device, dtype=x.dtype)
@@ -656,7 +656,7 @@ def linear(x, w, bias=None):
 def matmul(x, w):
     """x @ w for a 2-D w [K, N], as linear."""
     x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
-    if _plain(x) and gemm_takes(x2, w, True):
+    if _plain(x, w) and gemm_takes(x2, w, True):
         out = torch.empty((x2.shape[0], w.shape[1]), device=x.device, dtype=x.dtype)
         gemm(x2, w, out, b_kn=True)
         return out.view(*x.shape[:-1], w.shape[1])

@@ -177,3 +177,55 @@ def test_recorded_pass_over_a_constant_gradient():
     out = _lora_function("delta", *ops)
     _, da, _ = torch.autograd.grad(out, ops, torch.ones_like(out), create_graph=True)
     assert da.requires_grad  # dA is a product with x
+
+
+class _State:
+    """A quant state of random NF4 bytes [n, k]."""
+
+    def __init__(self, n, k):
+        g = torch.Generator(device=DEV).manual_seed(n + k)
+        nb = n * k // 64
+        self.packed = torch.randint(0, 256, (nb * 32,), generator=g, device=DEV, dtype=torch.uint8)
+        self.quant_type, self.blocksize, self.nested, self.shape = "nf4", 64, True, (n, k)
+        self.absmax = torch.randint(0, 256, (nb,), generator=g, device=DEV, dtype=torch.uint8)
+        self.code = torch.linspace(-1, 1, 16, device=DEV)
+        self.offset = torch.tensor(0.02, device=DEV)
+        self.state2 = type("S", (), dict(absmax=torch.full(((nb + 255) // 256,), 0.02, device=DEV),
+                                         code=torch.linspace(-1, 1, 256, device=DEV), blocksize=256))()
+
+
+@pytest.mark.parametrize("multi", [False, True])
+def test_nf4_backward_under_vmap_and_forward_mode(multi):
+    """The NF4 linears' dX where esep_gemm would take it (n = 1536 outputs contracted)."""
+    from solution import nf4
+    from solution.body import _hip
+
+    st = _State(1536, 64)
+    x = _rnd(T, 64).requires_grad_()
+    y = (nf4.NF4MultiLinear.apply(x, None, ([st.packed], [st], None)) if multi
+         else nf4.nf4_linear(x, st.packed, None, st))
+    d = torch.stack([_rnd(T, 1536), _rnd(T, 1536, seed=3)])
+    with _hip.count_launches() as names:
+        want = [torch.autograd.grad(y, x, di, retain_graph=True)[0] for di in d]
+    assert "_gemm" in names
+    (got,) = torch.autograd.grad(y, x, d, is_grads_batched=True, retain_graph=True)
+    for a, b in zip(got, want):
+        torch.testing.assert_close(a, b, rtol=4e-3, atol=2e-2)  # sums of 1536 terms, two kernels
+    with fwd.dual_level():
+        (dx,) = torch.autograd.grad(y, x, fwd.make_dual(d[0], d[1]), retain_graph=True)
+        torch.testing.assert_close(fwd.unpack_dual(dx).tangent, want[1], rtol=4e-3, atol=2e-2)
+
+
+def test_linear_and_matmul_see_every_operand():
+    """A weight or a bias that requires grad in grad mode goes to torch's product too."""
+    from solution.body import _hip
+
+    x, w, wk, b = _rnd(T, 1536), _rnd(N, 1536), _rnd(1536, N), _rnd(N)
+    for t in (w, b):
+        t.requires_grad_()
+        assert _hip.linear(x, w, b).requires_grad
+        t.requires_grad_(False)
+    assert _hip.matmul(x, wk.requires_grad_()).requires_grad
+    with torch.no_grad(), _hip.count_launches() as names:
+        _hip.linear(x, w, b), _hip.matmul(x, wk)
+    assert names == ["_gemm", "_gemm"]
