@@ -229,3 +229,20 @@ def test_linear_and_matmul_see_every_operand():
     with torch.no_grad(), _hip.count_launches() as names:
         _hip.linear(x, w, b), _hip.matmul(x, wk)
     assert names == ["_gemm", "_gemm"]
+
+
+def test_head_loss_gradient_batched_and_tangent():
+    from solution.head import fused_linear_ce
+
+    g = torch.Generator(device=DEV).manual_seed(1)
+    x = torch.randn(30, 64, generator=g, device=DEV, requires_grad=True)
+    w = (torch.randn(100, 64, generator=g, device=DEV) * 0.1).half()
+    target = torch.randint(-5, 100, (30,), generator=g, device=DEV)
+    loss, _ = fused_linear_ce(x, w, target, torch.rand(30, generator=g, device=DEV))
+    (plain,) = torch.autograd.grad(loss, x, retain_graph=True)
+    scale = torch.tensor([1.0, -2.5], device=DEV)
+    (got,) = torch.autograd.grad(loss, x, scale, is_grads_batched=True, retain_graph=True)
+    torch.testing.assert_close(got, torch.stack([plain, -2.5 * plain]), rtol=1e-6, atol=0)
+    with fwd.dual_level():
+        (dx,) = torch.autograd.grad(loss, x, fwd.make_dual(scale[0], scale[1]))
+        torch.testing.assert_close(fwd.unpack_dual(dx).tangent, -2.5 * plain, rtol=1e-6, atol=0)
