@@ -63,7 +63,7 @@ class _RowOrder:
             self._host = torch.empty(1, dtype=torch.int32, pin_memory=True)
             self._host.copy_(n_live, non_blocking=True)
             self._event = torch.cuda.Event()
-            self._event.record()
+            self._event.record(torch.cuda.current_stream(target.device))
 
     def n_live(self):
         if self._event is not None:
