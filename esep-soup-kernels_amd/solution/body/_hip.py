@@ -190,7 +190,9 @@ def recorded(*tensors):
     tensors = [t for t in tensors if t is not None]
     if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
         return True
-    if any(map(torch._C._functorch.is_functorch_wrapped_tensor, tensors)):
+    functorch = torch._C._functorch
+    if any(functorch.is_functorch_wrapped_tensor(t) or functorch.is_legacy_batchedtensor(t)
+           for t in tensors):
         return True
     return forward_ad._current_level >= 0 and any(
         forward_ad.unpack_dual(t).tangent is not None for t in tensors)
