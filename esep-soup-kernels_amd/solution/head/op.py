@@ -16,10 +16,10 @@ Never materializes all N x V logits. Rows go through in chunks of `chunk_rows`: 
 logits z = x_c W^T (esep_gemm or hipBLASLt, the weight's dtype, fp32 accumulation) land in one reused
 [chunk, V] buffer; the row kernel reads them once for the statistics and, when a gradient is
 wanted, rewrites the rows that carry a loss with g = (softmax - onehot) * G_SCALE; then
-dX_c = g W (esep_gemm or hipBLASLt, fp32 out) for those rows, scaled by ce_weight / G_SCALE. The rows that
+dX_c = g W (esep_gemm or hipBLASLt, fp32 out) for those rows. The rows that
 carry a loss are moved to the front first (a stable partition), so the g pass and the dX
-product work on a prefix of each chunk. dX is finished in the forward; the backward only
-scales it by the incoming gradient.
+product work on a prefix of each chunk. The dX product is made in the forward (no logits are kept);
+the backward puts its rows back in place, scaled by ce_weight / G_SCALE and the incoming gradient.
 """
 
 import torch
@@ -147,7 +147,8 @@ def _forward(x, w16, target, ce_weight, want_dx, chunk_rows):
     dX; from tensor operations it took about forty (5000 rows: 230 us of kernels, now 40)."""
     vocab = w16.shape[0]
     target = target.contiguous()
-    cew = ce_weight.detach().to(torch.float32).contiguous()
+    # with a gradient a copy of its own: backward reads it, and the caller may refill ce_weight
+    cew = ce_weight.detach().to(torch.float32, copy=want_dx).contiguous()
     order = _RowOrder(target, cew, vocab, want_dx)
     lse, tlogit, ce, ent, amax, prod = _Chunks(order.take(x.to(w16.dtype)), w16, target, cew, order,
                                                want_dx, chunk_rows).run()
@@ -157,7 +158,7 @@ def _forward(x, w16, target, ce_weight, want_dx, chunk_rows):
 
 class FusedLinearCE(torch.autograd.Function):
     """apply(x, w16, target, ce_weight, chunk_rows) -> (loss, lse, target_logit, ce, entropy,
-    argmax). Only the loss is differentiable, in x; its dX comes from the forward."""
+    argmax). Only the loss is differentiable, in x; its dX product comes from the forward."""
 
     @staticmethod
     def forward(ctx, x, w16, target, ce_weight, chunk_rows):

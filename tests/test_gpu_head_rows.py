@@ -105,3 +105,37 @@ def test_odd_width_and_recorded_backward():
         torch.testing.assert_close(dx, 2 * plain, rtol=1e-6, atol=0)
         torch.testing.assert_close(dc, plain.sum(), rtol=1e-3, atol=1e-7)
         assert bool((plain[~live] == 0).all()) and bool((plain[live] != 0).any())
+
+
+def _loss(seed, dtype=torch.float32):
+    from solution.head import fused_linear_ce
+
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    x = torch.randn(50, 64, generator=g, device=DEV).to(dtype).requires_grad_()
+    w = (torch.randn(V, 64, generator=g, device=DEV) * 0.1).half()
+    target, cew, live, _ = _rows(50, seed)
+    cew = torch.where(live, cew, 0.0)
+    loss, _ = fused_linear_ce(x, w, target, cew)
+    return x, cew, live, loss
+
+
+def test_weights_refilled_before_backward():
+    """The caller's ce_weight is read by the forward only: its buffer may be refilled before the backward
+    pass."""
+    x, cew, _, loss = _loss(4)
+    (want,) = torch.autograd.grad(loss, x, retain_graph=True)
+    cew.fill_(3.0)
+    (got,) = torch.autograd.grad(loss, x)
+    assert torch.equal(got, want)
+
+
+def test_weights_from_inference_mode():
+    from solution.head import fused_linear_ce
+
+    with torch.inference_mode():
+        cew = torch.rand(20, device=DEV)
+    x = torch.randn(20, 64, device=DEV, requires_grad=True)
+    w, target = torch.randn(V, 64, device=DEV).half(), torch.arange(20, device=DEV)
+    (got,) = torch.autograd.grad(fused_linear_ce(x, w, target, cew)[0], x)
+    (want,) = torch.autograd.grad(fused_linear_ce(x, w, target, cew.clone())[0], x)
+    assert torch.equal(got, want)
