@@ -277,7 +277,8 @@ __global__ __launch_bounds__(kPartThreads) void k_head_loss(const int64_t* targe
 }
 
 // The product's rows back in place, scaled and cast in one pass (8 columns per thread), where a
-// multiply, a gather, another multiply and a cast took four.
+// multiply, a gather, another multiply and a cast took four. A row without a loss is 0 * dloss: a
+// non-finite dloss marks it like the others.
 template <typename O>
 __global__ __launch_bounds__(256) void k_head_dx(const float* prod, int64_t n_live,
                                                  const int32_t* inv, const float* cew,
@@ -288,13 +289,14 @@ __global__ __launch_bounds__(256) void k_head_dx(const float* prod, int64_t n_li
   if (i >= N) return;
   const int c = (int)(e % per);
   const int64_t at = inv[i];
-  float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  const float d = *dloss;
+  float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, s = 0.f;
   if (at < n_live) {
     Chunk<float>::load(prod + at * 8 * per + 8 * c, v);
-    const float s = cew[i] * inv_scale, d = *dloss;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) v[k] = v[k] * s * d;
+    s = cew[i] * inv_scale;
   }
+#pragma unroll
+  for (int k = 0; k < 8; ++k) v[k] = v[k] * s * d;
   Chunk<O>::store(dx + i * 8 * per + 8 * c, v);
 }
 

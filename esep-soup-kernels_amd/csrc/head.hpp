@@ -34,7 +34,7 @@ hipError_t launch_head_partition(const int64_t* target, const float* cew, int64_
 // *loss = sum of cew * ce over the rows with a target in [0, V).
 hipError_t launch_head_loss(const int64_t* target, const float* cew, const float* ce, int64_t N,
                             int64_t V, float* loss, hipStream_t s);
-// dx[i] = prod[inv[i]] * (cew[i] * inv_scale) * *dloss where inv[i] < n_live, else 0.
+// dx[i] = prod[inv[i]] * (cew[i] * inv_scale) * *dloss where inv[i] < n_live, else 0 * *dloss.
 hipError_t launch_head_dx(const float* prod, int64_t n_live, const int32_t* inv, const float* cew,
                           const float* dloss, float inv_scale, void* dx, int dx_dt, int64_t N,
                           int64_t H, hipStream_t s);

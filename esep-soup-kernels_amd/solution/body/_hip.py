@@ -803,7 +803,7 @@ def head_loss(target, cew, ce, V, name="_head_loss"):
 
 
 def head_dx(prod, inv, cew, dloss, g_scale, dx, name="_head_dx"):
-    """dx[i] = prod[inv[i]] * (cew[i] / g_scale) * dloss for the rows with inv[i] < len(prod), else 0
+    """dx[i] = prod[inv[i]] * (cew[i] / g_scale) * dloss for the rows with inv[i] < len(prod), else 0 * dloss
     (esep_head_dx). prod fp32 [n_live, H], inv int32 [N], cew fp32 [N], dloss one fp32 on the device,
     dx [N, H] of a float dtype; all contiguous, H a multiple of 8."""
     dev = _dev(prod, inv, cew, dloss, dx)

@@ -405,7 +405,7 @@ int esep_head_row_softmax(void* z, int64_t ld, const int64_t* target, const floa
  *                        in order; inv its inverse (int32 [N]); *n_live the first part's length
  *   esep_head_loss       *loss = sum of cew * ce over the rows with a target in [0, V), fixed order
  *   esep_head_dx         dx[i, :] = prod[inv[i], :] * (cew[i] / g_scale) * *dloss for inv[i] < n_live,
- *                        else 0: prod fp32 [n_live, H], dx [N, H] of dx_dt; H a multiple of 8,
+ *                        else 0 * *dloss: prod fp32 [n_live, H], dx [N, H] of dx_dt; H a multiple of 8,
  *                        prod and dx 16-byte aligned
  * 1 <= N < 2^31. No host synchronization.
  */

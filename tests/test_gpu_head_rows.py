@@ -139,3 +139,16 @@ def test_weights_from_inference_mode():
     (got,) = torch.autograd.grad(fused_linear_ce(x, w, target, cew)[0], x)
     (want,) = torch.autograd.grad(fused_linear_ce(x, w, target, cew.clone())[0], x)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("dloss", [float("inf"), float("-inf"), float("nan")])
+def test_gradient_of_a_loss_that_overflowed(dloss):
+    """dX is the finished gradient times the loss's: a non-finite one marks every row, also those without
+    a loss (0 * inf), in the kernel as in the tensor operations (odd widths, recorded passes)."""
+    x, _, live, loss = _loss(6, torch.float16)
+    assert bool(live.any()) and not bool(live.all())
+    (got,) = torch.autograd.grad(loss, x, torch.tensor(dloss, device=DEV), retain_graph=True)
+    scale = torch.tensor(dloss, device=DEV, requires_grad=True)
+    (want,) = torch.autograd.grad(loss, x, scale, create_graph=True)
+    torch.testing.assert_close(got, want.detach(), rtol=0, atol=0, equal_nan=True)
+    assert not bool(torch.isfinite(got[~live]).any())
