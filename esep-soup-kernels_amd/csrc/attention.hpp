@@ -30,6 +30,8 @@
 
 #include <cstdint>
 
+#include "common.hpp"
+
 namespace esep {
 
 struct AttnArgs {
@@ -330,14 +332,15 @@ __device__ __forceinline__ int seq_of_rank(const int32_t* cu, int n_seq, int64_t
 }
 
 // Longest blocks first over the whole launch (n_seq <= 64): what is started last is short, and the
-// CUs end with near-equal work. A block's work
-// is its tile's level (a query tile's keys, a key tile's queries, in 128-row tiles: 1 .. the
-// sequence's tile count), so the (sequence, tile) pairs are walked level by level from the
-// longest sequence's down, each pair's gps blocks (heads) in a row, and every wavefront finds its
-// pair with a ballot per level. Each second run of 256 places is reversed: the hardware deals
-// blocks breadth-first over the 256 CUs, so a CU that got one of the longest blocks of a run gets
-// one of the shortest of the next. The heads of a kv head then lie on different XCDs: an input of up
-// to a few rounds of blocks fits their L2s and the Infinity Cache.
+// CUs end with near-equal work. A block's work is its tile's level (a query tile's keys, a key
+// tile's queries, in 128-row tiles: 1 .. the sequence's tile count), so the (sequence, tile) pairs
+// are walked level by level from the longest sequence's down, each pair's gps blocks (heads) in a
+// row, and every wavefront finds its pair with a ballot per level. The walk starts at the longest
+// sequence's tiles, and blocks past the last pair leave before it: max_seqlen may be any bound, and
+// the grid's own count is as loose as that. Each second run of 256 places is reversed: the hardware
+// deals blocks breadth-first over the 256 CUs, so a CU that got one of the longest blocks of a run
+// gets one of the shortest of the next. The heads of a kv head then lie on different XCDs: an input
+// of up to a few rounds of blocks fits their L2s and the Infinity Cache.
 // Against xcd_order_lpt / the sorted order (bf16, us): dK / dV 123 -> 98, dQ 79 -> 65, forward 65 ->
 // 48 at 12011 tokens in 9 sequences, 14 / 2 heads, D = 64; dK / dV 98 -> 87, dQ 72 -> 68, forward 48 ->
 // 46 at 8 x 1024, 12 / 2 heads, D = 128. Without the reversal dQ of 5933 tokens is 46.0 against
@@ -356,15 +359,14 @@ __device__ __forceinline__ int level_order(int b, int nblk, int C, int groups, i
     tiles = (e - s + kAttnBM - 1) / kAttnBM;
     if (tiles > C) tiles = C;  // a sequence past max_seqlen: the tiles the grid holds, as elsewhere
   }
-  int pair = p / gps, level = C;
-  uint64_t has = 0;
-  for (; level >= 1; --level) {
-    has = __ballot(tiles >= level);
-    const int n = __popcll(has);
-    if (pair < n) break;
+  int pair = p / gps;
+  if (pair >= wave_sum_i(tiles)) return groups * C;
+  int level = wave_max_i(tiles);
+  uint64_t has = __ballot(tiles >= level);
+  for (int n = __popcll(has); pair >= n; n = __popcll(has)) {
     pair -= n;
+    has = __ballot(tiles >= --level);
   }
-  if (level < 1) return groups * C;
   const int rank = __popcll(has & ((1ull << lane) - 1));
   const uint64_t hit = __ballot(tiles >= level && rank == pair);
   const int seq = (int)__builtin_ctzll(hit);

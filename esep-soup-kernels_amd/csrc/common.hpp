@@ -266,6 +266,23 @@ __device__ __forceinline__ float wave_sum(float v) {
   return (r0 + r1) + (r2 + r3);
 }
 
+// The same for integers (all 64 lanes take part).
+template <typename F>
+__device__ __forceinline__ int wave_reduce_i(int v, F f) {
+  v = f(v, __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, false));
+  v = f(v, __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, false));
+  v = f(v, __builtin_amdgcn_update_dpp(0, v, 0x141, 0xF, 0xF, false));
+  v = f(v, __builtin_amdgcn_update_dpp(0, v, 0x140, 0xF, 0xF, false));
+  return f(f(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
+           f(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+}
+__device__ __forceinline__ int wave_sum_i(int v) {
+  return wave_reduce_i(v, [](int a, int b) { return a + b; });
+}
+__device__ __forceinline__ int wave_max_i(int v) {
+  return wave_reduce_i(v, [](int a, int b) { return a > b ? a : b; });
+}
+
 // Wave-scope ordering for a wave that writes LDS and then reads what other lanes wrote.
 __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
