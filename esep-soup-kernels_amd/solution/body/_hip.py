@@ -647,8 +647,8 @@ def linear(x, w, bias=None):
     else the vendor BLAS (which also serves a recorded backward pass)."""
     x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
     if (_plain(x, w, bias) and gemm_takes(x2, w, False)
-            and (bias is None or (bias.dtype == x.dtype and bias.dim() == 1 and bias.is_contiguous()
-                                  and bias.data_ptr() % 16 == 0))):
+            and (bias is None or (bias.dtype == x.dtype and bias.shape == w.shape[:1]
+                                  and bias.is_contiguous() and bias.data_ptr() % 16 == 0))):
         out = torch.empty((x2.shape[0], w.shape[0]), device=x.device, dtype=x.dtype)
         gemm(x2, w, out, bias=bias)
         return out.view(*x.shape[:-1], w.shape[0])

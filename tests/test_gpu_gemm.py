@@ -75,3 +75,12 @@ def test_linear_and_matmul_routes():
         assert _hip.linear(xx, ww).shape == (100, 256)
     with torch.autocast("cuda", dtype=torch.bfloat16):
         assert _hip.linear(x, w).dtype == torch.bfloat16
+
+
+def test_a_bias_that_broadcasts():
+    """F.linear takes biases that broadcast to the output: those are the library's."""
+    from solution.body import _hip
+
+    x, w = torch.randn(64, 1536, device=DEV).half(), torch.randn(128, 1536, device=DEV).half()
+    for bias in (torch.randn(1, device=DEV).half(), torch.randn(1, 128, device=DEV).half()):
+        assert torch.equal(_hip.linear(x, w, bias), torch.nn.functional.linear(x, w, bias))
