@@ -292,6 +292,18 @@ __device__ __forceinline__ int xcd_order(int b, int C) {
 }
 inline int64_t xcd_grid(int64_t C, int64_t groups) { return (groups + 7) / 8 * 8 * C; }
 
+// The launch of n such blocks and a block's number in it. A grid dimension counts its threads in 32
+// bits, silently: of 2^24 blocks of 256 threads and more only the remainder would run. Past
+// kGridFold blocks (a multiple of 8: the XCDs' turns go on) the grid has rows of that many; the
+// last row's spare numbers belong to no group.
+constexpr int64_t kGridFold = 1 << 22;
+inline dim3 attn_grid(int64_t n) {
+  return n <= kGridFold ? dim3((unsigned)n)
+                        : dim3((unsigned)kGridFold, (unsigned)((n + kGridFold - 1) / kGridFold));
+}
+inline bool attn_grid_ok(int64_t n) { return n <= 0x7fffffff - kGridFold; }  // numbers are ints
+__device__ __forceinline__ int attn_block() { return (int)(blockIdx.y * gridDim.x + blockIdx.x); }
+
 // xcd_order with each XCD running its groups tile-major: tile 0 of every group it holds, then
 // tile 1, and so on, in the order the hardware dispatches its workgroups; groups stay whole on one
 // XCD as with xcd_order. The kernels number a group's tiles heaviest first (causal: the query tile

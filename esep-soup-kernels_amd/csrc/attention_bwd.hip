@@ -118,7 +118,7 @@ __global__ __launch_bounds__(64 * NW, kDqPerCU<D>) void k_attn_bwd_dq_dma(const 
   constexpr int BM = 32 * NW;  // queries per block
   __shared__ __align__(1024) char kv[2][2][BN * RB];  // [buffer][K, V][swizzled tile]
 
-  const int lin = block_order((int)blockIdx.x, qtiles, a.HQ * a.n_seq, order, a.HQ, a.cu, a.n_seq,
+  const int lin = block_order(attn_block(), qtiles, a.HQ * a.n_seq, order, a.HQ, a.cu, a.n_seq,
                               a.T);
   const int bx = lin % qtiles, rest = lin / qtiles;
   const int h = rest % a.HQ, seq = rest / a.HQ;
@@ -236,7 +236,7 @@ __global__ __launch_bounds__(64 * NW, kDkdvPerCU) void k_attn_bwd_dkdv(const Att
   __shared__ __align__(1024) char vsm[BK * ROWB];  // this block's V rows (B operands of dP)
 
   const int split = b.split;                 // query-head groups per kv head
-  const int lin = block_order((int)blockIdx.x, ktiles, a.HK * split * a.n_seq, order, a.HK * split,
+  const int lin = block_order(attn_block(), ktiles, a.HK * split * a.n_seq, order, a.HK * split,
                               a.cu, a.n_seq, a.T);
   const int bx = lin % ktiles, rest = lin / ktiles;
   const int yy = rest % (a.HK * split), seq = rest / (a.HK * split);
@@ -470,16 +470,16 @@ hipError_t bwd_run(const AttnBwdArgs& b, int max_seqlen, hipStream_t s) {
   constexpr int QW = 4;
   const dim3 gq((max_seqlen + 32 * QW - 1) / (32 * QW), b.f.HQ, b.f.n_seq);
   const int64_t nq = xcd_grid(gq.x, (int64_t)gq.y * gq.z);
-  if (nq > 0x7fffffff) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((k_attn_bwd_dq_dma<T, D, D == 128 ? 32 : 64, QW>), dim3((unsigned)nq),
+  if (!attn_grid_ok(nq)) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((k_attn_bwd_dq_dma<T, D, D == 128 ? 32 : 64, QW>), attn_grid(nq),
                      dim3(64 * QW), 0, s, b, (int)gq.x, attn_order(nq, kDqPerCU<D>, b.f.n_seq, kRoundsQ));
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   constexpr int NW = 4, BQ = 32;
   const int64_t ktiles = (max_seqlen + 32 * NW - 1) / (32 * NW);
   const int64_t nk = xcd_grid(ktiles, (int64_t)b.f.HK * b.split * b.f.n_seq);
-  if (nk > 0x7fffffff) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((k_attn_bwd_dkdv<T, D, NW, BQ>), dim3((unsigned)nk), dim3(64 * NW), 0, s, b,
+  if (!attn_grid_ok(nk)) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((k_attn_bwd_dkdv<T, D, NW, BQ>), attn_grid(nk), dim3(64 * NW), 0, s, b,
                      (int)ktiles, attn_order(nk, kDkdvPerCU, b.f.n_seq, kRoundsKV));
   e = hipGetLastError();
   if (e != hipSuccess || b.split == 1) return e;

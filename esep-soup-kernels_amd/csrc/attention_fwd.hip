@@ -119,7 +119,7 @@ __global__ __launch_bounds__(kAttnThreads, kFwdPerCU<D>) void k_attn_fwd_swz(con
   using V8 = typename Mfma<T>::v8;
   __shared__ __align__(1024) char kv[NBUF][2][TILE];  // [buffer][K, V][swizzled rows]
 
-  const int lin = block_order((int)blockIdx.x, qtiles, a.HQ * a.n_seq, order, a.HQ, a.cu, a.n_seq,
+  const int lin = block_order(attn_block(), qtiles, a.HQ * a.n_seq, order, a.HQ, a.cu, a.n_seq,
                               a.T);
   const int bx = lin % qtiles, rest = lin / qtiles;
   const int h = rest % a.HQ, seq = rest / a.HQ;
@@ -207,8 +207,8 @@ __global__ __launch_bounds__(kAttnThreads, kFwdPerCU<D>) void k_attn_fwd_swz(con
 template <typename T, int D, int BN>
 hipError_t fwd_run(const AttnArgs& a, dim3 grid, hipStream_t s) {
   const int64_t n = xcd_grid(grid.x, (int64_t)grid.y * grid.z);
-  if (n > 0x7fffffff) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((k_attn_fwd_swz<T, D, BN, 2>), dim3((unsigned)n), dim3(kAttnThreads), 0, s, a,
+  if (!attn_grid_ok(n)) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((k_attn_fwd_swz<T, D, BN, 2>), attn_grid(n), dim3(kAttnThreads), 0, s, a,
                      (int)grid.x, attn_order(n, kFwdPerCU<D>, a.n_seq, kRoundsQ));
   return hipGetLastError();
 }

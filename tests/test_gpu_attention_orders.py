@@ -76,3 +76,13 @@ def test_a_loose_bound_costs_little(D):
 
     tight, loose = us(128), us(65536)
     assert loose < 3 * tight, (tight, loose)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_more_blocks_than_one_grid_dimension_holds(D):
+    """20000 short sequences under a loose bound: 17.9 million blocks, where HIP takes fewer than 2^32
+    threads (2^24 blocks) per grid dimension."""
+    lens = [1 + i % 8 for i in range(20000)]
+    ins = _inputs(sum(lens), 14, 2, D)
+    for a, b in zip(_run(ins, lens, 8192), _run(ins, lens, 8)):
+        assert torch.equal(a, b)
