@@ -873,7 +873,7 @@ int esep_nf4_dequant(const void* packed, const uint8_t* absmax, const float* abs
     return fail(ESEP_EINVAL, "nf4_dequant: every pointer is required");
   if ((reinterpret_cast<uintptr_t>(packed) & 7) || !aligned16(out))
     return fail(ESEP_EALIGN, "nf4_dequant: packed needs 8-byte and out 16-byte alignment");
-  if (n_blocks > (int64_t{1} << 36))  // 4 TiB of packed bytes: past every memory, and the grid's limit
+  if (n_blocks > (int64_t{1} << 36))  // 2 TiB of packed bytes: past every memory
     return fail(ESEP_ESHAPE, "nf4_dequant: too many blocks for one launch");
   esep::Nf4Multi m{};
   m.n = 1;

@@ -72,6 +72,13 @@ __device__ __forceinline__ float nf4_scale(const uint8_t* __restrict__ absmax,
   return prod + off;
 }
 
+// A grid dimension counts its threads in 32 bits, silently: of 2^24 blocks and more only the
+// remainder would run. Grids past kNf4Fold blocks have rows of that many.
+constexpr int64_t kNf4Fold = 1 << 22;
+__device__ __forceinline__ int64_t nf4_block() {
+  return (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
+}
+
 // Several weights, their units laid end to end (weight w: units [u0[w], u0[w + 1]), whole scale
 // blocks). A block takes U runs of 256 units. While the packed bytes are on their way, one thread per
 // scale block resolves its scale (absmax -> code2 is a dependent pair of loads) into LDS, so the
@@ -82,7 +89,7 @@ __global__ __launch_bounds__(kNf4Threads) void k_nf4_dequant_multi(const Nf4Mult
   __shared__ float tab[kNf4MultiMax][16];
   __shared__ float scl[kScales];
   const int tid = threadIdx.x;
-  const int64_t g0 = (int64_t)blockIdx.x * (kNf4Threads * U);
+  const int64_t g0 = nf4_block() * (kNf4Threads * U);
   const int64_t total = m.u0[m.n];
   auto weight_of = [&](int64_t u) {
     int wi = 0;
@@ -125,7 +132,7 @@ template <typename TO, int U>
 __global__ __launch_bounds__(kNf4Threads) void k_nf4_dequant_one(const Nf4Args w) {
   __shared__ float tab[16];
   const int tid = threadIdx.x;
-  const int64_t g0 = (int64_t)blockIdx.x * (kNf4Threads * U) + tid;
+  const int64_t g0 = nf4_block() * (kNf4Threads * U) + tid;
   const int64_t total = 8 * w.n_blocks;
   uint32_t raw[U];
   float scale[U];
@@ -150,8 +157,9 @@ template <typename TO>
 void launch(const Nf4Multi& m, hipStream_t s) {
   const int64_t units = m.u0[m.n];
   auto grid = [&](int u) {
-    const int64_t per = (int64_t)kNf4Threads * u;
-    return dim3((unsigned)((units + per - 1) / per));
+    const int64_t per = (int64_t)kNf4Threads * u, blocks = (units + per - 1) / per;
+    return blocks <= kNf4Fold ? dim3((unsigned)blocks)
+                              : dim3((unsigned)kNf4Fold, (unsigned)((blocks + kNf4Fold - 1) / kNf4Fold));
   };
   const dim3 block(kNf4Threads);
   if (m.n == 1)

@@ -61,3 +61,31 @@ def test_several_weights(sizes, dtype):
     for nb, (raw, table, dev, buf) in zip(sizes, ws):
         assert torch.equal(buf[:nb * 64].cpu(), _want(raw, table, dtype))
         assert (buf[nb * 64:] == 7).all()
+
+
+def test_more_units_than_one_grid_dimension_holds():
+    """2^30 scale blocks and more: a launch of 2^32 threads, which a grid dimension cannot count
+    (34 GB of packed bytes, 137 GB of fp16)."""
+    from solution.body import _hip
+
+    nb = (1 << 30) + 1000
+    if torch.cuda.mem_get_info()[0] < 200 << 30:
+        pytest.skip("needs 200 GB of free GPU memory")
+    _, _, (_, _, _, code2, offset, table), _ = _weight(4, 1, torch.float16)
+    packed = torch.zeros(nb * 32, device=DEV, dtype=torch.uint8)
+    absmax = torch.zeros(nb, device=DEV, dtype=torch.uint8)
+    absmax2 = torch.full(((nb + 255) // 256,), 0.25, device=DEV)
+    out = torch.zeros(nb, 64, device=DEV, dtype=torch.float16)
+    at = torch.tensor([0, 999, (1 << 22), (1 << 29) + 3, nb - 1001, nb - 1], device=DEV)
+    g = torch.Generator(device=DEV).manual_seed(1)
+    bytes_ = torch.randint(0, 256, (6, 32), generator=g, device=DEV, dtype=torch.uint8)
+    packed.view(nb, 32)[at] = bytes_
+    absmax[at] = torch.arange(6, device=DEV, dtype=torch.uint8) * 40 + 3
+    want = torch.empty(6, 64, device=DEV, dtype=torch.float16)
+    _hip.nf4_dequant(bytes_, absmax[at], absmax2[:1], code2, offset, table, want)
+    _hip.nf4_dequant(packed, absmax, absmax2, code2, offset, table, out)
+    assert torch.equal(out[at], want)
+    zero = out[at + torch.tensor([1, 1, 1, 1, 1, -1], device=DEV)]  # neighbours: one value each
+    assert bool((zero == zero[0, 0]).all()) and float(zero[0, 0]) != 0
+    del packed, out
+    torch.cuda.empty_cache()
