@@ -1001,8 +1001,9 @@ int esep_head_dx(const float* prod, int64_t n_live, const int32_t* inv, const fl
                  void* stream) {
   g_err[0] = 0;
   if (!float_dt(dx_dt)) return fail(ESEP_EINVAL, "head_dx: bad dtype code %d", dx_dt);
-  if (N < 1 || H < 8 || H % 8 != 0 || n_live < 0 || n_live > N || H > (1 << 24) ||
-      N * (H / 8) > (1LL << 38))
+  // N < 2^31 before the product; a grid dimension counts fewer than 2^32 threads, one per 8 columns
+  if (N < 1 || N > 0x7fffffffLL || H < 8 || H % 8 != 0 || n_live < 0 || n_live > N ||
+      H > (1 << 24) || N * (H / 8) > (1LL << 32) - 256)
     return fail(ESEP_ESHAPE, "head_dx: N=%lld, H=%lld, n_live=%lld", (long long)N, (long long)H,
                 (long long)n_live);
   if ((n_live > 0 && prod == nullptr) || inv == nullptr || cew == nullptr || dloss == nullptr ||

@@ -58,6 +58,7 @@ EINVAL, ESHAPE, EALIGN = -1, -2, -3
     ("esep_head_loss", LOSS, dict(V=0), ESHAPE), ("esep_head_loss", LOSS, dict(ce=None), EINVAL),
     ("esep_head_dx", DX, dict(dx_dt=7), EINVAL), ("esep_head_dx", DX, dict(H=60), ESHAPE),
     ("esep_head_dx", DX, dict(n_live=5), ESHAPE), ("esep_head_dx", DX, dict(prod=None), EINVAL),
+    ("esep_head_dx", DX, dict(N=1 << 29, H=64), ESHAPE), ("esep_head_dx", DX, dict(N=1 << 62), ESHAPE),
     ("esep_head_dx", DX, dict(g_scale=0.0), EINVAL), ("esep_head_dx", DX, dict(dx=A + 4), EALIGN),
 ])
 def test_arguments_are_refused(name, base, kw, status):
