@@ -1,8 +1,8 @@
 // C[M, N] = A[M, K] . B (+ bias) on MFMA for 16-bit operands with fp32 accumulation, B given as
 // [N, K] (a weight as it is stored: the forward's x W^T) or as [K, N] (the same weight in the
-// backward's dy W). Used where it beats hipBLASLt (gemm_plan): few output tiles under a long
+// backward's dy W). Used where it beats hipBLASLt (gemm_pays): few output tiles under a long
 // contraction, where the library leaves most CUs idle (fp16, 1031 x 1536 x 17920, B [K, N]:
-// 197 us against 71 here on four splits of the contraction), and few rows.
+// 199 us against 74 here on four splits of the contraction).
 //
 // A block of WM x WN wavefronts owns a tile of C, each wavefront 32 TM x 32 TN of it in fp32
 // accumulators. A and B move in 64-deep tiles by dwordx4 LDS DMA through two buffers: rows of
@@ -389,25 +389,42 @@ GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K) {
   return best;
 }
 
-// Against hipBLASLt (fp16, torch.mm), by the count t of 256 x 256 output tiles; library / here, us:
-//   B [K, N]: t <= 100 wins (1031 x 1536 x 8960 63 / 42, 4096 x 1536 x 17920 296 / 223, and the LM head's
-//     904 x 1536 x 151936 829 / 500) except near t = 56 at K = 4608 (45 / 47) and at the head's full
-//     chunk (4096 x 1536 x 151936 1692 / 1720; 3750 rows 2485 / 1673); so does t >= 250 with a short
-//     contraction up to 4096 rows (2300 x 8960 x 1536 78 / 67). 1031 x 8960 x 1536 (t = 141) 32 / 37 and
-//     8192 x 1536 x 17920 357 / 424 stay with the library.
-//   B [N, K]: t <= 30 (1031 x 1536 x 8960 47 / 42), up to 512 rows t <= 64 or t >= 400 (400 x 8960 x 1536
-//     23 / 18.5, 200 x 151936 x 1536 175 / 144), a very long contraction t <= 100 (4096 x 1536 x 17920
-//     303 / 223); the library is ahead elsewhere (2300 x 1536 x 8960 66 / 71, 1031 x 8960 x 1536
-//     30 / 38, 400 x 17920 x 1536 29 / 36, 3000 x 151936 x 1536 1213 / 1320).
+// A table, placed by hand from 3660 products measured against hipBLASLt (torch.mm), M = 16 .. 8192 over
+// the projections of fifteen decoder widths and vocabularies, fp16 and bf16 (alike within a few
+// percent), launches back to back on warm operands. Ranges of t, the count of 256 x 256 output tiles,
+// with the ratio here / library in them (geometric mean, worst) and, after the bar, outside:
+//   B [K, N], where the library rarely splits the contraction: the longer it is, the wider the range
+//     K >= 16384    t < 96           0.50, 1.09 (1031 x 1536 x 17920 199 us / 74) | 1.02 at the LM head's full
+//                                    chunk (4096 x 1536 x 151936 1721 / 1764), 1.1 .. 1.25 past it
+//     12288 ..      t <= 75          0.61, 0.92 | 1.06 .. 1.26
+//     8192 ..       t <= 48, 64 .. 80  0.65, 1.11 | 1.06 .. 1.16 between, where the plan's unsplit 128-wide
+//                                    tiles lose (2300 x 1536 x 8960 79 us / 91), 1.2 past 88
+//     3328 ..       t = 1 .. 36      0.81, 1.12 | 1.1 .. 1.33 past 40
+//     2049 ..       none             0.64 .. 1.30 without a pattern
+//     1281 ..       t = 52 .. 72     0.89, 1.05 (3001 x 1536 x 1536 29 us / 24) | 1.04 .. 1.37 on either side
+//     896 ..        t = 12 .. 64     0.82, 1.07 | up to 1.56 below, 1.26 above
+//   B [N, K], which the library serves better
+//     K >= 16384    t = 1 .. 95      0.56, 1.06
+//     12288 ..      t = 4 .. 40      0.86, 1.05 | 1.1 .. 1.4
+//     8192 ..       t = 4 .. 20      0.85, 1.06 | 1.05 .. 1.4
+//     896 ..        the LM head's logits up to 32 rows 0.79, 0.98, and at 385 .. 512 (two full 256-row tiles)
+//                   0.91, 0.98 | 300 rows 185 us / 240; 4096 x 256 x 1536 9 / 22, 512 x 2048 x 1536 9 / 18
+// Of the 995 measured products that it takes, 11 are more than 5% slower here.
 bool gemm_pays(int64_t M, int64_t N, int64_t K, bool b_kn) {
-  if (K < 896) return false;  // not measured
   const double t = (double)M * N / 65536;
   if (b_kn) {
-    if (t <= 40) return true;
-    if (t <= 100) return K <= 2560 || (K >= 6144 && (t <= 94 || K <= 32768));
-    return t >= 250 && K <= 2560 && M <= 4096;
+    if (K >= 16384) return t < 96;
+    if (K >= 12288) return t <= 75;
+    if (K >= 8192) return t <= 48 || (t >= 64 && t <= 80);
+    if (K >= 3328) return t >= 1 && t <= 36;
+    if (K > 2048) return false;
+    if (K > 1280) return t >= 52 && t < 72;
+    return K >= 896 && t >= 12 && t <= 64;  // below 896 not measured
   }
-  return t <= 30 || (M <= 512 && (t <= 64 || t >= 400)) || (K >= 12288 && t <= 100);
+  if (K >= 16384) return t >= 1 && t < 96;
+  if (K >= 12288) return t >= 4 && t <= 40;
+  if (K >= 8192) return t >= 4 && t <= 20;
+  return K >= 896 && ((M <= 32 && t >= 32) || (M > 384 && M <= 512 && t >= 800));
 }
 
 hipError_t launch_gemm(const GemmArgs& a, int shape, int b_kn, int dt, int out_dt, hipStream_t s,

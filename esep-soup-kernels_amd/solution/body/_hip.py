@@ -642,11 +642,19 @@ def _plain(x, w, bias=None):
     return not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == x.dtype
 
 
+def _gemm_pays(x, w, b_kn):
+    """The sizes alone: asked first, so that the library's products pay for nothing more."""
+    if not x.is_cuda or w.dim() != 2:
+        return False
+    k, n = w.shape if b_kn else (w.shape[1], w.shape[0])
+    return k > 0 and x.shape[-1:] == (k,) and lib().esep_gemm_pays(x.numel() // k, n, k, int(b_kn))
+
+
 def linear(x, w, bias=None):
     """F.linear(x, w, bias) for autograd Functions: esep_gemm where it takes the operands and pays,
     else the vendor BLAS (which also serves a recorded backward pass)."""
-    x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
-    if (_plain(x, w, bias) and gemm_takes(x2, w, False)
+    if (_gemm_pays(x, w, False) and _plain(x, w, bias)
+            and gemm_takes(x2 := x.reshape(-1, x.shape[-1]), w, False, pays=False)
             and (bias is None or (bias.dtype == x.dtype and bias.shape == w.shape[:1]
                                   and bias.is_contiguous() and bias.data_ptr() % 16 == 0))):
         out = torch.empty((x2.shape[0], w.shape[0]), device=x.device, dtype=x.dtype)
@@ -657,8 +665,8 @@ def linear(x, w, bias=None):
 
 def matmul(x, w):
     """x @ w for a 2-D w [K, N], as linear."""
-    x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
-    if _plain(x, w) and gemm_takes(x2, w, True):
+    if (_gemm_pays(x, w, True) and _plain(x, w)
+            and gemm_takes(x2 := x.reshape(-1, x.shape[-1]), w, True, pays=False)):
         out = torch.empty((x2.shape[0], w.shape[1]), device=x.device, dtype=x.dtype)
         gemm(x2, w, out, b_kn=True)
         return out.view(*x.shape[:-1], w.shape[1])

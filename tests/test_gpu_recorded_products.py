@@ -196,31 +196,31 @@ class _State:
 
 @pytest.mark.parametrize("multi", [False, True])
 def test_nf4_backward_under_vmap_and_forward_mode(multi):
-    """The NF4 linears' dX where esep_gemm would take it (n = 1536 outputs contracted)."""
+    """The NF4 linears' dX where esep_gemm would take it (17920 outputs contracted)."""
     from solution import nf4
     from solution.body import _hip
 
-    st = _State(1536, 64)
+    st = _State(17920, 64)
     x = _rnd(T, 64).requires_grad_()
     y = (nf4.NF4MultiLinear.apply(x, None, ([st.packed], [st], None)) if multi
          else nf4.nf4_linear(x, st.packed, None, st))
-    d = torch.stack([_rnd(T, 1536), _rnd(T, 1536, seed=3)])
+    d = torch.stack([_rnd(T, 17920), _rnd(T, 17920, seed=3)])
     with _hip.count_launches() as names:
         want = [torch.autograd.grad(y, x, di, retain_graph=True)[0] for di in d]
     assert "_gemm" in names
     (got,) = torch.autograd.grad(y, x, d, is_grads_batched=True, retain_graph=True)
     for a, b in zip(got, want):
-        torch.testing.assert_close(a, b, rtol=4e-3, atol=2e-2)  # sums of 1536 terms, two kernels
+        torch.testing.assert_close(a, b, rtol=4e-3, atol=1e-2)  # |dX| about 0.5, two kernels
     with fwd.dual_level():
         (dx,) = torch.autograd.grad(y, x, fwd.make_dual(d[0], d[1]), retain_graph=True)
-        torch.testing.assert_close(fwd.unpack_dual(dx).tangent, want[1], rtol=4e-3, atol=2e-2)
+        torch.testing.assert_close(fwd.unpack_dual(dx).tangent, want[1], rtol=4e-3, atol=1e-2)
 
 
 def test_linear_and_matmul_see_every_operand():
     """A weight or a bias that requires grad in grad mode goes to torch's product too."""
     from solution.body import _hip
 
-    x, w, wk, b = _rnd(T, 1536), _rnd(N, 1536), _rnd(1536, N), _rnd(N)
+    x, w, wk, b = _rnd(T, 17920), _rnd(2048, 17920), _rnd(17920, N), _rnd(2048)
     for t in (w, b):
         t.requires_grad_()
         assert _hip.linear(x, w, b).requires_grad
