@@ -183,19 +183,20 @@ def _stream(dev):
     return _current_stream(dev) if _raw_stream is None else _raw_stream(dev.index)
 
 
+_functorch_wrapped = torch._C._functorch.is_functorch_wrapped_tensor
+_batched = torch._C._functorch.is_legacy_batchedtensor
+
+
 def recorded(*tensors):
     """Torch has to see the operations on these tensors as its own (a kernel would fill a buffer behind
     its back): one requires grad in grad mode, carries a forward-mode tangent, or is a functorch
     wrapper (vmap, batched gradients, torch.func), which has no memory of its own."""
-    tensors = [t for t in tensors if t is not None]
-    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
-        return True
-    functorch = torch._C._functorch
-    if any(functorch.is_functorch_wrapped_tensor(t) or functorch.is_legacy_batchedtensor(t)
-           for t in tensors):
-        return True
-    return forward_ad._current_level >= 0 and any(
-        forward_ad.unpack_dual(t).tangent is not None for t in tensors)
+    grad, dual = torch.is_grad_enabled(), forward_ad._current_level >= 0
+    for t in tensors:
+        if t is not None and ((grad and t.requires_grad) or _functorch_wrapped(t) or _batched(t)
+                              or (dual and forward_ad.unpack_dual(t).tangent is not None)):
+            return True
+    return False
 
 
 def _rows_ld(t, n):
