@@ -1,6 +1,7 @@
 """LoRA terms of q_proj / v_proj with dropout on the LoRA input, on this repository's fused HIP
 products (esep_lora_down / esep_lora_up / esep_lora_grads: the mask regenerated inside them), or
-its dropout kernels around vendor-BLAS products for the ranks and sizes those do not take.
+its dropout kernels around vendor-BLAS products for the ranks and sizes that those do not take or
+are slower at.
 
 Public API as in the reference's solution/body/lora.py (reference lora.py:140-359):
 new_dropout_key, cast_lora_weights, lora_dropout, lora_down_fwd, lora_down_bwd, lora_delta,
@@ -74,6 +75,56 @@ def _fused(rank, *mats):
     return True
 
 
+# Where each fused product is the faster one, by rows, width (the long side) and rank, against the
+# library's products and the dropout kernels around them: measured on an MI355X for 16 .. 40000 rows,
+# widths 64 .. 18944 and ranks 8, 16, 32, 64 in fp16 and bf16 (alike), kernel time of launches back to
+# back, library / fused in us. The down kernel's blocks own 16 .. 64 rows and read all of the weight, so
+# it loses on wide weights (width x rank) and on few blocks; the gradients' partial sums grow
+# with the rank. The term without a base is always the fused kernel's (0.2 .. 0.8 of the library's).
+
+
+def _down_pays(rows, width, rank, dropout):
+    """xa. Without dropout the library reads x once too (rows x width x rank): 4096 x 1536 x 16 5.0 / 4.9,
+    5933 x 1536 x 16 5.8 / 7.6, 200 x 8960 x 64 9.9 / 40. With it, the dropout pass is extra: 5933 x 1536
+    x 16 26 / 12, but 64 x 8960 x 64 21 / 42 and 40000 x 896 x 64 48 / 61."""
+    if dropout:
+        return (width <= 2048 or rows >= 1000) if rank <= 32 else width <= 2048 and rows < 8192
+    return rows <= 4096 and width * max(rank, 16) <= 32768
+
+
+def _dxa_pays(rows, width, rank):
+    """dxa = scaling * dterm B (two library launches): 5933 x 1536 x 16 8.7 / 6.1, 1000 x 3584 x 16 9.6 / 7.3, but
+    2000 x 8960 x 32 21 / 34 and 9000 x 1536 x 64 14 / 20."""
+    if width > 2048:
+        return width <= 4096 and 32 <= rows <= 2048
+    return rank <= 16 or rows < (8192 if rank > 32 else 32768)
+
+
+def _down_grads_pay(rows, width, rank, dropout, need_dx):
+    """dx and dA from one read of x: 5933 x 1536 x 16 29 / 21, with dropout 55 / 26, but 200 x 3584 x 64 11 / 16
+    and without dropout 9000 x 8960 x 64 111 / 145. dA alone without dropout is one library product: 4096
+    x 1536 x 16 11 / 15, 9000 x 1536 x 16 25 / 18."""
+    if not need_dx and not dropout:
+        return rows >= 5000 and width <= 4096
+    if rank > 32:
+        return rows >= 1000 and (dropout or width <= 4096)
+    return rank <= 16 or dropout or rows >= 100
+
+
+def _up_grads_pay(rows, width, rank):
+    """dB: 0.3 .. 0.9 of the library up to 4096 wide, but 4096 x 8960 x 16 21 / 27, 4096 x 18944 x 64 42 / 69 and
+    64 x 3584 x 64 6.8 / 8.3."""
+    if width <= 4096:
+        return rank <= 32 or rows >= 450
+    return rank <= 16 and rows <= 1000
+
+
+def _base_pays(rank):
+    """base + term, one library product: 4096 x 1536 x 16 10.9 / 7.5 (0.4 .. 1.1 up to rank 16), 9000 x 1536 x 64
+    13 / 22 (0.5 .. 1.7 from 32 on)."""
+    return rank <= 16
+
+
 _OUT_DTYPE_OK = True
 
 
@@ -89,14 +140,18 @@ def _mm_fp32(a, b):
     return torch.mm(a, b).float()
 
 
-def lora_down_fwd(x, a16, key, p):
-    """xa = drop(x) @ A^T for a dense x [T, in] (no dropout when p == 0)."""
-    if (not _hip.recorded(x, a16) and _fused(a16.shape[0], x, a16) and x.is_contiguous()
-            and a16.is_contiguous()):
+def _xa(x, a16, key, p, fused):
+    if fused and _down_pays(*x.shape, a16.shape[0], p > 0.0):
         xa = torch.empty((x.shape[0], a16.shape[0]), device=x.device, dtype=x.dtype)
         _hip.lora_down(x, a16, xa, key=key if p > 0.0 else None, p=p)
         return xa
     return torch.mm(lora_dropout(x, key, p) if p > 0.0 else x, a16.t())
+
+
+def lora_down_fwd(x, a16, key, p):
+    """xa = drop(x) @ A^T for a dense x [T, in] (no dropout when p == 0)."""
+    return _xa(x, a16, key, p, not _hip.recorded(x, a16) and _fused(a16.shape[0], x, a16)
+               and x.is_contiguous() and a16.is_contiguous())
 
 
 def _dense(t, like):
@@ -115,10 +170,12 @@ def _up_bwd_fused(dout, xa, b16):
             and dout.dtype == xa.dtype == b16.dtype)
 
 
-def _dxa(dout, b16, scaling):
-    dxa = torch.empty((dout.shape[0], b16.shape[1]), device=dout.device, dtype=dout.dtype)
-    _hip.lora_down(dout, b16, dxa, scale=scaling, w_kr=True)
-    return dxa
+def _dxa(dout, b16, scaling, fused):
+    if fused and _dxa_pays(*dout.shape, b16.shape[1]):
+        dxa = torch.empty((dout.shape[0], b16.shape[1]), device=dout.device, dtype=dout.dtype)
+        _hip.lora_down(dout, b16, dxa, scale=scaling, w_kr=True)
+        return dxa
+    return torch.mm(dout, b16).mul_(scaling)
 
 
 def lora_down_bwd(x, a16, dxa, key, p, need_dx=True, dx_accum=None):
@@ -126,6 +183,7 @@ def lora_down_bwd(x, a16, dxa, key, p, need_dx=True, dx_accum=None):
     [T, in] buffer, e.g. the base projection's dx) the LoRA part of dx is added into it in
     place and it is returned as dx."""
     if (not _hip.recorded(x, a16, dxa, dx_accum) and _grads_fused(x, a16, dxa)
+            and _down_grads_pay(*x.shape, a16.shape[0], p > 0.0, need_dx)
             and (not need_dx or dx_accum is None or _dense(dx_accum, x))):
         dx = None
         if need_dx:
@@ -162,11 +220,13 @@ def lora_delta(xa, b16, scaling):
 
 def lora_up_bwd(dout, xa, b16, scaling):
     """(dxa [T, r], dB fp32 [out, r]) for the term's gradient dout."""
-    if not _hip.recorded(dout, xa, b16) and _up_bwd_fused(dout, xa, b16):
+    fused = not _hip.recorded(dout, xa, b16) and _up_bwd_fused(dout, xa, b16)
+    if fused and _up_grads_pay(*dout.shape, b16.shape[1]):
         db = torch.empty(b16.shape, device=dout.device, dtype=torch.float32)
         _hip.lora_grads(dterm=dout, xa=xa, scale=scaling, db=db)
-        return _dxa(dout, b16, scaling), db
-    return torch.mm(dout, b16).mul_(scaling), _mm_fp32(dout.t(), xa).mul_(scaling)
+    else:
+        db = _mm_fp32(dout.t(), xa).mul_(scaling)
+    return _dxa(dout, b16, scaling, fused), db
 
 
 def _rows(t, dtype):
@@ -197,11 +257,7 @@ class _LoRATerm:
         key = new_dropout_key(x2.device) if p > 0.0 else None
         ctx.fused = (_fused(a16.shape[0], x2, a16, b16) and a16.is_contiguous()
                      and b16.is_contiguous() and b16.shape[0] % 8 == 0)
-        if ctx.fused:
-            xa = torch.empty((x2.shape[0], a16.shape[0]), device=x2.device, dtype=dtype)
-            _hip.lora_down(x2, a16, xa, key=key, p=p)
-        else:
-            xa = lora_down_fwd(x2, a16, key, p)
+        xa = _xa(x2, a16, key, p, True) if ctx.fused else lora_down_fwd(x2, a16, key, p)
         ctx.save_for_backward(x2, xa, a16, b16, key)
         ctx.p, ctx.scaling, ctx.dtype = p, scaling, dtype
         ctx.x_shape, ctx.x_dtype = x.shape, x.dtype
@@ -215,9 +271,11 @@ class _LoRATerm:
         dt2 = _rows_mm(dterm, ctx.dtype)
         # torch's products for a pass with create_graph, under vmap (is_grads_batched), with a tangent
         recorded = _hip.recorded(dt2, x2, xa, a16, b16)
-        if ctx.fused and not recorded and _fused(b16.shape[1], dt2):
+        rank, dropout = b16.shape[1], ctx.p > 0.0
+        if (ctx.fused and not recorded and _fused(rank, dt2) and _up_grads_pay(*dt2.shape, rank)
+                and _down_grads_pay(*x2.shape, rank, dropout, need[x_index])):
             # dx, dA and dB in one launch after dxa
-            dxa = _dxa(dt2, b16, ctx.scaling)
+            dxa = _dxa(dt2, b16, ctx.scaling, True)
             dx = torch.empty_like(x2) if need[x_index] else None
             da = torch.empty(a16.shape, device=x2.device, dtype=torch.float32)
             db = torch.empty(b16.shape, device=x2.device, dtype=torch.float32)
@@ -243,14 +301,14 @@ class LoRAFunction(torch.autograd.Function):
         ctx.base_dtype = base.dtype
         if base.dtype == ctx.dtype and base.is_contiguous() and not base._is_view():
             flat = base.view(-1, base.shape[-1])
-            if ctx.fused and _fused(b16.shape[1], flat):
+            if ctx.fused and _base_pays(b16.shape[1]) and _fused(b16.shape[1], flat):
                 _hip.lora_up(xa, b16, flat, scaling, base=flat)
             else:
                 flat.addmm_(xa, b16.t(), alpha=scaling)
             ctx.mark_dirty(base)
             return base
         flat = base.reshape(-1, base.shape[-1]).to(ctx.dtype)
-        if ctx.fused and _fused(b16.shape[1], flat):
+        if ctx.fused and _base_pays(b16.shape[1]) and _fused(b16.shape[1], flat):
             out = torch.empty(flat.shape, device=flat.device, dtype=flat.dtype)
             _hip.lora_up(xa, b16, out, scaling, base=flat)
             return out.view(base.shape)

@@ -17,6 +17,17 @@ from oracle import lora_ref as ref
 pytestmark = pytest.mark.gpu
 
 U = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}
+
+
+@pytest.fixture
+def kernels(monkeypatch):
+    """Every product on the fused kernels, also where the library is the faster one."""
+    from solution.body import lora as L
+
+    for name in ("_down_pays", "_dxa_pays", "_down_grads_pay", "_up_grads_pay", "_base_pays"):
+        monkeypatch.setattr(L, name, lambda *a: True)
+
+
 KEY = 0x1357_9BDF_2468_ACE
 
 # (T, in, out, rank): one row; a ragged 16-row tile with narrow sides; ranks between tiles; the
@@ -34,7 +45,7 @@ def _close(got, want, bound, what):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
 @pytest.mark.parametrize("p", [0.0, 0.1])
 @pytest.mark.parametrize("T,K,N,r", SHAPES)
-def test_fused_products(T, K, N, r, p, dtype):
+def test_fused_products(T, K, N, r, p, dtype, kernels):
     from solution.body import lora as L
 
     g, u, s = gen(T + K + r), U[dtype], 2.0
@@ -107,3 +118,30 @@ def test_other_ranks_and_layouts_keep_their_path():
         for got, w in zip((term, *grads), (want, *wants)):
             # a chain of three fp16 roundings
             assert (got.double() - w).abs().max() <= 4 * 2.0 ** -11 * w.abs().max()
+
+
+@pytest.mark.parametrize("p", [0.0, 0.1])
+@pytest.mark.parametrize("T,K,N,r", [(200, 3584, 256, 64), (64, 8960, 64, 32), (2000, 256, 8960, 16),
+                                     (6000, 1536, 64, 16)])
+def test_routes_agree(T, K, N, r, p, monkeypatch):
+    """Where a product goes changes its rounding alone: the whole term, forward and backward, on the
+    kernels, on the library and as the rules say. Results of a chain of at most four fp16 roundings."""
+    from solution.body import lora as L
+
+    g = gen(T + K)
+    x = torch.randn(T, K, generator=g).half().to(DEV).requires_grad_()
+    a = (torch.randn(r, K, generator=g) * 0.05).to(DEV).requires_grad_()
+    b = (torch.randn(N, r, generator=g) * 0.05).to(DEV).requires_grad_()
+    base, d = (torch.randn(T, N, generator=g).half().to(DEV) for _ in range(2))
+    monkeypatch.setattr(L, "new_dropout_key", lambda device: torch.tensor([KEY], device=device))
+    names = ("_down_pays", "_dxa_pays", "_down_grads_pay", "_up_grads_pay", "_base_pays")
+    outs = []
+    for route in (True, False, None):
+        with monkeypatch.context() as m:
+            for name in names if route is not None else ():
+                m.setattr(L, name, lambda *args, route=route: route)
+            out = L.LoRAFunction.apply(x, base.clone(), a, b, p, 2.0)
+            outs.append((out, *torch.autograd.grad(out, (x, a, b), d)))
+    for one in outs[1:]:
+        for got, want in zip(one, outs[0]):
+            assert (got - want).float().abs().max() <= 4 * 2.0 ** -11 * want.float().abs().max()
