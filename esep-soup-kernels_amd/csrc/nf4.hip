@@ -12,12 +12,7 @@
 // apart, all requested before any is decoded. The 16-entry NF4 tables sit in LDS. 16 elements per
 // thread left every store of a wavefront a stride of 32 bytes (fp32: 64) apart. Before -> now in us:
 // 17920 x 1536 in fp32 86 -> 35 by k_nf4_dequant_one; in fp16 20 -> 19.5 by it, two weights of half that size
-// 19.7 -> 18 by k_nf4_dequant_multi (69 MB: 3.8 TB/s). The stores are plain: past the caches
-// (non-temporal) the same kernels take 18.7 and 16.7, but the GEMM that reads the weight next
-// loses more than that (1031 x 17920 x 1536: 64.5 -> 61 with the weight in the caches, its dX
-// 69.5 -> 68; 3001 x 8960 x 1536: 100 -> 92).
-// Where nothing reads the weight (one launch over a layer's seven, written again and again) they
-// cost 28.8 -> 30.6.
+// 19.7 -> 18 by k_nf4_dequant_multi (69 MB: 3.8 TB/s). Stores: see kNf4Stream.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -34,9 +29,17 @@ constexpr int kNf4Threads = 256;
 // 7.4 / 8.3 at 688 k; 14.4 / 12.1 at 1.7 M, 26.8 / 23.2 at 3.4 M).
 constexpr int64_t kNf4Wide = 1 << 20;
 
+// Output bytes of 16-bit types from which the stores go past the caches (non-temporal). Below, the GEMM
+// that reads the weight next finds it there: decode + product of 256 rows, plain / non-temporal in us,
+// 32 / 36 at 28 MiB, 60 / 68 at 84, 88 / 96 at 168 MiB (the decode alone 8.7 / 6.5, 21 / 16, 36 / 35). What
+// the 256 MiB Infinity Cache cannot hold is written back all the same: 147 / 118 at 224 MiB (alone
+// 77 / 45), 175 / 146 at 259, 355 / 315 at 518 MiB; at 4096 rows within 2% either way. In fp32 the plain
+// stores are the faster ones at every size (168 MiB 36 / 69, 1036 MiB 311 / 416).
+constexpr int64_t kNf4Stream = int64_t{192} << 20;
+
 // Decode one unit (4 packed bytes, 8 elements, low byte first) with its block's scale into o;
 // tab = the weight's NF4 table (LDS).
-template <typename TO>
+template <typename TO, bool NT>
 __device__ __forceinline__ void nf4_decode(uint32_t raw, float scale, const float* tab,
                                            TO* __restrict__ o) {
 #pragma clang fp contract(off)
@@ -52,7 +55,10 @@ __device__ __forceinline__ void nf4_decode(uint32_t raw, float scale, const floa
     v8t e;
 #pragma unroll
     for (int k = 0; k < 8; ++k) e[k] = Elt<TO>::from_f(v[k]);
-    *reinterpret_cast<v8t*>(o) = e;
+    if constexpr (NT)
+      __builtin_nontemporal_store(__builtin_bit_cast(u32x4, e), reinterpret_cast<u32x4*>(o));
+    else
+      *reinterpret_cast<v8t*>(o) = e;
   } else {
 #pragma unroll
     for (int h = 0; h < 2; ++h)
@@ -83,7 +89,7 @@ __device__ __forceinline__ int64_t nf4_block() {
 // blocks). A block takes U runs of 256 units. While the packed bytes are on their way, one thread per
 // scale block resolves its scale (absmax -> code2 is a dependent pair of loads) into LDS, so the
 // search for the weight and that chain are paid once per 8 units.
-template <typename TO, int U>
+template <typename TO, int U, bool NT>
 __global__ __launch_bounds__(kNf4Threads) void k_nf4_dequant_multi(const Nf4Multi m) {
   constexpr int kScales = kNf4Threads * U / 8;
   __shared__ float tab[kNf4MultiMax][16];
@@ -120,7 +126,7 @@ __global__ __launch_bounds__(kNf4Threads) void k_nf4_dequant_multi(const Nf4Mult
   for (int t = 0; t < U; ++t) {
     const int64_t g = g0 + t * kNf4Threads + tid;
     if (g < total)
-      nf4_decode<TO>(raw[t], scl[(t * kNf4Threads + tid) >> 3], tab[wi[t]],
+      nf4_decode<TO, NT>(raw[t], scl[(t * kNf4Threads + tid) >> 3], tab[wi[t]],
                      static_cast<TO*>(m.w[wi[t]].out) + 8 * (g - m.u0[wi[t]]));
   }
 }
@@ -128,7 +134,7 @@ __global__ __launch_bounds__(kNf4Threads) void k_nf4_dequant_multi(const Nf4Mult
 // One weight: every thread reads its own scales (8 threads the same ones), no wait between them and the
 // packed bytes: 5.2 us at 1536 x 1536 against 5.6 through LDS, 10.7 against 14.4 at 1536 x 8960. Two
 // runs of units per block: four take 10.3 there but 5.8 at 1536 x 1536, one 12.5 and 5.2.
-template <typename TO, int U>
+template <typename TO, int U, bool NT>
 __global__ __launch_bounds__(kNf4Threads) void k_nf4_dequant_one(const Nf4Args w) {
   __shared__ float tab[16];
   const int tid = threadIdx.x;
@@ -149,12 +155,12 @@ __global__ __launch_bounds__(kNf4Threads) void k_nf4_dequant_one(const Nf4Args w
 #pragma unroll
   for (int t = 0; t < U; ++t) {
     const int64_t g = g0 + t * kNf4Threads;
-    if (g < total) nf4_decode<TO>(raw[t], scale[t], tab, static_cast<TO*>(w.out) + 8 * g);
+    if (g < total) nf4_decode<TO, NT>(raw[t], scale[t], tab, static_cast<TO*>(w.out) + 8 * g);
   }
 }
 
-template <typename TO>
-void launch(const Nf4Multi& m, hipStream_t s) {
+template <typename TO, bool NT>
+void launch_nt(const Nf4Multi& m, hipStream_t s) {
   const int64_t units = m.u0[m.n];
   auto grid = [&](int u) {
     const int64_t per = (int64_t)kNf4Threads * u, blocks = (units + per - 1) / per;
@@ -163,11 +169,18 @@ void launch(const Nf4Multi& m, hipStream_t s) {
   };
   const dim3 block(kNf4Threads);
   if (m.n == 1)
-    hipLaunchKernelGGL((k_nf4_dequant_one<TO, 2>), grid(2), block, 0, s, m.w[0]);
+    hipLaunchKernelGGL((k_nf4_dequant_one<TO, 2, NT>), grid(2), block, 0, s, m.w[0]);
   else if (units < kNf4Wide)
-    hipLaunchKernelGGL((k_nf4_dequant_multi<TO, 2>), grid(2), block, 0, s, m);
+    hipLaunchKernelGGL((k_nf4_dequant_multi<TO, 2, NT>), grid(2), block, 0, s, m);
   else
-    hipLaunchKernelGGL((k_nf4_dequant_multi<TO, 4>), grid(4), block, 0, s, m);
+    hipLaunchKernelGGL((k_nf4_dequant_multi<TO, 4, NT>), grid(4), block, 0, s, m);
+}
+
+template <typename TO>
+void launch(const Nf4Multi& m, hipStream_t s) {
+  if constexpr (sizeof(TO) == 2)
+    if (m.u0[m.n] * 16 >= kNf4Stream) return launch_nt<TO, true>(m, s);  // 8 elements per unit
+  launch_nt<TO, false>(m, s);
 }
 
 }  // namespace

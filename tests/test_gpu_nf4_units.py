@@ -89,3 +89,33 @@ def test_more_units_than_one_grid_dimension_holds():
     assert bool((zero == zero[0, 0]).all()) and float(zero[0, 0]) != 0
     del packed, out
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32],
+                         ids=["fp16", "bf16", "fp32"])
+@pytest.mark.parametrize("blocks", [1572863, 1572864, 1572929])
+def test_outputs_past_the_caches(blocks, dtype):
+    """The stores change at 192 MiB of 16-bit output (1572864 scale blocks): the same bits as decoded in
+    pieces, one weight and several, and nothing past the output."""
+    from solution.body import _hip
+
+    g = torch.Generator(device=DEV).manual_seed(blocks)
+    packed = torch.randint(0, 256, (blocks * 32,), generator=g, device=DEV, dtype=torch.uint8)
+    absmax = torch.randint(0, 256, (blocks,), generator=g, device=DEV, dtype=torch.uint8)
+    absmax2 = torch.rand((blocks + 255) // 256, generator=g, device=DEV)
+    _, _, (_, _, _, code2, offset, table), _ = _weight(4, 1, dtype)
+    want = torch.empty(blocks * 64, device=DEV, dtype=dtype)
+    step = 1 << 18  # whole groups of 256 scale blocks
+    for b in range(0, blocks, step):
+        e = min(blocks, b + step)
+        _hip.nf4_dequant(packed[32 * b:32 * e], absmax[b:e], absmax2[b // 256:], code2, offset, table,
+                         want[64 * b:64 * e])
+    for cut in (0, 512 * 1000):
+        out = torch.full((blocks * 64 + 64,), 7.0, device=DEV, dtype=dtype)
+        parts = [(packed[32 * b:32 * e], absmax[b:e], absmax2[b // 256:], code2, offset, table,
+                  out[64 * b:64 * e]) for b, e in ((0, cut), (cut, blocks)) if b < e]
+        if cut:
+            _hip.nf4_dequant_multi(parts)
+        else:
+            _hip.nf4_dequant(*parts[0])
+        assert torch.equal(out[:-64], want) and bool((out[-64:] == 7).all())
