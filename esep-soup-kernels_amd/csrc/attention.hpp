@@ -308,7 +308,7 @@ __device__ __forceinline__ int attn_block() { return (int)(blockIdx.y * gridDim.
 // tile 1, and so on, in the order the hardware dispatches its workgroups; groups stay whole on one
 // XCD as with xcd_order. The kernels number a group's tiles heaviest first (causal: the query tile
 // with the most keys, the key tile with the most queries), so every XCD starts its longest blocks
-// before its short ones. It serves short inputs of more than 64 sequences (level_order the others).
+// before its short ones.
 __device__ __forceinline__ int xcd_order_lpt(int b, int C, int groups) {
   const int xcd = b % 8, slot = b / 8;
   const int per_xcd = (groups + 7) / 8;
@@ -387,8 +387,7 @@ __device__ __forceinline__ int level_order(int b, int nblk, int C, int groups, i
 
 // Block orders of the attention kernels, chosen per launch (attn_order):
 //   kOrderGroups  xcd_order: each XCD runs its groups one after another;
-//   kOrderLpt     grids of a few rounds of residency: level_order, or xcd_order_lpt past 64
-//                 sequences;
+//   kOrderTiles   xcd_order_lpt: each XCD runs its groups tile-major, longest tiles first;
 //   kOrderSorted  the groups (gps per sequence, sequence-major) sorted by their sequence's
 //                 length, longest first, and dealt to the 8 XCDs in snake order (XCD 0..7, then
 //                 7..0, ...): every XCD gets a near-equal share of the work and runs its groups
@@ -396,16 +395,16 @@ __device__ __forceinline__ int level_order(int b, int nblk, int C, int groups, i
 //                 (n_seq <= 64), which keeps a group's K / V (or Q / dO) reads close together in its
 //                 XCD's L2. Dealing groups round-robin in index order instead put a
 //                 sequence's 4 kv-head groups of config 5's dK / dV on XCDs 0-3 or 4-7 by the
-//                 sequence's parity, and the two halves' work differed by 38%.
+//                 sequence's parity, and the two halves' work differed by 38%;
+//   kOrderLevel   level_order: longest blocks first over the whole launch (n_seq <= 64).
 // The result is the block's index in the group-major order (group * C + tile, C tiles of 128 rows);
 // a padding block gets an index past the last group and exits.
-constexpr int kOrderGroups = 0, kOrderLpt = 1, kOrderSorted = 2;
+constexpr int kOrderGroups = 0, kOrderTiles = 1, kOrderSorted = 2, kOrderLevel = 3;
 __device__ __forceinline__ int block_order(int b, int C, int groups, int mode, int gps,
                                            const int32_t* cu, int n_seq, int64_t T) {
   if (mode == kOrderGroups) return xcd_order(b, C);
-  if (mode == kOrderLpt)
-    return n_seq <= 64 ? level_order(b, (int)gridDim.x, C, groups, gps, cu, n_seq, T)
-                       : xcd_order_lpt(b, C, groups);
+  if (mode == kOrderTiles) return xcd_order_lpt(b, C, groups);
+  if (mode == kOrderLevel) return level_order(b, (int)gridDim.x, C, groups, gps, cu, n_seq, T);
   const int xcd = b % 8, slot = b / 8;
   const int j = slot / C, tile = slot % C;
   const int p = 8 * j + ((j & 1) ? 7 - xcd : xcd);  // position in the sorted group list
@@ -414,14 +413,35 @@ __device__ __forceinline__ int block_order(int b, int C, int groups, int mode, i
   return (seq * gps + p % gps) * C + tile;
 }
 
+// Workgroups of a kernel that stay resident on a CU (the launch bounds): at D = 128 three wavefronts
+// per SIMD in the forward and two in dQ (unbounded, the compiler settles at one), at D = 64 four and
+// three; two blocks of dK / dV.
+template <int D>
+constexpr int kFwdPerCU = D == 128 ? 3 : 4;
+template <int D>
+constexpr int kDqPerCU = D == 128 ? 2 : 3;
+constexpr int kDkdvPerCU = 2;
+
 // The order a grid of `blocks` workgroups takes when `per_cu` of them stay resident on each of
-// MI355X's 256 CUs: longest first up to `rounds` rounds of residency (two past 64 sequences).
+// MI355X's 256 CUs.
+//   A block per CU at most: no order matters and the search for a block's place costs 0.3 .. 0.5 us (300
+//   tokens in 4 sequences, 14 / 2 heads, D = 64, forward 4.4 us against 4.8 in level_order).
+//   Up to `rounds` rounds of residency: longest first over the launch, kRoundsQ for the forward and dQ,
+//   kRoundsKV for dK / dV (level_order's figures). At D = 128, sequences of one length (the tokens fill
+//   the bound to 15 / 16) within two rounds: each XCD longest first, which keeps its groups' reads (4 x
+//   16384 tokens, 16 / 2 heads, backward 14.1 -> 13.4 ms; 4 x 8192, 28 / 4 heads 6.26 -> 5.99; 8 x 1024, 12 / 2
+//   heads 156 -> 155 us, forward 40 -> 41); with ragged ones it is 4 .. 10% behind.
+//   More than 64 sequences (the searches hold one per lane): the same within two rounds.
 constexpr int64_t kAttnCUs = 256;
-inline int attn_order(int64_t blocks, int per_cu, int n_seq, int rounds) {
-  if (blocks <= (n_seq <= 64 ? rounds : 2) * kAttnCUs * per_cu) return kOrderLpt;
-  return n_seq <= 64 ? kOrderSorted : kOrderGroups;
+constexpr int kRoundsQ = 4, kRoundsKV = 16;
+inline int attn_order(int64_t blocks, int per_cu, int rounds, int D, int64_t T, int n_seq,
+                      int max_seqlen) {
+  const bool two = blocks <= 2 * kAttnCUs * per_cu;
+  if (blocks <= kAttnCUs) return kOrderGroups;
+  if (n_seq > 64) return two ? kOrderTiles : kOrderGroups;
+  if (D == 128 && two && 16 * T >= (int64_t)15 * n_seq * max_seqlen) return kOrderTiles;
+  return blocks <= rounds * kAttnCUs * per_cu ? kOrderLevel : kOrderSorted;
 }
-constexpr int kRoundsQ = 4, kRoundsKV = 16;  // forward and dQ; dK / dV (level_order's figures)
 
 // A [ROWS x D] tile (token rows r0 .. r0 + ROWS - 1 below rend; the rest reads as 0) moved
 // through registers into a swizzled LDS tile. load() issues every global read of the thread

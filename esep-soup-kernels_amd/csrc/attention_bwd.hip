@@ -99,12 +99,6 @@ __device__ __forceinline__ void dq_tile_swz(const char* ks, const char* vs, int 
   __builtin_amdgcn_s_setprio(0);
 }
 
-// Blocks of 4 wavefronts resident per CU (launch bounds): at D = 128 two wavefronts per SIMD
-// (unbounded, the compiler settles at one), at D = 64 three.
-template <int D>
-constexpr int kDqPerCU = D == 128 ? 2 : 3;
-constexpr int kDkdvPerCU = 2;
-
 // dQ with the K / V tiles moved as the forward moves them: swizzled BN-key tiles filled by dwordx4
 // LDS DMA through a ring of two buffers (tile t + 1 in flight while tile t is consumed, one
 // barrier per tile). At D = 64 (the dK / dV kernel's sizes below) 78 us, against 133 staged through
@@ -468,22 +462,24 @@ hipError_t bwd_run(const AttnBwdArgs& b, int max_seqlen, hipStream_t s) {
   // 4 wavefronts (128 queries) per dQ block: 8 measured slower (with 256 causal queries per
   // block the early wavefronts idle through the later key tiles).
   constexpr int QW = 4;
-  const dim3 gq((max_seqlen + 32 * QW - 1) / (32 * QW), b.f.HQ, b.f.n_seq);
-  const int64_t nq = xcd_grid(gq.x, (int64_t)gq.y * gq.z);
+  const AttnArgs& f = b.f;
+  const int64_t C = (max_seqlen + 32 * QW - 1) / (32 * QW);
+  const int64_t nq = xcd_grid(C, (int64_t)f.HQ * f.n_seq);
   if (!attn_grid_ok(nq)) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((k_attn_bwd_dq_dma<T, D, D == 128 ? 32 : 64, QW>), attn_grid(nq),
-                     dim3(64 * QW), 0, s, b, (int)gq.x, attn_order(nq, kDqPerCU<D>, b.f.n_seq, kRoundsQ));
+  hipLaunchKernelGGL((k_attn_bwd_dq_dma<T, D, D == 128 ? 32 : 64, QW>), attn_grid(nq), dim3(64 * QW),
+                     0, s, b, (int)C,
+                     attn_order(nq, kDqPerCU<D>, kRoundsQ, D, f.T, f.n_seq, max_seqlen));
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   constexpr int NW = 4, BQ = 32;
-  const int64_t ktiles = (max_seqlen + 32 * NW - 1) / (32 * NW);
-  const int64_t nk = xcd_grid(ktiles, (int64_t)b.f.HK * b.split * b.f.n_seq);
+  static_assert(NW == QW, "C counts the key tiles too");
+  const int64_t nk = xcd_grid(C, (int64_t)f.HK * b.split * f.n_seq);
   if (!attn_grid_ok(nk)) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((k_attn_bwd_dkdv<T, D, NW, BQ>), attn_grid(nk), dim3(64 * NW), 0, s, b,
-                     (int)ktiles, attn_order(nk, kDkdvPerCU, b.f.n_seq, kRoundsKV));
+  hipLaunchKernelGGL((k_attn_bwd_dkdv<T, D, NW, BQ>), attn_grid(nk), dim3(64 * NW), 0, s, b, (int)C,
+                     attn_order(nk, kDkdvPerCU, kRoundsKV, D, f.T, f.n_seq, max_seqlen));
   e = hipGetLastError();
   if (e != hipSuccess || b.split == 1) return e;
-  const int64_t quads = b.f.T * b.f.HK * D / 4;
+  const int64_t quads = f.T * f.HK * D / 4;
   hipLaunchKernelGGL((k_attn_dkdv_reduce<T>), dim3((unsigned)((quads + 255) / 256)), dim3(256), 0,
                      s, b, D);
   return hipGetLastError();

@@ -98,11 +98,6 @@ __device__ __forceinline__ void fwd_tile_swz(const char* ks, const char* vs, int
   __builtin_amdgcn_s_setprio(0);
 }
 
-// Blocks resident per CU (the kernel's launch bound): three of D = 128's wavefronts per SIMD, four
-// of D = 64's.
-template <int D>
-constexpr int kFwdPerCU = D == 128 ? 3 : 4;
-
 // The forward kernel: blocks of 4 wavefronts own 128 queries of one (sequence, query head) with the
 // online softmax in registers; the BN-key K / V tiles go through a ring of NBUF = 2 swizzled LDS
 // buffers filled by LDS DMA (tile t + 1 in flight while tile t is consumed, one barrier per tile
@@ -205,19 +200,20 @@ __global__ __launch_bounds__(kAttnThreads, kFwdPerCU<D>) void k_attn_fwd_swz(con
 }
 
 template <typename T, int D, int BN>
-hipError_t fwd_run(const AttnArgs& a, dim3 grid, hipStream_t s) {
-  const int64_t n = xcd_grid(grid.x, (int64_t)grid.y * grid.z);
+hipError_t fwd_run(const AttnArgs& a, int max_seqlen, hipStream_t s) {
+  const int64_t C = (max_seqlen + kAttnBM - 1) / kAttnBM;
+  const int64_t n = xcd_grid(C, (int64_t)a.HQ * a.n_seq);
   if (!attn_grid_ok(n)) return hipErrorInvalidValue;
   hipLaunchKernelGGL((k_attn_fwd_swz<T, D, BN, 2>), attn_grid(n), dim3(kAttnThreads), 0, s, a,
-                     (int)grid.x, attn_order(n, kFwdPerCU<D>, a.n_seq, kRoundsQ));
+                     (int)C, attn_order(n, kFwdPerCU<D>, kRoundsQ, D, a.T, a.n_seq, max_seqlen));
   return hipGetLastError();
 }
 
 template <typename T>
-hipError_t fwd_d(const AttnArgs& a, int D, dim3 grid, hipStream_t s, bool* sup) {
+hipError_t fwd_d(const AttnArgs& a, int D, int max_seqlen, hipStream_t s, bool* sup) {
   *sup = true;
-  if (D == 128) return fwd_run<T, 128, 32>(a, grid, s);
-  if (D == 64) return fwd_run<T, 64, 64>(a, grid, s);
+  if (D == 128) return fwd_run<T, 128, 32>(a, max_seqlen, s);
+  if (D == 64) return fwd_run<T, 64, 64>(a, max_seqlen, s);
   *sup = false;
   return hipErrorInvalidValue;
 }
@@ -226,9 +222,8 @@ hipError_t fwd_d(const AttnArgs& a, int D, dim3 grid, hipStream_t s, bool* sup) 
 
 hipError_t launch_attn_fwd(const AttnArgs& a, int dt, int D, int max_seqlen, hipStream_t s,
                            bool* sup) {
-  const dim3 grid((max_seqlen + kAttnBM - 1) / kAttnBM, a.HQ, a.n_seq);
-  if (dt == 1) return fwd_d<_Float16>(a, D, grid, s, sup);
-  if (dt == 2) return fwd_d<__bf16>(a, D, grid, s, sup);
+  if (dt == 1) return fwd_d<_Float16>(a, D, max_seqlen, s, sup);
+  if (dt == 2) return fwd_d<__bf16>(a, D, max_seqlen, s, sup);
   *sup = false;
   return hipErrorInvalidValue;
 }

@@ -525,7 +525,7 @@ int esep_rope(const void* q, const int64_t q_strides[3], const void* q_delta,
 
 // Token strides of the attention tensors, in elements, at most 2^22 (8 MiB of 16-bit
 // elements): the LDS-DMA tile fills address a wavefront's rows with 32-bit per-lane byte
-// offsets of up to 20 strides from an SGPR base.
+// offsets of up to 39 strides from an SGPR base (64-key tiles: row groups 32 rows apart, 8 rows each).
 constexpr int64_t kAttnMaxStride = int64_t{1} << 22;
 
 int esep_attn_fwd(const void* q, int64_t q_rs, const void* k, int64_t k_rs, const void* v,
@@ -574,6 +574,22 @@ int esep_attn_fwd(const void* q, int64_t q_rs, const void* k, int64_t k_rs, cons
   const hipError_t e = esep::launch_attn_fwd(a, dt, D, max_seqlen, static_cast<hipStream_t>(stream), &sup);
   if (!sup) return fail(ESEP_EINVAL, "attn_fwd: unsupported dtype / D");
   return e == hipSuccess ? 0 : hip_fail(e, "attn_fwd launch");
+}
+
+int esep_attn_orders(int64_t T, int HQ, int HK, int D, int n_seq, int max_seqlen) {
+  g_err[0] = 0;
+  if ((D != 64 && D != 128) || T < 1 || T > 0x7fffffff || HQ < 1 || HK < 1 || HQ % HK != 0 ||
+      n_seq < 1 || max_seqlen < 1)
+    return fail(ESEP_ESHAPE, "attn_orders: bad sizes T=%lld HQ=%d HK=%d D=%d n_seq=%d max_seqlen=%d",
+                (long long)T, HQ, HK, D, n_seq, max_seqlen);
+  const int64_t C = (max_seqlen + esep::kAttnBM - 1) / esep::kAttnBM;
+  auto order = [&](int64_t heads, int per_cu, int rounds) {
+    return esep::attn_order(esep::xcd_grid(C, heads * n_seq), per_cu, rounds, D, T, n_seq, max_seqlen);
+  };
+  const int64_t hs = (int64_t)HK * attn_split(T, HQ, HK);
+  return order(HQ, D == 128 ? esep::kFwdPerCU<128> : esep::kFwdPerCU<64>, esep::kRoundsQ) |
+         order(HQ, D == 128 ? esep::kDqPerCU<128> : esep::kDqPerCU<64>, esep::kRoundsQ) << 4 |
+         order(hs, esep::kDkdvPerCU, esep::kRoundsKV) << 8;
 }
 
 int64_t esep_attn_bwd_workspace(int64_t T, int HQ, int HK, int D) {

@@ -50,6 +50,7 @@ SIGNATURES = {
     "esep_attn_fwd": (_i32, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i32, _i64, _i32,
                              _i32, _i32, _vp, _i32, _i32, _f32, _vp]),
     "esep_attn_bwd_workspace": (_i64, [_i64, _i32, _i32, _i32]),
+    "esep_attn_orders": (_i32, [_i64, _i32, _i32, _i32, _i32, _i32]),
     "esep_swiglu_fwd": (_i32, [_vp, _vp, _vp, _i64, _i32, _vp]),
     "esep_lora_dropout_fwd": (_i32, [_vp, _vp, _vp, _i64, _f32, _i32, _vp]),
     "esep_nf4_dequant": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i64, _vp]),

@@ -244,6 +244,13 @@ int esep_attn_fwd(const void* q, int64_t q_rs, const void* k, int64_t k_rs, cons
 int64_t esep_attn_bwd_workspace(int64_t T, int HQ, int HK, int D);
 
 /*
+ * The block orders that esep_attn_fwd and esep_attn_bwd take for this shape, for tests and traces:
+ * forward | dQ << 4 | dK / dV << 8, each 0 (groups one after another), 1 (tile-major per XCD), 2 (sorted
+ * by length) or 3 (longest blocks first). Results do not depend on them. ESEP_ESHAPE for bad sizes.
+ */
+int esep_attn_orders(int64_t T, int HQ, int HK, int D, int n_seq, int max_seqlen);
+
+/*
  * Backward of esep_attn_fwd (same layout and argument meanings), deterministic (no atomics).
  * Replaces the autograd backward of the reference's per-row SDPA calls (packed.py:428-429).
  *

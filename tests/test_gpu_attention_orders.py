@@ -30,16 +30,61 @@ def _run(ins, lens, bound):
     return o, lse, dq, dk, dv
 
 
+GROUPS, TILES, SORTED, LEVEL = range(4)
+RAGGED, ALIKE = [129, 1, 0, 700, 257], [300 + i for i in range(16)]
+MANY = [100 + 37 * i % 200 for i in range(70)]
+# lens, heads, then per bound the expected orders of (forward, dQ, dK / dV) at D = 64 and at D = 128: a block
+# per CU at most; a few rounds of blocks; more rounds than the forward and dQ, then than dK / dV take
+# longest first; several reversed runs of 256 blocks; sequences of one length; past 64 sequences
+CASES = [
+    (RAGGED, 4, 2, {700: ((GROUPS,) * 3, (GROUPS,) * 3), 5000: ((LEVEL,) * 3, (LEVEL,) * 3),
+                    30000: ((SORTED, SORTED, LEVEL),) * 2, 50000: ((SORTED,) * 3,) * 2}),
+    (ALIKE, 12, 12, {315: ((LEVEL,) * 3, (TILES,) * 3), 400: ((LEVEL,) * 3,) * 2,
+                     3000: ((SORTED, SORTED, LEVEL),) * 2}),
+    (MANY, 4, 4, {299: ((TILES,) * 3,) * 2, 4000: ((GROUPS,) * 3,) * 2}),
+]
+
+
+def _orders(lens, hq, hk, D, bound):
+    from solution.body import _hip
+
+    code = _hip.lib().esep_attn_orders(sum(lens), hq, hk, D, len(lens), bound)
+    assert code >= 0
+    return code & 15, code >> 4 & 15, code >> 8
+
+
 @pytest.mark.parametrize("D", [64, 128])
-@pytest.mark.parametrize("lens,bounds", [([100], (128, 4097, 65536)),
-                                         ([129, 1, 0, 700, 257], (700, 1000, 5000)),
-                                         ([200] * 12, (200, 1024, 8192))])
-def test_any_bound_gives_the_same_bits(lens, bounds, D):
-    ins = _inputs(sum(lens), 4, 2, D)
-    want = _run(ins, lens, max(lens))
-    for bound in bounds:
-        for a, b in zip(_run(ins, lens, bound), want):
+@pytest.mark.parametrize("lens,hq,hk,bounds", CASES, ids=["ragged", "alike", "many"])
+def test_every_order_gives_the_same_bits(lens, hq, hk, bounds, D):
+    ins, want = _inputs(sum(lens), hq, hk, D), None
+    for bound, orders in bounds.items():
+        assert _orders(lens, hq, hk, D, bound) == orders[D == 128], bound
+        got = _run(ins, lens, bound)
+        want = want or got
+        for a, b in zip(got, want):
             assert torch.equal(a, b), bound
+    # and against each sequence on its own (the forward and dQ; dK / dV's sums are split by the shape)
+    t0 = 0
+    for n in lens[:6]:
+        one = [t[t0:t0 + n].contiguous() for t in ins]
+        if n:
+            o, _, dq, _, _ = _run(one, [n], n)
+            assert torch.equal(o, want[0][t0:t0 + n]) and torch.equal(dq, want[2][t0:t0 + n])
+        t0 += n
+
+
+@pytest.mark.parametrize("D,order", [(64, LEVEL), (128, TILES)])
+def test_sequences_past_the_bound(D, order):
+    """A bound below the longest sequence (not a supported call, but in bounds): the grid holds two
+    tiles per sequence, the last ones of the forward and dQ, and nothing else is written."""
+    lens = [700] * 12
+    ins = _inputs(sum(lens), 16, 16, D)
+    assert _orders(lens, 16, 16, D, 256)[:2] == (order, order)
+    want, got = _run(ins, lens, 700), _run(ins, lens, 256)
+    for i in (0, 2):  # o, dq: query tiles 4 and 5 of 6
+        for t0 in range(0, sum(lens), 700):
+            assert torch.equal(got[i][t0 + 512:t0 + 700], want[i][t0 + 512:t0 + 700])
+            assert not bool(got[i][t0:t0 + 512].any())
 
 
 @pytest.mark.parametrize("D", [64, 128])
