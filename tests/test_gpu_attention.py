@@ -159,11 +159,13 @@ def test_attn_bwd_long_sequences_sampled_keys(lengths):
     K_j over the causal keys). The ragged lengths put the end of every sequence inside a query
     tile (rows past the end staged and masked); the sample takes keys from the last 40 tokens of
     each sequence as well as from anywhere. These grids are too large for the longest-first
-    block order, so the forward and dQ kernels (and, with 9 sequences, the dK / dV kernel) run
-    the length-sorted XCD order (kOrderSorted), equal-length sequences ranked by index."""
+    block order in the forward and dQ kernels, which run the length-sorted XCD order
+    (kOrderSorted, equal-length sequences ranked by index), but not in the dK / dV kernel
+    (kOrderLevel)."""
     from solution.body import _hip
 
     HQ, HK, D = 28, 4, 128
+    assert _hip.lib().esep_attn_orders(sum(lengths), HQ, HK, D, len(lengths), max(lengths)) == 0x322
     q, k, v, cu = _inputs(lengths, HQ, HK, D, torch.bfloat16, seed=31)
     T = q.shape[0]
     assert ((T + 255) // 256) * HK >= 256  # no split: the 4-wavefront kernel
@@ -220,7 +222,7 @@ def test_attn_bwd_long_sequences_sampled_keys(lengths):
 @pytest.mark.parametrize("n_seq", [60, 70], ids=["sorted_order", "group_order"])
 def test_attn_many_sequences_block_orders(n_seq):
     """Many packed sequences (lengths 0 .. 640 with empty ones, 28 / 4 heads, D = 128): grids past
-    two rounds of residency, so the kernels run the length-sorted XCD order (kOrderSorted: up to
+    the rounds of the longest-first orders, so the kernels run the length-sorted XCD order (kOrderSorted: up to
     64 sequences, ranked by length with ties and empty sequences) or, past 64 sequences, the
     group-by-group order. Output and gradients against torch's SDPA computed in float32 from the
     same bf16 inputs, within 1e-2 of the largest magnitude plus 1e-2 relative."""
@@ -231,6 +233,8 @@ def test_attn_many_sequences_block_orders(n_seq):
     lengths[3] = lengths[17] = 0
     lengths[5] = lengths[30] = 640
     HQ, HK, D = 28, 4, 128
+    orders = _hip.lib().esep_attn_orders(sum(lengths), HQ, HK, D, n_seq, max(lengths))
+    assert orders == (0x222 if n_seq <= 64 else 0)
     q, k, v, cu = _inputs(lengths, HQ, HK, D, torch.bfloat16, seed=50 + n_seq)
     do = torch.randn(q.shape, generator=gen(60 + n_seq)).to(torch.bfloat16).to(DEV)
     T, scale, L = q.shape[0], D ** -0.5, max(lengths)
@@ -255,7 +259,7 @@ def test_attn_many_sequences_block_orders(n_seq):
 
 def test_attn_config4_shape():
     """Config 4's attention as bench.py times it: 8 rows of 1024 tokens, 12 / 2 heads, D = 128,
-    bf16 (a grid of one residency round: the longest-first block order; the dK / dV kernel with
+    bf16 (equal rows within two residency rounds: the tile-major block order; the dK / dV kernel with
     the query heads of a kv head split six ways and the partials' reduce). Output and gradients
     against torch's SDPA in float32 from the same bf16 inputs, within 1e-2 of the largest
     magnitude plus 1e-2 relative."""
