@@ -843,6 +843,15 @@ int esep_gemm_pays(int64_t M, int64_t N, int64_t K, int b_kn) {
   return gemm_sizes_ok(M, N, K) && esep::gemm_pays(M, N, K, b_kn != 0) ? 1 : 0;
 }
 
+int esep_gemm_plan(int64_t M, int64_t N, int64_t K) {
+  g_err[0] = 0;
+  if (!gemm_sizes_ok(M, N, K))
+    return fail(ESEP_ESHAPE, "gemm_plan: bad sizes %lld x %lld x %lld", (long long)M, (long long)N,
+                (long long)K);
+  const esep::GemmPlan p = esep::gemm_plan(M, N, K);
+  return p.shape | p.splits << 4;
+}
+
 int64_t esep_gemm_workspace(int64_t M, int64_t N, int64_t K) {
   if (!gemm_sizes_ok(M, N, K)) return 0;
   const esep::GemmPlan p = esep::gemm_plan(M, N, K);

@@ -147,14 +147,10 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm(const GemmArgs g) {
   uint32_t bro = 0, bto[2] = {0, 0};
   if constexpr (KN) {
     const int k = (lane >> 2) & 3, m = lane & 3, G1 = (lane >> 4) & 1;
+    static_assert(TN % 2 == 0, "two 32-column operands per 64-byte swizzle period");
 #pragma unroll
     for (int u = 0; u < 2; ++u)
-      bto[u] = (uint32_t)((8 * hi + k) * 2 * S::BN + 64 * TN * wn + 8 * m) +
-               (TN % 2 == 0 ? 32u * ((2 * u + G1) ^ k) : 0u);
-    if constexpr (TN == 1) {
-      const int u = 2 * wn + G1;
-      bto[0] = (uint32_t)((8 * hi + k) * 2 * S::BN + 8 * m) + 32u * (u ^ k);
-    }
+      bto[u] = (uint32_t)((8 * hi + k) * 2 * S::BN + 64 * TN * wn + 8 * m) + 32u * ((2 * u + G1) ^ k);
   } else {
     bro = (uint32_t)((32 * TN * wn + lq) * 128) + sw;
   }

@@ -71,6 +71,7 @@ SIGNATURES = {
     "esep_head_dx": (_i32, [_vp, _i64, _vp, _vp, _vp, _f32, _vp, _i32, _i64, _i64, _vp]),
     "esep_gemm_pays": (_i32, [_i64, _i64, _i64, _i32]),
     "esep_gemm_workspace": (_i64, [_i64, _i64, _i64]),
+    "esep_gemm_plan": (_i32, [_i64, _i64, _i64]),
     "esep_gemm": (_i32, [_vp, _i64, _vp, _i64, _i32, _vp, _vp, _i64, _i32, _vp, _i64, _i64, _i64,
                          _i32, _vp]),
     "esep_swiglu_bwd": (_i32, [_vp, _vp, _vp, _vp, _vp, _i64, _i32, _vp]),

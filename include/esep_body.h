@@ -341,9 +341,13 @@ int esep_lora_grads(const void* x, const void* a, const void* dxa, const int64_t
  * Deterministic (no atomics).
  *   esep_gemm_pays        1 where this product is expected to beat the vendor BLAS, else 0
  *   esep_gemm_workspace   fp32 elements (0 for most sizes)
+ *   esep_gemm_plan        the launch for a size, for tests and traces: the output tile of a block (0 256 x
+ *                         256, 1 128 x 256, 2 256 x 128, 3 128 x 128, 4 64 x 128) | the splits of the
+ *                         contraction << 4; ESEP_ESHAPE for a size that esep_gemm does not take
  */
 int esep_gemm_pays(int64_t M, int64_t N, int64_t K, int b_kn);
 int64_t esep_gemm_workspace(int64_t M, int64_t N, int64_t K);
+int esep_gemm_plan(int64_t M, int64_t N, int64_t K);
 int esep_gemm(const void* a, int64_t lda, const void* b, int64_t ldb, int b_kn, const void* bias,
               void* c, int64_t ldc, int c_dt, float* workspace, int64_t M, int64_t N, int64_t K,
               int dt, void* stream);

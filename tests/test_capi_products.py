@@ -80,6 +80,7 @@ def test_gemm_plan_bounds():
                     if lib.esep_gemm_pays(M, N, K, kn):
                         assert K >= 896, (M, N, K)
     assert lib.esep_gemm_pays(1031, 1536, 17920, 1) == 1  # few tiles, long contraction
+    assert lib.esep_gemm_plan(1031, 1536, 17950) == ESHAPE and lib.esep_gemm_plan(1, 8, 64) == 4 | 1 << 4
     assert lib.esep_gemm_pays(1031, 1536, 17950, 1) == 0 and lib.esep_gemm_workspace(4, 60, 64) == 0
     assert lib.esep_lora_grads_workspace(0, 64, 64, 8) == 0
     assert lib.esep_lora_grads_workspace(100, 64, 128, 16) % (16 * (64 + 128)) == 0

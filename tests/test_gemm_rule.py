@@ -1,4 +1,5 @@
-"""Which products esep_gemm takes from the vendor BLAS (esep_gemm_pays), on the CPU: the ranges where it
+"""Which products esep_gemm takes from the vendor BLAS (esep_gemm_pays) and how it launches them, on the
+CPU: the ranges where it
 measured faster, and not the ones around them (microseconds of the library / of the kernel on an
 MI355X, operands warm, fp16; the rule's own comment in csrc/gemm.hip has the whole table)."""
 
@@ -26,3 +27,12 @@ MEASURED = [
 @pytest.mark.parametrize("M,N,K,b_kn,library,here", MEASURED)
 def test_the_faster_one_is_taken(M, N, K, b_kn, library, here):
     assert _hip.lib().esep_gemm_pays(M, N, K, b_kn) == int(here < library)
+
+
+def test_the_gpu_tests_cover_the_plans():
+    """The sizes of test_gpu_gemm.py reach every tile shape, with one split of the contraction and with
+    several (the plan's prices decide, so a retuned figure could drop one)."""
+    from test_gpu_gemm import SIZES
+
+    plans = [_hip.lib().esep_gemm_plan(*size) for size in SIZES]
+    assert {(p & 15, p >> 4 > 1) for p in plans} == {(s, m) for s in range(5) for m in (False, True)}

@@ -14,12 +14,13 @@ pytestmark = pytest.mark.gpu
 
 U = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float32: 0.0}
 
-# (M, N, K): one row and one 8-column chunk, one contraction step; ragged 64 x 128 tiles; ragged
-# 128 x 128 tiles with and without splits; many splits of few rows; 256-row tiles (several rounds, a
-# ragged last tile, an odd number of steps) and their splits; 128 x 256 and 256 x 128 tiles
+# (M, N, K): one row and one 8-column chunk, one contraction step; ragged tiles of every shape with and
+# without splits of the contraction (several rounds, a ragged last tile, an odd number of steps, many
+# splits of few rows)
 SIZES = [(1, 8, 64), (65, 264, 704), (130, 136, 128), (16, 1536, 17920), (40, 1096, 4096),
          (1031, 896, 9728), (2300, 8960, 256), (3001, 8960, 192), (1031, 1536, 17920),
-         (1285, 1544, 4160), (4096, 1544, 1088), (260, 8200, 1024)]
+         (1285, 1544, 4160), (4096, 1544, 1088), (260, 8200, 1024), (8254, 888, 192),
+         (1203, 888, 9728), (1750, 896, 4864)]
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
