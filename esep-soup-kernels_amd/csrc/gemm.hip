@@ -399,13 +399,15 @@ GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K) {
 //     2049 ..       none             0.64 .. 1.30 without a pattern
 //     1281 ..       t = 52 .. 72     0.89, 1.05 (3001 x 1536 x 1536 29 us / 24) | 1.04 .. 1.37 on either side
 //     896 ..        t = 12 .. 64     0.82, 1.07 | up to 1.56 below, 1.26 above
+//     up to 2048    t >= 250, M <= 4096, where the plan is whole 256 x 256 tiles: 0.97, 1.00 (3001 x 8960 x 1536 87
+//                   us / 83) | the smaller tiles 0.80 .. 1.16 (3750 x 8960 x 1536 109 / 119)
 //   B [N, K], which the library serves better
 //     K >= 16384    t = 1 .. 95      0.56, 1.06
 //     12288 ..      t = 4 .. 40      0.86, 1.05 | 1.1 .. 1.4
 //     8192 ..       t = 4 .. 20      0.85, 1.06 | 1.05 .. 1.4
 //     896 ..        the LM head's logits up to 32 rows 0.79, 0.98, and at 385 .. 512 (two full 256-row tiles)
 //                   0.91, 0.98 | 300 rows 185 us / 240; 4096 x 256 x 1536 9 / 22, 512 x 2048 x 1536 9 / 18
-// Of the 995 measured products that it takes, 11 are more than 5% slower here.
+// Of the 1030 measured products that it takes, 11 are more than 5% slower here.
 bool gemm_pays(int64_t M, int64_t N, int64_t K, bool b_kn) {
   const double t = (double)M * N / 65536;
   if (b_kn) {
@@ -413,9 +415,12 @@ bool gemm_pays(int64_t M, int64_t N, int64_t K, bool b_kn) {
     if (K >= 12288) return t <= 75;
     if (K >= 8192) return t <= 48 || (t >= 64 && t <= 80);
     if (K >= 3328) return t >= 1 && t <= 36;
-    if (K > 2048) return false;
-    if (K > 1280) return t >= 52 && t < 72;
-    return K >= 896 && t >= 12 && t <= 64;  // below 896 not measured
+    if (K > 2048 || K < 896) return false;  // below 896 not measured
+    if (t >= 250 && M <= 4096) {
+      const GemmPlan p = gemm_plan(M, N, K);
+      return p.shape == kGemm256x256 && p.splits == 1;
+    }
+    return K > 1280 ? t >= 52 && t < 72 : t >= 12 && t <= 64;
   }
   if (K >= 16384) return t >= 1 && t < 96;
   if (K >= 12288) return t >= 4 && t <= 40;

@@ -1,7 +1,6 @@
 """Which products esep_gemm takes from the vendor BLAS (esep_gemm_pays) and how it launches them, on the
-CPU: the ranges where it
-measured faster, and not the ones around them (microseconds of the library / of the kernel on an
-MI355X, operands warm, fp16; the rule's own comment in csrc/gemm.hip has the whole table)."""
+CPU: the ranges where it measured faster, and not the ones around them (microseconds of the library / of
+the kernel on an MI355X, operands warm, fp16; the rule's comment in csrc/gemm.hip has the whole table)."""
 
 import pytest
 
@@ -19,6 +18,7 @@ MEASURED = [
     (1031, 1536, 17920, 1, 199.4, 73.7), (16, 1536, 151936, 1, 288.2, 113.4), (3750, 1536, 151936, 1, 2496.1, 1717.0),
     (1031, 1536, 8960, 1, 63.3, 53.0), (3001, 1536, 8960, 1, 95.8, 89.4), (1285, 896, 9728, 1, 73.5, 41.8),
     (128, 3584, 3584, 1, 27.7, 16.4), (1500, 896, 4864, 1, 39.7, 27.2), (3001, 1536, 1536, 1, 29.4, 24.1),
+    (3750, 8960, 1536, 1, 108.8, 119.4), (3001, 8960, 1536, 1, 86.5, 82.8), (4096, 11008, 2048, 1, 174.4, 168.2),
     (1500, 896, 896, 1, 12.0, 8.1), (400, 3584, 18944, 0, 167.0, 72.0), (400, 1536, 8960, 0, 33.7, 26.2),
     (400, 151936, 1536, 0, 254.7, 231.3), (16, 151936, 1536, 0, 160.5, 90.3),
 ]
