@@ -75,6 +75,12 @@ def _fused(rank, *mats):
     return True
 
 
+def _number(scaling):
+    """The kernels take the scaling as a number; a tensor (which may be on the graph, or one value per
+    column) is torch's to multiply by."""
+    return isinstance(scaling, (int, float))
+
+
 # Where each fused product is the faster one, by rows, width (the long side) and rank, against the
 # library's products and the dropout kernels around them: measured on an MI355X for 16 .. 40000 rows,
 # widths 64 .. 18944 and ranks 8, 16, 32, 64 in fp16 and bf16 (alike), kernel time of launches back to
@@ -209,8 +215,8 @@ def lora_down_bwd(x, a16, dxa, key, p, need_dx=True, dx_accum=None):
 
 def lora_delta(xa, b16, scaling):
     """The term scaling * xa @ B^T on its own."""
-    if (not _hip.recorded(xa, b16) and _fused(b16.shape[1], xa, b16) and xa.is_contiguous()
-            and b16.is_contiguous() and b16.shape[0] % 8 == 0):
+    if (_number(scaling) and not _hip.recorded(xa, b16) and _fused(b16.shape[1], xa, b16)
+            and xa.is_contiguous() and b16.is_contiguous() and b16.shape[0] % 8 == 0):
         term = torch.empty((xa.shape[0], b16.shape[0]), device=xa.device, dtype=xa.dtype)
         _hip.lora_up(xa, b16, term, scaling)
         return term
@@ -220,7 +226,8 @@ def lora_delta(xa, b16, scaling):
 
 def lora_up_bwd(dout, xa, b16, scaling):
     """(dxa [T, r], dB fp32 [out, r]) for the term's gradient dout."""
-    fused = not _hip.recorded(dout, xa, b16) and _up_bwd_fused(dout, xa, b16)
+    fused = (_number(scaling) and not _hip.recorded(dout, xa, b16)
+             and _up_bwd_fused(dout, xa, b16))
     if fused and _up_grads_pay(*dout.shape, b16.shape[1]):
         db = torch.empty(b16.shape, device=dout.device, dtype=torch.float32)
         _hip.lora_grads(dterm=dout, xa=xa, scale=scaling, db=db)
@@ -256,7 +263,7 @@ class _LoRATerm:
         a16, b16 = cast_lora_weights(weight_a, weight_b, dtype)
         key = new_dropout_key(x2.device) if p > 0.0 else None
         ctx.fused = (_fused(a16.shape[0], x2, a16, b16) and a16.is_contiguous()
-                     and b16.is_contiguous() and b16.shape[0] % 8 == 0)
+                     and b16.is_contiguous() and b16.shape[0] % 8 == 0 and _number(scaling))
         xa = _xa(x2, a16, key, p, True) if ctx.fused else lora_down_fwd(x2, a16, key, p)
         ctx.save_for_backward(x2, xa, a16, b16, key)
         ctx.p, ctx.scaling, ctx.dtype = p, scaling, dtype

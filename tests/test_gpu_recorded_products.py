@@ -92,6 +92,23 @@ def test_graph_of_the_dropped_product():
     _same(da, want)
 
 
+def test_scaling_given_as_a_tensor():
+    """A scaling on the graph gets its gradient, and one value per column is taken."""
+    from solution.body import lora as L
+
+    xa, b, d = _rnd(T, R), _rnd(N, R), _rnd(T, N)
+    scale = torch.tensor(S, device=DEV, requires_grad=True)
+    out = L.lora_delta(xa, b, scale)
+    _same(out.detach(), _ref_delta(xa, b))
+    (ds,) = torch.autograd.grad(out, scale, d)
+    torch.testing.assert_close(ds, ((xa @ b.t()).float() * d.float()).sum(), rtol=2e-2, atol=2.0)
+    columns = torch.rand(N, device=DEV).half()
+    _same(L.lora_delta(xa, b, columns), (xa @ b.t()) * columns)
+    _same(L.lora_up_bwd(d, xa, b, torch.tensor(S, device=DEV)), _ref_up_bwd(d, xa, b))
+    term = L.LoRADeltaFunction.apply(_rnd(T, K), _rnd(R, K), b, 0.0, torch.tensor(S, device=DEV))
+    _same(term, S * ((_rnd(T, K) @ _rnd(R, K).t()) @ b.t()))
+
+
 @pytest.mark.parametrize("name,which,out", [("up_bwd", 2, 0), ("down_bwd", 1, 0)])
 def test_graph_of_the_backward_products(name, which, out):
     """Their 16-bit results are differentiable in every operand, not in the incoming gradient alone."""
