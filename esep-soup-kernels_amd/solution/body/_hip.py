@@ -187,15 +187,22 @@ def _stream(dev):
 
 _functorch_wrapped = torch._C._functorch.is_functorch_wrapped_tensor
 _batched = torch._C._functorch.is_legacy_batchedtensor
+_trace, _dispatch_modes = torch._C._get_tracing_state, torch._C._len_torch_dispatch_stack
+_PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
 
 
 def recorded(*tensors):
     """Torch has to see the operations on these tensors as its own (a kernel would fill a buffer behind
     its back): one requires grad in grad mode, carries a forward-mode tangent, or is a functorch
-    wrapper (vmap, batched gradients, torch.func), which has no memory of its own."""
+    wrapper (vmap, batched gradients, torch.func), which has no memory of its own; one is of a
+    subclass (fake and distributed tensors have no memory either), or a trace, a compiler or a
+    dispatch mode looks on."""
+    if torch.compiler.is_compiling() or _trace() is not None or _dispatch_modes():
+        return True
     grad, dual = torch.is_grad_enabled(), forward_ad._current_level >= 0
     for t in tensors:
-        if t is not None and ((grad and t.requires_grad) or _functorch_wrapped(t) or _batched(t)
+        if t is not None and (type(t) not in _PLAIN_TYPES or (grad and t.requires_grad)
+                              or _functorch_wrapped(t) or _batched(t)
                               or (dual and forward_ad.unpack_dual(t).tangent is not None)):
             return True
     return False

@@ -262,8 +262,9 @@ class _LoRATerm:
         x2 = _rows(x, dtype)
         a16, b16 = cast_lora_weights(weight_a, weight_b, dtype)
         key = new_dropout_key(x2.device) if p > 0.0 else None
-        ctx.fused = (_fused(a16.shape[0], x2, a16, b16) and a16.is_contiguous()
-                     and b16.is_contiguous() and b16.shape[0] % 8 == 0 and _number(scaling))
+        ctx.fused = (_number(scaling) and not _hip.recorded(x2, a16, b16)
+                     and _fused(a16.shape[0], x2, a16, b16) and a16.is_contiguous()
+                     and b16.is_contiguous() and b16.shape[0] % 8 == 0)
         xa = _xa(x2, a16, key, p, True) if ctx.fused else lora_down_fwd(x2, a16, key, p)
         ctx.save_for_backward(x2, xa, a16, b16, key)
         ctx.p, ctx.scaling, ctx.dtype = p, scaling, dtype
@@ -297,6 +298,11 @@ class _LoRATerm:
                 db.to(ctx.b_dtype) if need[a_index + 1] else None)
 
 
+def _base_fused(ctx, base, b16):
+    rank = b16.shape[1]
+    return (ctx.fused and _base_pays(rank) and not _hip.recorded(base) and _fused(rank, base))
+
+
 class LoRAFunction(torch.autograd.Function):
     """apply(x, base, weight_a, weight_b, p, scaling) -> base + term. The term is added into
     base's own buffer when base is a fresh dense (non-view) tensor of the compute dtype (it is
@@ -308,14 +314,14 @@ class LoRAFunction(torch.autograd.Function):
         ctx.base_dtype = base.dtype
         if base.dtype == ctx.dtype and base.is_contiguous() and not base._is_view():
             flat = base.view(-1, base.shape[-1])
-            if ctx.fused and _base_pays(b16.shape[1]) and _fused(b16.shape[1], flat):
+            if _base_fused(ctx, flat, b16):
                 _hip.lora_up(xa, b16, flat, scaling, base=flat)
             else:
                 flat.addmm_(xa, b16.t(), alpha=scaling)
             ctx.mark_dirty(base)
             return base
         flat = base.reshape(-1, base.shape[-1]).to(ctx.dtype)
-        if ctx.fused and _base_pays(b16.shape[1]) and _fused(b16.shape[1], flat):
+        if _base_fused(ctx, flat, b16):
             out = torch.empty(flat.shape, device=flat.device, dtype=flat.dtype)
             _hip.lora_up(xa, b16, out, scaling, base=flat)
             return out.view(base.shape)

@@ -109,6 +109,61 @@ def test_scaling_given_as_a_tensor():
     _same(term, S * ((_rnd(T, K) @ _rnd(R, K).t()) @ b.t()))
 
 
+@pytest.mark.parametrize("name", ["delta", "down_fwd", "up_bwd", "down_bwd"])
+def test_traced(name):
+    """A trace holds the products themselves: it computes them for other inputs."""
+    fn, ref, ops = _functions()[name]
+    traced = torch.jit.trace(fn, ops, check_trace=False)
+    other = tuple(t.flip(0).contiguous() for t in ops)
+    _same(traced(*other), ref(*other))
+
+
+@pytest.mark.parametrize("name", ["delta", "down_fwd", "up_bwd", "down_bwd"])
+def test_seen_by_modes_and_subclasses(name):
+    """A dispatch mode sees the products, and a subclass gets its own type back."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Count(TorchDispatchMode):
+        n = 0
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.n += func.overloadpacket is torch.ops.aten.mm
+            return func(*args, **(kwargs or {}))
+
+    class Marked(torch.Tensor):
+        pass
+
+    fn, ref, ops = _functions()[name]
+    with Count() as count:
+        got = fn(*ops)
+    assert count.n == (2 if name.endswith("bwd") else 1)
+    _same(got, ref(*ops))
+    marked = fn(*(t.as_subclass(Marked) for t in ops))
+    assert all(type(t) is Marked for t in (marked if isinstance(marked, tuple) else (marked,)))
+
+
+@pytest.mark.parametrize("name", ["delta", "down_fwd", "up_bwd", "down_bwd"])
+def test_compiled_and_fake(name):
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    fn, ref, ops = _functions()[name]
+    compiled = torch.compile(fn, backend="eager", fullgraph=True)
+    _same(compiled(*ops), ref(*ops))
+    with FakeTensorMode() as mode:
+        fakes = fn(*(mode.from_tensor(t) for t in ops))
+    for f, r in zip(*((t if isinstance(t, tuple) else (t,)) for t in (fakes, ref(*ops)))):
+        assert f.shape == r.shape and f.dtype == r.dtype
+
+
+def test_term_under_a_trace():
+    from solution.body import lora as L
+
+    traced = torch.jit.trace(lambda x, a, b: L.LoRADeltaFunction.apply(x, a, b, 0.0, S),
+                             (_rnd(T, K), _rnd(R, K), _rnd(N, R)), check_trace=False)
+    x, a, b = _rnd(T, K, seed=1), _rnd(R, K, seed=1), _rnd(N, R, seed=1)
+    _same(traced(x, a, b), S * ((x @ a.t()) @ b.t()))
+
+
 @pytest.mark.parametrize("name,which,out", [("up_bwd", 2, 0), ("down_bwd", 1, 0)])
 def test_graph_of_the_backward_products(name, which, out):
     """Their 16-bit results are differentiable in every operand, not in the incoming gradient alone."""
