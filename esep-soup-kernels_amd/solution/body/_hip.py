@@ -208,6 +208,12 @@ def recorded(*tensors):
     return False
 
 
+def dense16(*tensors):
+    """Contiguous, at 16-byte addresses: asked of saved tensors, whose hooks may give back other
+    strides and addresses than the forward pass saw."""
+    return all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in tensors)
+
+
 def _rows_ld(t, n):
     """Leading dimension of a [rows, n] tensor whose last dim is contiguous. The column stride
     is checked whenever a row has more than one element (a one-row view such as t[:, ::2] or an

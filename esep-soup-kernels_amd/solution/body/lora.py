@@ -280,7 +280,8 @@ class _LoRATerm:
         # torch's products for a pass with create_graph, under vmap (is_grads_batched), with a tangent
         recorded = _hip.recorded(dt2, x2, xa, a16, b16)
         rank, dropout = b16.shape[1], ctx.p > 0.0
-        if (ctx.fused and not recorded and _fused(rank, dt2) and _up_grads_pay(*dt2.shape, rank)
+        if (ctx.fused and not recorded and _hip.dense16(x2, xa, a16, b16) and _fused(rank, dt2)
+                and _up_grads_pay(*dt2.shape, rank)
                 and _down_grads_pay(*x2.shape, rank, dropout, need[x_index])):
             # dx, dA and dB in one launch after dxa
             dxa = _dxa(dt2, b16, ctx.scaling, True)

@@ -318,3 +318,33 @@ def test_head_loss_gradient_batched_and_tangent():
     with fwd.dual_level():
         (dx,) = torch.autograd.grad(loss, x, fwd.make_dual(scale[0], scale[1]))
         torch.testing.assert_close(fwd.unpack_dual(dx).tangent, -2.5 * plain, rtol=1e-6, atol=0)
+
+
+def _transposed(t):
+    return t.t().contiguous().t() if t.dim() == 2 else t
+
+
+def _moved(t):
+    """The same values at an address that is 8 bytes past a 16-byte one."""
+    room = torch.empty(t.numel() + 16 // t.element_size(), device=t.device, dtype=t.dtype)
+    return room[8 // t.element_size():][:t.numel()].view(t.shape).copy_(t)
+
+
+@pytest.mark.parametrize("unpack", [_transposed, _moved])
+@pytest.mark.parametrize("what", ["lora", "delta"])
+def test_saved_tensors_given_back_otherwise(what, unpack):
+    """Saved-tensor hooks may give back other strides and addresses."""
+    from solution.body import lora as L
+
+    def run():
+        x, a, b = (_rnd(*s).requires_grad_() for s in ((T, K), (R, K), (N, R)))
+        if what == "lora":
+            out = L.LoRAFunction.apply(x, _rnd(T, N), a, b, 0.0, S)
+        else:
+            out = L.LoRADeltaFunction.apply(x, a, b, 0.0, S)
+        return torch.autograd.grad(out, (x, a, b), _rnd(T, N, seed=2))
+
+    want = run()
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+        got = run()
+    _same(got, want)
