@@ -175,7 +175,7 @@ class FusedLinearCE(torch.autograd.Function):
             return None, None, None, None, None
         prod, inv, cew = ctx.saved_tensors
         n, h = ctx.x_shape
-        if h % 8 == 0 and not _hip.recorded(dloss):
+        if h % 8 == 0 and not _hip.recorded(dloss) and _hip.dense16(prod, inv, cew):
             dx = torch.empty((n, h), device=prod.device, dtype=ctx.x_dtype)
             _hip.head_dx(prod, inv, cew, dloss, G_SCALE, dx)
             return dx, None, None, None, None

@@ -331,12 +331,19 @@ def _moved(t):
 
 
 @pytest.mark.parametrize("unpack", [_transposed, _moved])
-@pytest.mark.parametrize("what", ["lora", "delta"])
+@pytest.mark.parametrize("what", ["lora", "delta", "head"])
 def test_saved_tensors_given_back_otherwise(what, unpack):
     """Saved-tensor hooks may give back other strides and addresses."""
     from solution.body import lora as L
+    from solution.head.op import fused_linear_ce
 
     def run():
+        if what == "head":
+            x, w = _rnd(T, K).requires_grad_(), _rnd(N, K)
+            target = torch.arange(T, device=DEV)
+            target[::5] = -100
+            out = fused_linear_ce(x, w, target, torch.ones(T, device=DEV), chunk_rows=16)[0]
+            return torch.autograd.grad(out, (x,))
         x, a, b = (_rnd(*s).requires_grad_() for s in ((T, K), (R, K), (N, R)))
         if what == "lora":
             out = L.LoRAFunction.apply(x, _rnd(T, N), a, b, 0.0, S)
