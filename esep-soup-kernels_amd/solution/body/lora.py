@@ -257,12 +257,12 @@ class _LoRATerm:
     fused products take x, the rank and the output width (everything between them is dense)."""
 
     @staticmethod
-    def begin(ctx, x, weight_a, weight_b, p, scaling):
+    def begin(ctx, x, weight_a, weight_b, p, scaling, base=None):
         dtype = _compute_dtype(x)
         x2 = _rows(x, dtype)
         a16, b16 = cast_lora_weights(weight_a, weight_b, dtype)
         key = new_dropout_key(x2.device) if p > 0.0 else None
-        ctx.fused = (_number(scaling) and not _hip.recorded(x2, a16, b16)
+        ctx.fused = (_number(scaling) and not _hip.recorded(x2, a16, b16, base)
                      and _fused(a16.shape[0], x2, a16, b16) and a16.is_contiguous()
                      and b16.is_contiguous() and b16.shape[0] % 8 == 0)
         xa = _xa(x2, a16, key, p, True) if ctx.fused else lora_down_fwd(x2, a16, key, p)
@@ -277,11 +277,11 @@ class _LoRATerm:
         x2, xa, a16, b16, key = ctx.saved_tensors
         need = ctx.needs_input_grad
         dt2 = _rows_mm(dterm, ctx.dtype)
-        # torch's products for a pass with create_graph, under vmap (is_grads_batched), with a tangent
-        recorded = _hip.recorded(dt2, x2, xa, a16, b16)
         rank, dropout = b16.shape[1], ctx.p > 0.0
-        if (ctx.fused and not recorded and _hip.dense16(x2, xa, a16, b16) and _fused(rank, dt2)
-                and _up_grads_pay(*dt2.shape, rank)
+        # torch's products for a pass with create_graph, under vmap (is_grads_batched), with a tangent; of
+        # the saved tensors only x2 can be on the graph (ctx.fused: none is a wrapper or a subclass)
+        if (ctx.fused and not _hip.recorded(dt2, x2) and _hip.dense16(x2, xa, a16, b16)
+                and _fused(rank, dt2) and _up_grads_pay(*dt2.shape, rank)
                 and _down_grads_pay(*x2.shape, rank, dropout, need[x_index])):
             # dx, dA and dB in one launch after dxa
             dxa = _dxa(dt2, b16, ctx.scaling, True)
@@ -299,11 +299,6 @@ class _LoRATerm:
                 db.to(ctx.b_dtype) if need[a_index + 1] else None)
 
 
-def _base_fused(ctx, base, b16):
-    rank = b16.shape[1]
-    return (ctx.fused and _base_pays(rank) and not _hip.recorded(base) and _fused(rank, base))
-
-
 class LoRAFunction(torch.autograd.Function):
     """apply(x, base, weight_a, weight_b, p, scaling) -> base + term. The term is added into
     base's own buffer when base is a fresh dense (non-view) tensor of the compute dtype (it is
@@ -311,18 +306,18 @@ class LoRAFunction(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, base, weight_a, weight_b, p, scaling):
-        xa, b16 = _LoRATerm.begin(ctx, x, weight_a, weight_b, p, scaling)
+        xa, b16 = _LoRATerm.begin(ctx, x, weight_a, weight_b, p, scaling, base)
         ctx.base_dtype = base.dtype
         if base.dtype == ctx.dtype and base.is_contiguous() and not base._is_view():
             flat = base.view(-1, base.shape[-1])
-            if _base_fused(ctx, flat, b16):
+            if ctx.fused and _base_pays(b16.shape[1]) and _fused(b16.shape[1], flat):
                 _hip.lora_up(xa, b16, flat, scaling, base=flat)
             else:
                 flat.addmm_(xa, b16.t(), alpha=scaling)
             ctx.mark_dirty(base)
             return base
         flat = base.reshape(-1, base.shape[-1]).to(ctx.dtype)
-        if _base_fused(ctx, flat, b16):
+        if ctx.fused and _base_pays(b16.shape[1]) and _fused(b16.shape[1], flat):
             out = torch.empty(flat.shape, device=flat.device, dtype=flat.dtype)
             _hip.lora_up(xa, b16, out, scaling, base=flat)
             return out.view(base.shape)
